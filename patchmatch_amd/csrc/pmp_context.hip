@@ -217,7 +217,7 @@ int ensure_quads(pmp_ctx* ctx, Image& im, int wrap, hipStream_t stream) {
     return PMP_OK;
 }
 
-int timing_begin(pmp_ctx* ctx, int stage) {
+int timing_begin(pmp_ctx* ctx, int stage, int passes) {
     if (!ctx->timing) return -1;
     const size_t k = ctx->events_used;
     while (ctx->events.size() < 2 * (k + 1)) {
@@ -225,8 +225,12 @@ int timing_begin(pmp_ctx* ctx, int stage) {
         if (hipEventCreate(&e) != hipSuccess) return -1;
         ctx->events.push_back(e);
     }
-    if (ctx->event_stage.size() < k + 1) ctx->event_stage.resize(k + 1);
+    if (ctx->event_stage.size() < k + 1) {
+        ctx->event_stage.resize(k + 1);
+        ctx->event_passes.resize(k + 1);
+    }
     ctx->event_stage[k] = stage;
+    ctx->event_passes[k] = passes;
     if (hipEventRecord(ctx->events[2 * k], ctx->stream) != hipSuccess) return -1;
     ctx->events_used = k + 1;
     return (int)k;
@@ -356,7 +360,7 @@ int pmp_get_timing(pmp_ctx* ctx, pmp_timing* out) {
         PMP_HIP(ctx, hipEventElapsedTime(&ms, ctx->events[2 * k], ctx->events[2 * k + 1]));
         switch (ctx->event_stage[k]) {
             case kStageInit: out->init_ms += ms; break;
-            case kStagePropagate: out->propagate_ms += ms; out->propagate_launches++; break;
+            case kStagePropagate: out->propagate_ms += ms; out->propagate_launches += ctx->event_passes[k]; break;
             default: out->finalize_ms += ms; break;
         }
     }

@@ -4,7 +4,7 @@
 // descriptor set with one slot (the context workspace):
 //   pmp_random_initialization  k_init_q       (PatchMatchCuda.cu:210-270)
 //   pmp_score_plane_depth      k_score_q      (PatchMatchCuda.cu:255-270)
-//   pmp_red_black_pass         k_propagate_q  one launch per red-black pass
+//   pmp_red_black_pass         k_propagate_q  its passes, in one launch or one each
 //                                             (PatchMatchCuda.cu:273-407)
 //   pmp_finalize               k_copyback_q, k_median_q x2, k_postfilter_q
 //                                             (depthmap.cc:673-687, :731-760,
@@ -144,8 +144,10 @@ int plain_prepare(pmp_ctx* ctx, const pmp_params* p, const uint8_t* dmask, bool 
     fill_list(q->plain.h_hdr->init, 1, &items[0]);
     fill_list(q->plain.h_hdr->prop, 1, &items[1]);
     fill_list(q->plain.h_hdr->rows, 1, &items[2]);
+    if ((rc = ensure_sync(ctx, q->plain, (size_t)items[1]))) return rc;
     if (propagates && (rc = epochs_arm(ctx, ctx->stream, 1, &q->plain.h_slots[0], &items[1], pass0))) return rc;
-    if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0, r))) return rc;
+    if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0, items[1], r)))
+        return rc;
     if (p->iterations > kMaxPasses / 2) return set_error(ctx, PMP_EINVAL, "iterations must be <= 64");
     return desc_upload(ctx, q->plain, 1, ctx->stream);
 }
@@ -288,14 +290,12 @@ int pmp_red_black_pass(pmp_ctx* ctx, const pmp_params* params, int32_t it_begin,
     int rc = plain_prepare(ctx, params, nullptr, false, 2 * it_begin, true, q, r);
     if (rc) return rc;
     const int passes = 2 * (it_end - it_begin);
-    if ((rc = q_clear(ctx, ctx->stream, q->plain, passes))) return rc;
-    for (int pass = 0; pass < passes; ++pass) {
-        const int tp = timing_begin(ctx, kStagePropagate);
-        rc = q_prop(ctx, ctx->stream, q->plain, r, pass);
-        timing_end(ctx, tp);
-        if (rc) return rc;
-    }
-    return PMP_OK;
+    if ((rc = q_clear(ctx, ctx->stream, q->plain, r, passes))) return rc;
+    if (passes == 0) return PMP_OK;
+    const int tp = timing_begin(ctx, kStagePropagate, passes);
+    rc = q_prop(ctx, ctx->stream, q->plain, r, passes);
+    timing_end(ctx, tp);
+    return rc;
 }
 
 int pmp_finalize(pmp_ctx* ctx, const pmp_params* params, const uint8_t* mask) {

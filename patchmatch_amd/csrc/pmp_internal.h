@@ -140,6 +140,7 @@ struct pmp_ctx {
     bool timing = false;
     std::vector<hipEvent_t> events;   // pairs: start, end
     std::vector<int> event_stage;     // stage of each pair
+    std::vector<int> event_passes;    // red-black passes of each pair
     size_t events_used = 0;           // pairs recorded
     int densify_calls = 0;
 
@@ -182,7 +183,8 @@ namespace pmp {
 int set_error(pmp_ctx* ctx, int code, const std::string& msg);
 // Stage timing: returns the pair index to close with timing_end (or -1 when off).
 enum { kStageInit = 0, kStagePropagate = 1, kStageFinalize = 2 };
-int timing_begin(pmp_ctx* ctx, int stage);
+// passes: the red-black passes of the launch.
+int timing_begin(pmp_ctx* ctx, int stage, int passes = 1);
 void timing_end(pmp_ctx* ctx, int pair);
 int check_hip(pmp_ctx* ctx, hipError_t e, const char* what);
 // `rows` host rows of `row` bytes, `pitch` bytes apart, to contiguous device

@@ -127,7 +127,7 @@ __device__ __forceinline__ void offer(const SlotDesc& d, const float* sWc, float
                                       float* __restrict__ cdep, float* __restrict__ cscore,
                                       unsigned long long* __restrict__ keys) {
     const int i = pix / d.a.W, j = pix - (pix / d.a.W) * d.a.W;
-    const RefStat rs = ref_stats(d.a, sWc, i, j);
+    const RefStat rs = ref_stats(d.a, global_taps(d.a), sWc, i, j);
     const float sc = score_plane<0, kZero>(d.a, sWc, rs, i, j, p0, p1, p2, sv, 256);
     cplane[q] = make_float4(p0, p1, p2, 0.0f);
     cdep[q] = dist;

@@ -17,6 +17,7 @@ namespace pmp {
 
 constexpr int kMaxSlots = PMP_MAX_BATCH;
 constexpr int kMaxPasses = 2 * 64;
+constexpr size_t kMaxTiles = size_t(1) << 24;   // a ring entry: pass << 24 | tile
 
 // Everything a kernel needs about one keyframe slot.
 struct SlotDesc {
@@ -57,19 +58,28 @@ struct WorkList {
 
 struct BatchHdr {
     WorkList init, prop, rows;
+    // of a launch over several passes: per propagation tile, in list order, the
+    // arrivals of even and of odd passes (total words each), then the bands'
+    // rings of ready tiles (total words)
+    unsigned int* sync;
 };
 
 // A descriptor set in device memory (read by the kernels) with its pinned
-// host staging copy, the per-pass band heads of the propagation queue, and
-// the hipGraphs captured over this set's device pointers.
-using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero, rows, blocks, bands, postprocess
+// host staging copy, the band heads of the propagation queue, its tiles'
+// arrivals and rings (reached through the header, grown on demand), and the
+// hipGraphs captured over this set's device pointers.
+using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero, rows, blocks, bands, postprocess + 2 fused
+constexpr int kHeadStride = 32;           // words: every head lies in a cache line of its own
+constexpr int kHeadWords = 24 * kHeadStride;
 struct DescSet {
     int cap = 0;
     SlotDesc* h_slots = nullptr;
     BatchHdr* h_hdr = nullptr;
     SlotDesc* d_slots = nullptr;
     BatchHdr* d_hdr = nullptr;
-    unsigned int* d_heads = nullptr;     // 8 per pass
+    unsigned int* d_heads = nullptr;     // kHeadWords per launch of a call
+    unsigned int* d_sync = nullptr;      // BatchHdr::sync
+    size_t sync_cap = 0;                 // tiles
     hipEvent_t uploaded = nullptr;       // recorded after the last upload
     bool pending = false;
     std::map<GraphKey, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
@@ -82,6 +92,7 @@ struct QueueRun {
     int rows = 8;             // tile rows
     int blocks = 0;           // persistent grid
     int bands = 1;            // per-XCD bands
+    bool fused = false;       // all passes of a call in one launch
 };
 
 // Default launch shape: 8 x 64 tiles (256-thread blocks), 3 blocks per CU.
@@ -122,11 +133,19 @@ int desc_upload(pmp_ctx* ctx, DescSet& d, int n, hipStream_t stream);
 int slot_fill(pmp_ctx* ctx, const pmp_params* p, const pmp_keyframe& kf, const SlotBuf& b, const uint8_t* dmask,
               int pass0, int rows, hipStream_t stream, SlotDesc& d, int items[3]);
 void fill_list(WorkList& L, int n, const int* items);
-int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, QueueRun& r);
-int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, int passes);
+// tiles: propagation tiles of a pass.
+int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
+              QueueRun& r);
+int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes);
 int q_init(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);
 int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);
-int q_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int pass);
+// The first `passes` red-black passes after the slots' pass0, in one launch or
+// one launch each (r.fused), after a q_clear with the same run and pass count.
+// One launch over several passes needs the set's arrivals and rings
+// (ensure_sync).
+int q_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes);
+// Arrivals and rings for `tiles` propagation tiles, named in the staged header.
+int ensure_sync(pmp_ctx* ctx, DescSet& d, size_t tiles);
 int q_finalize(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);
 // clear + init + `passes` passes + finalize, replayed from a graph cached in d
 // when use_graph (the set's contents may change between replays).

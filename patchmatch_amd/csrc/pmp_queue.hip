@@ -19,6 +19,8 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "pmp_trace.h"
 #include "pmp_internal.h"
 #include "pmp_math.h"
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(256) void k_init_q(const SlotDesc PMP_CONST* slots,
         if constexpr (kScore) {
             if (!in_score_grid(d.a, i, j)) continue;
             const size_t k = (size_t)i * d.a.W + j;
-            const RefStat rs = ref_stats(d.a, sWc, i, j);
+            const RefStat rs = ref_stats(d.a, tp, sWc, i, j);
             const float4 p = d.plane[k];
             d.score[k] = score_plane_t<0, kZero>(d.a, tp, sWc, rs, i, j, p.x, p.y, p.z, &sv[0][threadIdx.x], 256);
         } else {
@@ -152,47 +154,169 @@ __device__ __forceinline__ void epoch_leave(const SlotDesc& d, int tx, int ty, i
     }
 }
 
+// ---- all red-black passes of a call in one launch
+// A tile may run pass p + 1 as soon as it and the 8 tiles around it have
+// completed pass p: they wrote what it reads, and, since they in turn wait for
+// this tile, none of them is ahead by more than one pass, which writes only
+// the colour that this one does not read.  So the tail of a pass, when its
+// last tiles leave compute units idle, overlaps the next pass.
+//
+// Every block takes tiles of its own XCD's band (home) and of bands that are
+// behind it.  Pass-0 tiles are handed out in list order through a ticket per
+// band.  A tile that completes pass p counts itself in at the 9 tiles it may
+// release (arrivals, one count per pass parity: a neighbour cannot complete
+// pass p + 2 before this tile has completed p + 1, so the counts of one parity
+// never mix two passes); the last of a tile's arrivals puts (tile, p + 1) into
+// its band's ring, from which blocks take tiles in that order.
+//
+// No block waits while it holds a tile, and none takes a ring entry that has
+// not been announced, so some block progresses whatever part of the grid is
+// resident: a tile that is ready lies in a ring, and any running block that
+// has no work looks through all rings.  The two waits for another block's
+// store (a ring slot announced but not written yet, one taken but not read
+// yet) are for blocks that are past every other wait.
+//
+// heads: three words per band, each in a cache line of its own.
+__device__ __forceinline__ unsigned int* head_of(unsigned int* heads, int kind, int band) {
+    return heads + (kind * 8 + band) * kHeadStride;
+}
+// A block without work looks again after 64 x 64 cycles, then after up to
+// kMaxNaps times that: the looks share a few cache lines with the others' atomics.
+constexpr int kNap = 64, kMaxNaps = 4;
+enum { kHeadFirst = 0, kHeadRing = 1, kHeadTail = 2 };   // pass-0 tickets; ring entries taken, announced
+
+__device__ __forceinline__ int load_agent(const unsigned int* p) {
+    return (int)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int band_lo(int total, int band, int nb) { return (int)(((long long)total * band) / nb); }
+
+// Takes the block's next (tile, pass) into sh.item (-1: nothing is left to
+// take) and sh.pass: from the band that is furthest behind among those with a
+// tile to take, its own on a tie.  (Own band first whatever its pass let a
+// keyframe's cheap bands run ahead of its dear ones, whose last passes then ran
+// on few tiles: a 1920x960 keyframe whose bottom eighth starts from random
+// planes and the rest from a warped result took 17.3 ms for 4 passes.)  Called
+// by the block's first wave; lane b < 8 looks at band home + b.
+template <int R, int NVS>
+__device__ __forceinline__ void take_tile(const BatchHdr PMP_CONST* hdr, int passes, unsigned int* heads, int bands,
+                                          PropShared<R, NVS>& sh) {
+    const int total = hdr->prop.total;
+    unsigned int* ring = hdr->sync + 2 * (size_t)total;
+    const int nb = bands ? 8 : 1;
+    const int home = bands ? (int)(blockIdx.x & 7) : 0;
+    const int lane = threadIdx.x;
+    const int band = (home + lane) & (nb - 1);
+    const int lo = band_lo(total, band, nb), n = band_lo(total, band + 1, nb) - lo;
+    unsigned int* h0 = head_of(heads, kHeadFirst, band);
+    unsigned int* hr = head_of(heads, kHeadRing, band);
+    unsigned int* ht = head_of(heads, kHeadTail, band);
+    int item = -1, pass = 0, naps = 1;
+    for (;;) {
+        int level = 0x7FFFFFFF, q = 0;   // the pass (about, in the ring) of the band's next tile
+        bool left = false;
+        if (lane < nb && n > 0) {
+            if (load_agent(h0) < n) {
+                level = 0;
+            } else if (passes > 1) {
+                q = load_agent(hr);
+                left = q < n * (passes - 1);
+                if (q < load_agent(ht)) level = 1 + q / n;
+            }
+        }
+        int best = level;
+#pragma unroll
+        for (int k = 1; k < 8; k <<= 1) best = min(best, __shfl_xor(best, k, 64));
+        const unsigned long long at = __ballot(lane < nb && level == best && level != 0x7FFFFFFF);
+        if (at == 0ull) {
+            if (__ballot(left) == 0ull) break;
+            for (int k = 0; k < naps; ++k) __builtin_amdgcn_s_sleep(kNap);
+            naps = min(2 * naps, kMaxNaps);
+            continue;
+        }
+        bool got = false;
+        if (lane == __ffsll((long long)at) - 1) {
+            if (level == 0) {
+                const int h = (int)atomicAdd(h0, 1u);
+                got = h < n;
+                item = lo + h;
+                pass = 0;
+            } else if ((int)atomicCAS(hr, (unsigned int)q, (unsigned int)q + 1u) == q) {
+                unsigned int v;
+                while ((v = atomicExch(&ring[lo + q % n], 0u)) == 0u) __builtin_amdgcn_s_sleep(1);
+                got = true;
+                item = (int)(v & 0xFFFFFFu);
+                pass = (int)(v >> 24);
+            }
+            if (got) {
+                sh.item = item;
+                sh.pass = pass;
+            }
+        }
+        if (__any(got)) return;
+    }
+    if (lane == 0) sh.item = -1;
+}
+
+// The block's tile (list index item, at (tx, ty) of slot d) has completed
+// pass `pass` of the launch, which is not the last: counts it in at the tiles
+// around it and announces those that are now ready.  Called by every thread.
+__device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, const SlotDesc& d, unsigned int* heads,
+                                              int bands, int item, int tx, int ty, int pass) {
+    // every thread's maps have reached memory before the tile counts as done
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x >= 9) return;
+    const int total = hdr->prop.total;
+    const int nb = bands ? 8 : 1;
+    const int nbx = d.nbx_prop, nby = d.nby_prop;
+    const int x = tx + (int)threadIdx.x % 3 - 1, y = ty + (int)threadIdx.x / 3 - 1;
+    if (x < 0 || y < 0 || x >= nbx || y >= nby) return;
+    const int t = item - (ty * nbx + tx) + y * nbx + x;
+    const int around = (min(x + 1, nbx - 1) - max(x - 1, 0) + 1) * (min(y + 1, nby - 1) - max(y - 1, 0) + 1);
+    const int arrived = (int)atomicAdd(&hdr->sync[(size_t)(pass & 1) * total + t], 1u) + 1;
+    if (arrived != around * (pass / 2 + 1)) return;
+    int band = (int)(((long long)t * nb) / total);
+    while (t >= band_lo(total, band + 1, nb)) ++band;
+    const int lo = band_lo(total, band, nb), n = band_lo(total, band + 1, nb) - lo;
+    const int q = (int)atomicAdd(head_of(heads, kHeadTail, band), 1u);
+    unsigned int* slot = hdr->sync + 2 * (size_t)total + lo + q % n;
+    while (atomicCAS(slot, 0u, ((unsigned int)(pass + 1) << 24) | (unsigned int)t) != 0u) __builtin_amdgcn_s_sleep(1);
+}
+
+// One launch over `passes` red-black passes of every slot, the first being
+// pass `first` of the call.
+//
 // The zero-edge variant is held to 4 waves per SIMD (<= 128 VGPRs; left
 // alone it takes 132 and runs at 3 waves, 28 % slower); the wrap/clamp
 // variant fits by itself and is faster with the compiler's own allocation.
 template <bool kZero, int R>
-__global__ __launch_bounds__(64 * R) __attribute__((amdgpu_waves_per_eu(kZero ? 4 : 1))) void k_propagate_q(const SlotDesc PMP_CONST* slots,
-                                                        const BatchHdr PMP_CONST* hdr, int pass,
-                                                        unsigned int* __restrict__ heads,
-                                                        unsigned long long* __restrict__ counters, int bands) {
+__global__ __launch_bounds__(64 * R) __attribute__((amdgpu_waves_per_eu(kZero ? 4 : 1))) void k_propagate_q(
+    const SlotDesc PMP_CONST* slots, const BatchHdr PMP_CONST* hdr, int first, int passes,
+    unsigned int* __restrict__ heads, unsigned long long* __restrict__ counters, int bands) {
     __shared__ PropShared<R, kMaxViews> sh;
     const WorkList PMP_CONST* L = &hdr->prop;
-    const int total = L->total;
-    const int nb = bands ? 8 : 1;
-    const int home = bands ? (int)(blockIdx.x & 7) : 0;
     unsigned int n_eval = 0, n_cand = 0;
     int cur = -1;
-    for (int k = 0; k < nb; ++k) {
-        const int band = (home + k) & (nb - 1);
-        const int lo = (int)(((long long)total * band) / nb);
-        const int hi = (int)(((long long)total * (band + 1)) / nb);
-        for (;;) {
-            // every block takes items until its band's head passes the end:
-            // each atomicAdd moves the head, so the loop ends for every block
-            if (threadIdx.x == 0) sh.item = lo + (int)atomicAdd(&heads[band], 1u);
-            __syncthreads();
-            const int item = sh.item;
-            __syncthreads();
-            if (item >= hi) break;
-            int local;
-            const int s = list_find(L, item, local);
-            const SlotDesc& d = slot_ref(slots, s);
-            if (s != cur) {
-                load_wc(d.a.Wc, sh.sWc);
-                cur = s;
-            }
-            const int pp = d.pass0 + pass;
-            const int tx = local % d.nbx_prop, ty = local / d.nbx_prop;
-            if (d.epochs) epoch_enter(d, tx, ty, pp);
-            propagate_tile<0, kZero, R>(d.a, sh, d.plane, d.depth, d.score, pp >> 1, pp & 1, tx, ty,
-                                        64 * (item & (R - 1)), n_eval, n_cand);
-            if (d.epochs) epoch_leave(d, tx, ty, pp);
+    for (;;) {
+        if (threadIdx.x < 64) take_tile(hdr, passes, heads, bands, sh);
+        __syncthreads();
+        const int item = sh.item, pass = sh.pass;
+        __syncthreads();
+        if (item < 0) break;
+        int local;
+        const int s = list_find(L, item, local);
+        const SlotDesc& d = slot_ref(slots, s);
+        if (s != cur) {
+            load_wc(d.a.Wc, sh.sWc);
+            cur = s;
         }
+        const int pp = d.pass0 + first + pass;
+        const int tx = local % d.nbx_prop, ty = local / d.nbx_prop;
+        if (d.epochs) epoch_enter(d, tx, ty, pp);
+        propagate_tile<0, kZero, R>(d.a, sh, d.plane, d.depth, d.score, pp >> 1, pp & 1, tx, ty, 64 * (item & (R - 1)),
+                                    n_eval, n_cand);
+        if (d.epochs) epoch_leave(d, tx, ty, pp);
+        if (pass + 1 < passes) release_tiles(hdr, d, heads, bands, item, tx, ty, pass);
     }
     count_add(&counters[0], n_eval);
     count_add(&counters[1], n_cand);
@@ -243,7 +367,7 @@ int desc_alloc(pmp_ctx* ctx, DescSet& d, int cap) {
     PMP_HIP(ctx, hipHostMalloc((void**)&d.h_hdr, sizeof(BatchHdr), hipHostMallocDefault));
     PMP_HIP(ctx, hipMalloc(&d.d_slots, cap * sizeof(SlotDesc)));
     PMP_HIP(ctx, hipMalloc(&d.d_hdr, sizeof(BatchHdr)));
-    PMP_HIP(ctx, hipMalloc(&d.d_heads, 8 * kMaxPasses * sizeof(unsigned int)));
+    PMP_HIP(ctx, hipMalloc(&d.d_heads, (size_t)kMaxPasses * kHeadWords * sizeof(unsigned int)));
     PMP_HIP(ctx, hipEventCreateWithFlags(&d.uploaded, hipEventDisableTiming));
     return PMP_OK;
 }
@@ -258,6 +382,7 @@ void desc_free(DescSet& d) {
     if (d.d_slots) (void)hipFree(d.d_slots);
     if (d.d_hdr) (void)hipFree(d.d_hdr);
     if (d.d_heads) (void)hipFree(d.d_heads);
+    if (d.d_sync) (void)hipFree(d.d_sync);
     if (d.uploaded) (void)hipEventDestroy(d.uploaded);
     d = DescSet();
 }
@@ -377,12 +502,23 @@ static int check_config(pmp_ctx* ctx, const pmp_batch_config& c) {
 
 // Persistent grid: the configured blocks per CU, capped by (and defaulting
 // to) what fits on a CU at once; a multiple of 8 with per-XCD bands.
-int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, QueueRun& r) {
+int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
+              QueueRun& r) {
     int occ = 0;
     PMP_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, prop_kernel(zero, c.tile_rows),
                                                               64 * c.tile_rows, 0));
     if (occ < 1) occ = 1;
-    const int bpc = (c.blocks_per_cu <= 0 || c.blocks_per_cu > occ) ? occ : c.blocks_per_cu;
+    int bpc = (c.blocks_per_cu <= 0 || c.blocks_per_cu > occ) ? occ : c.blocks_per_cu;
+    // blocks beyond one per tile would only look for work
+    if (tiles > 0) bpc = std::min(bpc, (tiles + q.cus - 1) / q.cus);
+    // One launch over all passes pays where the blocks in flight hold less
+    // than two thirds of the tiles (1920x960, 6 views: 51.5 against 57.9 ms;
+    // 1120x560, 8 views, 4 iterations: 17.7 against 19.9 ms), and where each
+    // tile has a compute unit to itself (480x240, 2 views: 2.9 against
+    // 3.3 ms).  In between most tiles are in flight at once and wait for each
+    // other tile by tile, while the launches' own barrier leaves the last ones
+    // whole compute units (800x400, 4 views, 4 iterations: 10.7 against 6.5 ms).
+    r.fused = tiles <= q.cus || 2 * tiles >= 3 * q.cus * bpc;
     r.zero = zero;
     r.post = post;
     r.rows = c.tile_rows;
@@ -401,13 +537,41 @@ static int grid_blocks(pmp_ctx* ctx) {
     return (q && q->cus > 0 ? q->cus : 256) * 8;
 }
 
-int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, int passes) {
-    // fill kernels, not memset nodes: the sequence may be captured
-    const int n = 8 * passes;
-    if (n > 0)
-        hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d.d_heads, n, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, (unsigned int*)ctx->counters, 4, 0u);
+// Before the launches of the propagation kernel: their band heads, the
+// evaluation counters and, for one launch over several passes, the tiles'
+// arrivals and the rings.
+__global__ void k_clear(const BatchHdr PMP_CONST* hdr, unsigned int* __restrict__ heads, int head_words,
+                        unsigned int* __restrict__ counters, int sync) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (int t = k; t < head_words; t += step) heads[t] = 0u;
+    if (k < 4) counters[k] = 0u;
+    if (sync)
+        for (int t = k; t < 3 * hdr->prop.total; t += step) hdr->sync[t] = 0u;
+}
+
+int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes) {
+    PMP_QPTRS
+    (void)sl;
+    // a fill kernel, not memset nodes: the sequence may be captured
+    const bool one = r.fused && passes > 1;
+    const int words = kHeadWords * (one ? 1 : std::max(passes, 1));
+    hipLaunchKernelGGL(k_clear, dim3(one ? 64 : (words + 255) / 256), dim3(256), 0, s, hd, d.d_heads, words,
+                       (unsigned int*)ctx->counters, one ? 1 : 0);
     PMP_HIP(ctx, hipGetLastError());
+    return PMP_OK;
+}
+
+int ensure_sync(pmp_ctx* ctx, DescSet& d, size_t tiles) {
+    if (tiles > kMaxTiles) return set_error(ctx, PMP_EINVAL, "too many propagation tiles in one call");
+    if (tiles > d.sync_cap) {
+        PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (d.d_sync) (void)hipFree(d.d_sync);
+        d.d_sync = nullptr;
+        d.sync_cap = 0;
+        PMP_HIP(ctx, hipMalloc(&d.d_sync, 3 * tiles * sizeof(unsigned int)));
+        d.sync_cap = tiles;
+    }
+    d.h_hdr->sync = d.d_sync;
     return PMP_OK;
 }
 
@@ -429,12 +593,13 @@ int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
     return PMP_OK;
 }
 
-int q_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int pass) {
+// One launch over passes [first, first + passes), with the heads of launch `launch`.
+static int launch_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int launch, int first, int passes) {
     PMP_QPTRS
     const dim3 grd((unsigned)r.blocks), blk((unsigned)(64 * r.rows));
-    unsigned int* heads = d.d_heads + 8 * pass;
-#define PMP_PROP(Z, R) \
-    hipLaunchKernelGGL((k_propagate_q<Z, R>), grd, blk, 0, s, sl, hd, pass, heads, ctx->counters, r.bands)
+    unsigned int* heads = d.d_heads + (size_t)launch * kHeadWords;
+#define PMP_PROP(Z, R)                                                                                              \
+    hipLaunchKernelGGL((k_propagate_q<Z, R>), grd, blk, 0, s, sl, hd, first, passes, heads, ctx->counters, r.bands)
     if (r.zero) {
         if (r.rows == 2) PMP_PROP(true, 2);
         else if (r.rows == 4) PMP_PROP(true, 4);
@@ -447,6 +612,13 @@ int q_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int pass)
 #undef PMP_PROP
     PMP_HIP(ctx, hipGetLastError());
     return PMP_OK;
+}
+
+int q_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes) {
+    if (r.fused) return passes > 0 ? launch_prop(ctx, s, d, r, 0, 0, passes) : PMP_OK;
+    int rc = PMP_OK;
+    for (int p = 0; p < passes && !rc; ++p) rc = launch_prop(ctx, s, d, r, p, p, 1);
+    return rc;
 }
 
 int q_finalize(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
@@ -500,13 +672,13 @@ int epochs_arm(pmp_ctx* ctx, hipStream_t s, int n, SlotDesc* slots, const int* t
 
 static int q_sequence(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes) {
     int rc;
-    if ((rc = q_clear(ctx, s, d, passes))) return rc;
+    if ((rc = q_clear(ctx, s, d, r, passes))) return rc;
     int tp = timing_begin(ctx, kStageInit);
     if ((rc = q_init(ctx, s, d, r))) return rc;
     timing_end(ctx, tp);
-    for (int p = 0; p < passes; ++p) {
-        tp = timing_begin(ctx, kStagePropagate);
-        if ((rc = q_prop(ctx, s, d, r, p))) return rc;
+    if (passes > 0) {
+        tp = timing_begin(ctx, kStagePropagate, passes);
+        if ((rc = q_prop(ctx, s, d, r, passes))) return rc;
         timing_end(ctx, tp);
     }
     tp = timing_begin(ctx, kStageFinalize);
@@ -518,7 +690,7 @@ static int q_sequence(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r
 int q_densify(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes, bool use_graph) {
     // per-stage timing needs events between the launches: no graph then
     if (!use_graph || ctx->timing) return q_sequence(ctx, s, d, r, passes);
-    const GraphKey key{passes, r.zero ? 1 : 0, r.rows, r.blocks, r.bands, r.post ? 1 : 0};
+    const GraphKey key{passes, r.zero ? 1 : 0, r.rows, r.blocks, r.bands, (r.post ? 1 : 0) + (r.fused ? 2 : 0)};
     auto it = d.graphs.find(key);
     if (it == d.graphs.end()) {
         hipGraph_t g = nullptr;
@@ -575,6 +747,7 @@ static int batch_prepare(pmp_ctx* ctx, QueueState* q, const pmp_params* params, 
     fill_list(q->batch.h_hdr->init, n, it_init);
     fill_list(q->batch.h_hdr->prop, n, it_prop);
     fill_list(q->batch.h_hdr->rows, n, it_rows);
+    if ((rc = ensure_sync(ctx, q->batch, (size_t)q->batch.h_hdr->prop.total))) return rc;
     if (arm && (rc = epochs_arm(ctx, ctx->stream, n, q->batch.h_slots, it_prop, 0))) return rc;
     return desc_upload(ctx, q->batch, n, ctx->stream);
 }
@@ -596,7 +769,9 @@ int pmp_batch_densify(pmp_ctx* ctx, const pmp_params* params, int32_t n, const p
     q->n_last = 0;
     if ((rc = batch_prepare(ctx, q, params, n, kfs, q->cfg.tile_rows, true))) return rc;
     QueueRun r;
-    if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0, r))) return rc;
+    if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0,
+                        q->batch.h_hdr->prop.total, r)))
+        return rc;
     if ((rc = q_densify(ctx, ctx->stream, q->batch, r, 2 * params->iterations, q->cfg.use_graph != 0))) return rc;
     q->n_last = n;
     ctx->densify_calls += n;
@@ -662,7 +837,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
         c.tile_rows = rows_set[ri];
         c.blocks_per_cu = 32;
         QueueRun r;
-        if ((rc = queue_run(ctx, *q, c, zero, false, r))) break;
+        if ((rc = queue_run(ctx, *q, c, zero, false, q->batch.h_hdr->prop.total, r))) break;
         const int occ = r.blocks / (q->cus > 0 ? q->cus : 1);   // blocks per CU that fit (rounding aside)
         // at least 8 waves per CU (rows waves per block): fewer leave SIMDs
         // idle and measured 1.3-4x slower, and their trials are the longest
@@ -671,7 +846,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
             for (int bands = 0; bands <= 1 && rc == 0; ++bands) {
                 c.blocks_per_cu = bpc;
                 c.xcd_bands = bands;
-                if ((rc = queue_run(ctx, *q, c, zero, false, r))) break;
+                if ((rc = queue_run(ctx, *q, c, zero, false, q->batch.h_hdr->prop.total, r))) break;
                 // same starting maps for every candidate: init, then time every
                 // pass.  The first passes score random planes (most candidates
                 // survive pre-rejection, the gathers scatter); the converged
@@ -679,11 +854,10 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
                 // The shapes rank differently on the two kinds, so a prefix of
                 // passes misranks them.
                 const int timed = 2 * params->iterations;
-                if ((rc = q_clear(ctx, ctx->stream, q->batch, timed))) break;   // every timed pass's heads
+                if ((rc = q_clear(ctx, ctx->stream, q->batch, r, timed))) break;
                 if ((rc = q_init(ctx, ctx->stream, q->batch, r))) break;
                 hipError_t e = hipEventRecord(e0, ctx->stream);
-                for (int pass = 0; pass < timed && e == hipSuccess && rc == 0; ++pass)
-                    rc = q_prop(ctx, ctx->stream, q->batch, r, pass);
+                if (e == hipSuccess) rc = q_prop(ctx, ctx->stream, q->batch, r, timed);
                 if (e == hipSuccess && rc == 0) e = hipEventRecord(e1, ctx->stream);
                 if (e == hipSuccess && rc == 0) e = hipEventSynchronize(e1);
                 float ms = 0.0f;

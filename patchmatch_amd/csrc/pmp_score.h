@@ -58,42 +58,6 @@ struct RefStat {
     float Ic, mx, inv, mxc, vx;
 };
 
-// Plane-independent reference-side moments of the patch (two passes).
-PMP_DF RefStat ref_stats(const KfArgs& a, const float* sWc, int i, int j) {
-    RefStat s;
-    const int W = a.W;
-    s.Ic = (float)a.ref[(size_t)i * W + j];
-    float Sw = 0.0f, Swx = 0.0f;
-    int t = 0;
-    for (int k1 = -a.half; k1 <= a.half; k1 += a.stride) {
-        const uint8_t* row = a.ref + (size_t)(i + k1) * W + j;
-        for (int k2 = -a.half; k2 <= a.half; k2 += a.stride, ++t) {
-            float xs = (float)row[k2] - s.Ic;
-            float w = sWc[(int)abs_(xs)] * a.Ws[t];
-            Sw = Sw + w;
-            Swx = fma_(w, xs, Swx);
-        }
-    }
-    s.inv = rcp_pos(Sw);
-    s.mx = Swx * s.inv;
-    float Sc = 0.0f, Scc = 0.0f;
-    t = 0;
-    for (int k1 = -a.half; k1 <= a.half; k1 += a.stride) {
-        const uint8_t* row = a.ref + (size_t)(i + k1) * W + j;
-        for (int k2 = -a.half; k2 <= a.half; k2 += a.stride, ++t) {
-            float xs = (float)row[k2] - s.Ic;
-            float w = sWc[(int)abs_(xs)] * a.Ws[t];
-            float xc = xs - s.mx;
-            float wxc = w * xc;
-            Sc = Sc + wxc;
-            Scc = fma_(wxc, xc, Scc);
-        }
-    }
-    s.mxc = Sc * s.inv;
-    s.vx = fma_(-s.mxc, s.mxc, Scc * s.inv);
-    return s;
-}
-
 PMP_DF float ncc(const RefStat& rs, float floor_, float Swy, float Swyy, float Swxy) {
     float my = Swy * rs.inv;
     float vy = fma_(-my, my, Swyy * rs.inv);
@@ -342,6 +306,53 @@ struct LdsTaps {
     PMP_DF uint32_t rowstep() const { return (uint32_t)kTileCols; }
     PMP_DF float refpx(uint32_t roff, int jj) const { return (float)sref[roff + (uint32_t)jj]; }
 };
+
+// Plane-independent reference-side moments of the patch (two passes),
+// the pixels read through tp.
+template <class Taps>
+PMP_DF RefStat ref_stats(const KfArgs& a, const Taps& tp, const float* sWc, int i, int j) {
+    RefStat s;
+    s.Ic = tp.refpx(tp.rowoff(i) + (uint32_t)j, 0);
+    float Sw = 0.0f, Swx = 0.0f;
+    int t = 0;
+    for (int k1 = -a.half; k1 <= a.half; k1 += a.stride) {
+        const uint32_t roff = tp.rowoff(i + k1) + (uint32_t)j;
+        for (int k2 = -a.half; k2 <= a.half; k2 += a.stride, ++t) {
+            float xs = tp.refpx(roff, k2) - s.Ic;
+            float w = sWc[(int)abs_(xs)] * a.Ws[t];
+            Sw = Sw + w;
+            Swx = fma_(w, xs, Swx);
+        }
+    }
+    s.inv = rcp_pos(Sw);
+    s.mx = Swx * s.inv;
+    float Sc = 0.0f, Scc = 0.0f;
+    t = 0;
+    for (int k1 = -a.half; k1 <= a.half; k1 += a.stride) {
+        const uint32_t roff = tp.rowoff(i + k1) + (uint32_t)j;
+        for (int k2 = -a.half; k2 <= a.half; k2 += a.stride, ++t) {
+            float xs = tp.refpx(roff, k2) - s.Ic;
+            float w = sWc[(int)abs_(xs)] * a.Ws[t];
+            float xc = xs - s.mx;
+            float wxc = w * xc;
+            Sc = Sc + wxc;
+            Scc = fma_(wxc, xc, Scc);
+        }
+    }
+    s.mxc = Sc * s.inv;
+    s.vx = fma_(-s.mxc, s.mxc, Scc * s.inv);
+    return s;
+}
+
+// Bearing of a pixel from the taps' tables.
+template <class Taps>
+PMP_DF void tap_bearing(const Taps& tp, int i, int j, float& bx, float& by, float& bz) {
+    const float2 r = tp.row(i);
+    const float2 c = tp.col(j);
+    bx = r.x * c.x;
+    by = -r.y;
+    bz = r.x * c.y;
+}
 
 // Shifted moments of one view: a0 = sum w yd, a1 = sum w yd^2,
 // a2 = sum w xc yd with yd = y - sh (sh = the centre tap's sample).

@@ -218,9 +218,9 @@ class GpuExec final : public sched::Executor {
         fill_list(d.h_hdr->prop, n, items_prop);
         fill_list(d.h_hdr->rows, n, items_rows);
         QueueRun run;
-        rc = queue_run(ctx, *ctx->queue, cfg, edge_mode == PMP_EDGE_ZERO, post, run);
+        rc = queue_run(ctx, *ctx->queue, cfg, edge_mode == PMP_EDGE_ZERO, post, d.h_hdr->prop.total, run);
         if (!rc) rc = desc_upload(ctx, d, n, ctx->stream);
-        if (!rc) rc = q_clear(ctx, ctx->stream, d, 1);
+        if (!rc) rc = q_clear(ctx, ctx->stream, d, run, 1);
         if (!rc && d.h_hdr->init.n) rc = q_init(ctx, ctx->stream, d, run);
         for (const sched::StepItem* it : seeds) {
             if (rc) break;
@@ -236,7 +236,7 @@ class GpuExec final : public sched::Executor {
             rc = preinit_warp_slot(ctx, d.d_slots + it->slot, j->W, j->H, (const double*)&j->kf.ref_pose,
                                    j->prev_pose, j->prev_plane4, j->prev_depth, edge_mode == PMP_EDGE_ZERO);
         }
-        if (!rc && d.h_hdr->prop.n) rc = q_prop(ctx, ctx->stream, d, run, 0);
+        if (!rc && d.h_hdr->prop.n) rc = q_prop(ctx, ctx->stream, d, run, 1);
         if (!rc && d.h_hdr->rows.n) rc = q_finalize(ctx, ctx->stream, d, run);
         for (const sched::StepItem* it : fin) {
             if (rc) break;

@@ -44,7 +44,7 @@ __device__ __forceinline__ void init_pixel(const KfArgs& a, const Taps& tp, cons
     if (in_init_grid(a, i, j)) random_plane(a, i, j, p0, p1, p2, dep);
     float sc = __uint_as_float(0xFFFFFFFFu);   // cudaMemset(score, 0xFF) (depthmap.cc:657)
     if (in_score_grid(a, i, j)) {
-        RefStat rs = ref_stats(a, sWc, i, j);
+        RefStat rs = ref_stats(a, tp, sWc, i, j);
         sc = score_plane_t<NV, kZero>(a, tp, sWc, rs, i, j, p0, p1, p2, sv, ld);
     }
     const size_t k = (size_t)i * a.W + j;
@@ -84,8 +84,11 @@ __device__ __forceinline__ void init_pixel(const KfArgs& a, const Taps& tp, cons
 // otherwise).
 // srow/scol/sref: the tile's rows and columns of the bearing tables and of
 // the reference image, with the patch halo (LdsTaps).
+// pl: the other colour's planes of the tile and 3 pixels around it, where its
+// candidates are (plane_at).
 // res[c * 64R + t]: raw score of candidate c of thread t's pixel; job: the
 // sweep's (candidate << 9 | thread) list.
+constexpr int kPlaneCols = kTileSame + 3;   // one colour's pixels in a row of the tile and 3 columns each side
 template <int R, int NVS = 1>
 struct PropShared {
     float sWc[256];
@@ -97,9 +100,34 @@ struct PropShared {
     float2 srow[64 * R / kTileSame + 2 * kMaxHalf];
     float2 scol[kTileCols];
     uint8_t sref[(64 * R / kTileSame + 2 * kMaxHalf) * kTileCols];
+    float4 pl[(64 * R / kTileSame + 6) * kPlaneCols];
     int cnt[8 * R];
-    int item;
+    int item, pass;
 };
+
+// The maps that tiles of one launch hand each other (pass fusion: a tile of
+// pass p + 1 runs beside tiles of pass p) go through agent-scope accesses:
+// the XCDs' L2 caches are not coherent with each other for plain ones within
+// a launch.
+__device__ __forceinline__ float load_map(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_map(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float4 load_map4(const float4* p) {
+    const unsigned long long* q = (const unsigned long long*)p;
+    const unsigned long long a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long b = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float4(u2f((uint32_t)a), u2f((uint32_t)(a >> 32)), u2f((uint32_t)b), u2f((uint32_t)(b >> 32)));
+}
+__device__ __forceinline__ void store_map4(float4* p, float4 v) {
+    unsigned long long* q = (unsigned long long*)p;
+    __hip_atomic_store(q, (unsigned long long)f2u(v.x) | ((unsigned long long)f2u(v.y) << 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(q + 1, (unsigned long long)f2u(v.z) | ((unsigned long long)f2u(v.w) << 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Offset (di, dj) of propagation candidate c: (0,+1) (+1,0) (0,-1) (-1,0)
 // (0,+3) (+3,0) (0,-3) (-3,0) (PatchMatchCuda.cu:305)
@@ -150,15 +178,25 @@ __device__ __forceinline__ bool cand_test(const KfArgs& a, float4 pn, float bx, 
 // [tby TR - half, tby TR + TR + half) and columns [2 kTileSame tbx - half,
 // 2 kTileSame (tbx + 1) + half) of the reference image and of the bearing
 // tables into sh (coordinates outside the image are clamped; only interior
-// pixels, whose taps lie inside the image, read them).  Waits for the previous
-// tile's readers first.
+// pixels, whose taps lie inside the image, read them), and the other colour's
+// planes of the tile and 3 pixels around it (0 outside the image, where no
+// interior pixel's candidate lies).  Waits for the previous tile's readers
+// first.
 template <int R, int NVS>
-__device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, NVS>& sh, int tbx, int tby) {
+__device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, NVS>& sh, const float4* plane, int colour,
+                                              int tbx, int tby) {
     constexpr int NT = 64 * R;
     constexpr int TR = NT / kTileSame;   // tile rows
     const int r0 = tby * TR - a.half, c0 = 2 * kTileSame * tbx - a.half;
     const int nr = TR + 2 * a.half, nc = 2 * kTileSame + 2 * a.half;
     __syncthreads();
+    const int pr0 = tby * TR - 3, pc0 = 2 * kTileSame * tbx - 3;
+    for (int e = threadIdx.x; e < (TR + 6) * kPlaneCols; e += NT) {
+        const int r = e / kPlaneCols, q = e - r * kPlaneCols;
+        const int y = pr0 + r, x = pc0 + 2 * q + ((y + pc0 + colour + 1) & 1);
+        const bool in = y >= 0 && y < a.H && x >= 0 && x < a.W;
+        sh.pl[e] = in ? load_map4(&plane[(size_t)y * a.W + x]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
     for (int e = threadIdx.x; e < nc; e += NT) {
         const int x = min(max(c0 + e, 0), a.W - 1);
         sh.scol[e] = a.coltab[x];
@@ -167,15 +205,21 @@ __device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, NVS
         const int y = min(max(r0 + e, 0), a.H - 1);
         sh.srow[e] = a.rowtab[y];
     }
-    for (int r = 0; r < nr; ++r) {
-        const int y = min(max(r0 + r, 0), a.H - 1);
-        for (int e = threadIdx.x; e < nc; e += NT) {
-            const int x = min(max(c0 + e, 0), a.W - 1);
-            sh.sref[r * kTileCols + e] = a.ref[(size_t)y * a.W + x];
-        }
+    for (int e = threadIdx.x; e < nr * nc; e += NT) {
+        const int r = e / nc, c = e - r * nc;
+        const int y = min(max(r0 + r, 0), a.H - 1), x = min(max(c0 + c, 0), a.W - 1);
+        sh.sref[r * kTileCols + c] = a.ref[(size_t)y * a.W + x];
     }
     __syncthreads();
     return LdsTaps{sh.srow, sh.scol, sh.sref, r0, c0};
+}
+
+// The staged plane of the other colour's pixel (i, j) of tile (tbx, tby) or
+// within 3 pixels of it.
+template <int R, int NVS>
+__device__ __forceinline__ float4 plane_at(const PropShared<R, NVS>& sh, int tbx, int tby, int i, int j) {
+    constexpr int TR = 64 * R / kTileSame;
+    return sh.pl[(i - (tby * TR - 3)) * kPlaneCols + ((j - (2 * kTileSame * tbx - 3)) >> 1)];
 }
 
 // One tile of one red-black pass.  sh.sWc holds a.Wc; rot (a multiple of 64)
@@ -192,19 +236,18 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
     const int i = tby * TR + tid / kTileSame;
     const int j = 2 * (tbx * kTileSame + tid % kTileSame) + ((i + colour) & 1);
     const bool active = i < a.H && j < a.W && in_prop_grid(a, i, j);
-    const int W = a.W;
-    const size_t k = active ? (size_t)i * W + j : 0;
+    const size_t k = active ? (size_t)i * a.W + j : 0;
 
-    const LdsTaps tp = stage_tile(a, sh, tbx, tby);
+    const LdsTaps tp = stage_tile(a, sh, plane, colour, tbx, tby);
     RefStat rs = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     float sc = 0.0f, h0 = 0.0f, h1 = 0.0f, h2 = 0.0f, bx = 0.0f, by = 0.0f, bz = 0.0f, d0 = 1.0f, inv_d0 = 1.0f;
     if (active) {
-        rs = ref_stats(a, sWc, i, j);
-        sc = score[k];
-        const float4 pk = plane[k];
+        sc = load_map(&score[k]);
+        const float4 pk = load_map4(&plane[k]);
+        d0 = load_map(&depth[k]);
+        rs = ref_stats(a, tp, sWc, i, j);
         h0 = pk.x; h1 = pk.y; h2 = pk.z;
-        bearing(a, i, j, bx, by, bz);
-        d0 = depth[k];
+        tap_bearing(tp, i, j, bx, by, bz);
         inv_d0 = rcp(d0);
     }
     sh.rs[tid] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
@@ -218,7 +261,7 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
         for (int c = 0; c < 8; ++c) {
             int di, dj;
             cand_offset(c, di, dj);
-            const float4 pn = plane[(size_t)(i + di) * W + (j + dj)];
+            const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
             float f;
             if (cand_test(a, pn, bx, by, bz, d0, inv_d0, h0, h1, h2, sc, f)) want |= 1u << c;
         }
@@ -260,7 +303,7 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
             const int jc = 2 * (tbx * kTileSame + jl % kTileSame) + ((il + colour) & 1);
             int di, dj;
             cand_offset(c, di, dj);
-            const float4 pn = plane[(size_t)(il + di) * W + (jc + dj)];
+            const float4 pn = plane_at(sh, tbx, tby, il + di, jc + dj);
             const float4 q = sh.rs[jl];
             RefStat r2;
             r2.Ic = sh.ic[jl]; r2.mx = q.x; r2.inv = q.y; r2.mxc = q.z; r2.vx = q.w;
@@ -275,7 +318,7 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
             while (cpos < 8) {
                 int di, dj;
                 cand_offset(cpos, di, dj);
-                const float4 pn = plane[(size_t)(i + di) * W + (j + dj)];
+                const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
                 float f;
                 if (cand_test(a, pn, bx, by, bz, d0, inv_d0, h0, h1, h2, sc, f)) {
                     if (!((listed >> cpos) & 1u)) break;
@@ -291,7 +334,7 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
                     if ((listed >> c) & 1u) continue;
                     int di, dj;
                     cand_offset(c, di, dj);
-                    const float4 pn = plane[(size_t)(i + di) * W + (j + dj)];
+                    const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
                     if (c == cpos || cand_bound(a, pn, bx, by, bz, d0, inv_d0) > sc) want |= 1u << c;
                 }
                 listed |= want;
@@ -322,9 +365,9 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
             ++n_cand;
             if (sh_ > sc) { c0 = q0; c1 = q1; c2 = q2; sc = sh_; dcur = dh; }
         }
-        score[k] = sc;
-        plane[k] = make_float4(c0, c1, c2, 0.0f);
-        depth[k] = depth_of_plane(bx, by, bz, c0, c1, c2);
+        store_map(&score[k], sc);
+        store_map4(&plane[k], make_float4(c0, c1, c2, 0.0f));
+        store_map(&depth[k], depth_of_plane(bx, by, bz, c0, c1, c2));
     }
 }
 
