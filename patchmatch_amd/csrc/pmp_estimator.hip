@@ -133,20 +133,22 @@ int plain_prepare(pmp_ctx* ctx, const pmp_params* p, const uint8_t* dmask, bool 
         memcpy(&kf.view_poses[v], &ctx->view_poses[12 * v], 12 * sizeof(double));
     }
     kf.mask_id = with_mask ? ctx->mask_id : -1;
-    int items[3];
-    rc = slot_fill(ctx, p, kf, ctx->ws, dmask, pass0, q->cfg.tile_rows, ctx->stream, q->plain.h_slots[0], items);
+    int items[2];
+    rc = slot_fill(ctx, p, kf, ctx->ws, dmask, pass0, ctx->stream, q->plain.h_slots[0], items);
     if (rc) {
         if (rc == PMP_ENOTFOUND && with_mask && !dmask && ctx->mask_id >= 0 &&
             ctx->images.find((uint64_t)ctx->mask_id) == ctx->images.end())
             return set_error(ctx, PMP_ENOTFOUND, "mask image was dropped");
         return rc;
     }
+    prop_shape(*q, q->cfg, 1, nullptr, q->plain.h_slots, r);
+    const int tiles = slot_tiles(q->plain.h_slots[0], r.rows);
     fill_list(q->plain.h_hdr->init, 1, &items[0]);
-    fill_list(q->plain.h_hdr->prop, 1, &items[1]);
-    fill_list(q->plain.h_hdr->rows, 1, &items[2]);
-    if ((rc = ensure_sync(ctx, q->plain, (size_t)items[1]))) return rc;
-    if (propagates && (rc = epochs_arm(ctx, ctx->stream, 1, &q->plain.h_slots[0], &items[1], pass0))) return rc;
-    if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0, items[1], r)))
+    fill_list(q->plain.h_hdr->prop, 1, &tiles);
+    fill_list(q->plain.h_hdr->rows, 1, &items[1]);
+    if ((rc = ensure_sync(ctx, q->plain, (size_t)tiles))) return rc;
+    if (propagates && (rc = epochs_arm(ctx, ctx->stream, 1, &q->plain.h_slots[0], &tiles, pass0))) return rc;
+    if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0, tiles, r)))
         return rc;
     if (p->iterations > kMaxPasses / 2) return set_error(ctx, PMP_EINVAL, "iterations must be <= 64");
     return desc_upload(ctx, q->plain, 1, ctx->stream);

@@ -46,6 +46,22 @@ PMP_DF float floor_(float x) { return __builtin_floorf(x); }
 // is zero, which no caller distinguishes)
 PMP_DF float clampf(float x, float lo, float hi) { return __builtin_fminf(__builtin_fmaxf(x, lo), hi); }
 
+// The sign bit, in a vector register: bit operations on vector registers alone
+// issue at twice the rate of those with a scalar operand.
+PMP_DF uint32_t sign_mask() {
+    uint32_t m;
+    asm("v_mov_b32 %0, 0x80000000" : "=v"(m));
+    return m;
+}
+// x with its sign flipped where s is negative (sign bit set)
+PMP_DF float flip_sign(float x, float s) {
+    return u2f(__builtin_amdgcn_bitop3_b32(f2u(x), f2u(s), sign_mask(), 0x78));   // x ^ (s & mask)
+}
+// copysign(a, s) for a with a clear sign bit
+PMP_DF float with_sign(float a, float s) {
+    return u2f(__builtin_amdgcn_bitop3_b32(f2u(a), f2u(s), sign_mask(), 0xF8));   // a | (s & mask)
+}
+
 constexpr float kPi = 3.14159265358979323846f;
 constexpr float kPiO2 = 1.57079632679489661923f;
 
@@ -192,11 +208,11 @@ PMP_DF void lonlat(float x, float y, float z, float& lon, float& lat) {
     float a = asin_oct(med3_(ax, az, 0.0f) * r);
     if (ax > az) a = kPiO2 - a;
     if (z < 0.0f) a = kPi - a;
-    lon = __builtin_copysignf(a, x);
+    lon = with_sign(a, x);
     const float t = abs_(y) * r;
     float b = atan_core(min_(t, rcp_pos(t)));
     if (t > 1.0f) b = kPiO2 - b;
-    lat = __builtin_copysignf(b, y);
+    lat = with_sign(b, y);
 }
 
 // exp(x); x <= -87.3 or NaN -> 0; x >= 88 clamped

@@ -68,7 +68,7 @@ struct BatchHdr {
 // host staging copy, the band heads of the propagation queue, its tiles'
 // arrivals and rings (reached through the header, grown on demand), and the
 // hipGraphs captured over this set's device pointers.
-using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero, rows, blocks, bands, postprocess + 2 fused
+using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero + 2 form, rows, blocks, bands, postprocess + 2 fused
 constexpr int kHeadStride = 32;           // words: every head lies in a cache line of its own
 constexpr int kHeadWords = 24 * kHeadStride;
 struct DescSet {
@@ -89,18 +89,18 @@ struct DescSet {
 struct QueueRun {
     bool zero = false;        // PMP_EDGE_ZERO sampling
     bool post = false;        // any slot post-processes
+    int form = 0;             // how the waves evaluate planes (PropForm)
     int rows = 8;             // tile rows
     int blocks = 0;           // persistent grid
     int bands = 1;            // per-XCD bands
     bool fused = false;       // all passes of a call in one launch
 };
 
-// Default launch shape: 8 x 64 tiles (256-thread blocks), 3 blocks per CU.
-// Measured against 16 x 64 tiles at 2 blocks per CU: 5 % faster on a
-// 1920x960 keyframe with 6 views, 3 % on 960x480 with 3 views, 1 % on
-// 2880x1440 with 10 views (4 blocks per CU were 1-2 % faster still on the
-// last and with zero edges, 2-4 % slower on the first two).
-constexpr pmp_batch_config kDefaultConfig = {4, 3, 1, 1};
+// Default launch shape: the tile rows follow the form that the size and the
+// view count ask for (prop_shape), 2 in small launches, 4 or 8 in large ones;
+// any other setting is taken as it is.  kLane's 8 x 64 tiles, 3 blocks per CU,
+// against 16 x 64 tiles, 2 blocks: 3 % faster on 960x480 with 3 views.
+constexpr pmp_batch_config kDefaultConfig = {2, 0, 1, 1};
 
 struct QueueState {
     pmp_batch_config cfg = kDefaultConfig;
@@ -128,12 +128,19 @@ void desc_free(DescSet& d);
 int desc_begin(pmp_ctx* ctx, DescSet& d);
 int desc_upload(pmp_ctx* ctx, DescSet& d, int n, hipStream_t stream);
 // Descriptor of one keyframe over the maps of b.  dmask (device, nullable)
-// replaces kf.mask_id when given.  items receives the keyframe's init tiles,
-// propagation tiles (for `rows` tile rows) and rows.
+// replaces kf.mask_id when given.  items receives the keyframe's init tiles
+// and rows; its propagation tiles follow from the launch's shape (prop_shape,
+// slot_tiles).
 int slot_fill(pmp_ctx* ctx, const pmp_params* p, const pmp_keyframe& kf, const SlotBuf& b, const uint8_t* dmask,
-              int pass0, int rows, hipStream_t stream, SlotDesc& d, int items[3]);
+              int pass0, hipStream_t stream, SlotDesc& d, int items[2]);
+// Partitions the slot into propagation tiles of `rows` tile rows; their number.
+int slot_tiles(SlotDesc& d, int rows);
+// Evaluation form and tile rows (r.form, r.rows) of a propagation over n filled
+// slots (slots[slot[k]]; slot null: 0..n-1).
+void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
+                QueueRun& r);
 void fill_list(WorkList& L, int n, const int* items);
-// tiles: propagation tiles of a pass.
+// The rest of a shaped run; tiles: propagation tiles of a pass.
 int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
               QueueRun& r);
 int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes);

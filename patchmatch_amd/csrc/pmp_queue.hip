@@ -5,16 +5,15 @@
 //   k_init_q       random init + initial score; items (slot, 64x4 tile), the
 //                  tile's reference taps staged in LDS
 //   k_score_q      score of the working planes; items (slot, 64x4 tile)
-//   k_propagate_q  one red-black pass; items (slot, R x 64 same-colour tile),
-//                  split into 8 contiguous bands, one per XCD, each taken
-//                  through an atomic head (a work queue); a block drains its
-//                  own XCD's band first, then the others
+//   k_propagate_q  one or several red-black passes; items (slot, tile of 64 R
+//                  same-colour pixels), split into 8 contiguous bands, one per
+//                  XCD, each taken through atomic heads (take_tile)
 //   k_copyback_q, k_median_q (x2), k_postfilter_q   finalize; items (slot, row)
 // Descriptors (SlotDesc) and work lists live in device memory and are read
 // with scalar loads (constant address space); launches carry only pointers,
 // so a captured hipGraph of a whole densification replays for any slots with
 // the same iteration count.  The view count is a run-time value (views in
-// groups of 3, 2, 1, per-view scores parked in LDS): one kernel serves
+// groups of at most 4, per-view scores parked in LDS): one kernel serves
 // keyframes of every size and view count in the same launch.
 #include <math.h>
 #include <string.h>
@@ -57,18 +56,28 @@ __global__ void k_fill_u32(unsigned int* __restrict__ p, int n, unsigned int v) 
 // patch and bearing-table entries (the tile plus a halo of half each side,
 // coordinates clamped: only interior pixels, whose taps lie inside the image,
 // read them) are staged in LDS, as for a propagation tile, so that the tap
-// reads never wait behind the neighbour gathers issued before them.
+// reads never wait behind the neighbour gathers issued before them.  The planes
+// are random, so each pixel's patches lie elsewhere and the gathers' cache
+// lines bound the kernel; by quads of lanes (score_wave) a 1920x960 keyframe
+// with 6 views takes 1.05 ms, with a plane per lane 1.32.
 constexpr int kInitRows = 4;
 constexpr int kInitStageRows = kInitRows + 2 * kMaxHalf;
-struct InitStage {
+struct InitShared {
+    QuadTap walk[kQuadTaps];
+    QuadShared quad[kInitRows];
+    float4 rs[64 * kInitRows];
+    float4 plane[64 * kInitRows];
+    float score[64 * kInitRows];
     float2 row[kInitStageRows];
     float2 col[kTileCols];
+    float sWc[256];
+    float ic[64 * kInitRows];
     uint8_t ref[kInitStageRows * kTileCols];
 };
 static_assert(64 + 2 * kMaxHalf <= kTileCols, "init tile columns");
 
 // Waits for the previous tile's readers first.
-__device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitStage& st, int tx, int ty) {
+__device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitShared& st, int tx, int ty) {
     const int r0 = ty * kInitRows - a.half, c0 = 64 * tx - a.half;
     const int nr = kInitRows + 2 * a.half, nc = 64 + 2 * a.half;
     __syncthreads();
@@ -84,38 +93,67 @@ __device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitStage& s
 }
 
 // kScore: only score the working planes (pmp_score_plane_depth); otherwise
-// random initialisation + score + snapshot.
+// random initialisation + score + snapshot (RandomInitialization,
+// PatchMatchCuda.cu:210-270, depthmap.cc:656-663).
 template <bool kZero, bool kScore>
 __global__ __launch_bounds__(256) void k_init_q(const SlotDesc PMP_CONST* slots, const BatchHdr PMP_CONST* hdr) {
-    __shared__ float sWc[256];
-    __shared__ float sv[kMaxViews][256];
-    __shared__ InitStage st;
+    __shared__ InitShared st;
     const WorkList PMP_CONST* L = &hdr->init;
     const int total = L->total;
+    const int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     int cur = -1;
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         int local;
         const int s = list_find(L, item, local);
         const SlotDesc& d = slot_ref(slots, s);
+        const KfArgs& a = d.a;
         if (s != cur) {
             __syncthreads();
-            load_wc(d.a.Wc, sWc);
+            load_wc(a.Wc, st.sWc);
+            load_walk(a, st.walk);
             cur = s;
         }
         const int tx = local % d.nbx_init, ty = local / d.nbx_init;
-        const LdsTaps tp = stage_init_tile(d.a, st, tx, ty);
-        const int j = tx * 64 + (threadIdx.x & 63);
-        const int i = ty * kInitRows + (threadIdx.x >> 6);
-        if (i >= d.a.H || j >= d.a.W) continue;
+        const LdsTaps tp = stage_init_tile(a, st, tx, ty);
+        const int j = tx * 64 + (t & 63);
+        const int i = ty * kInitRows + (t >> 6);
+        const bool in = i < a.H && j < a.W;
+        const bool scored = in && in_score_grid(a, i, j);
+        const size_t k = in ? (size_t)i * a.W + j : 0;
+        float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, dep = 0.0f;
         if constexpr (kScore) {
-            if (!in_score_grid(d.a, i, j)) continue;
-            const size_t k = (size_t)i * d.a.W + j;
-            const RefStat rs = ref_stats(d.a, tp, sWc, i, j);
-            const float4 p = d.plane[k];
-            d.score[k] = score_plane_t<0, kZero>(d.a, tp, sWc, rs, i, j, p.x, p.y, p.z, &sv[0][threadIdx.x], 256);
+            if (scored) {
+                const float4 p = d.plane[k];
+                p0 = p.x; p1 = p.y; p2 = p.z;
+            }
         } else {
-            init_pixel<0, kZero>(d.a, tp, sWc, i, j, d.plane, d.depth, d.score, d.iplane, d.idepth, d.iscore,
-                                 &sv[0][threadIdx.x], 256);
+            if (in && in_init_grid(a, i, j)) random_plane(a, i, j, p0, p1, p2, dep);
+        }
+        RefStat rs = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (scored) rs = ref_stats(a, tp, st.sWc, i, j);
+        st.rs[t] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
+        st.ic[t] = rs.Ic;
+        st.plane[t] = make_float4(p0, p1, p2, 0.0f);
+        wave_exchange();   // a wave reads its own pixels' entries
+        auto at = [&](int p, int& row, int& col) {
+            row = (p >> 6) + a.half;
+            col = (p & 63) + a.half;
+        };
+        auto job = [&](int l, int& jt, float& px, float& py, float& pz) {
+            jt = 64 * wave + l;
+            const float4 p = st.plane[jt];
+            px = p.x; py = p.y; pz = p.z;
+        };
+        auto put = [&](int l, float v) { st.score[64 * wave + l] = v; };
+        score_wave<kZero>(a, tp, st.walk, st.sWc, st.rs, st.ic, at, job, put, __ballot(scored), st.quad[wave]);
+        const float sc = scored ? st.score[t] : __uint_as_float(0xFFFFFFFFu);   // cudaMemset(score, 0xFF) (depthmap.cc:657)
+        if constexpr (kScore) {
+            if (scored) d.score[k] = sc;
+        } else if (in) {
+            const float4 pl = make_float4(p0, p1, p2, 0.0f);
+            d.plane[k] = pl; d.depth[k] = dep; d.score[k] = sc;
+            d.iplane[k] = pl; d.idepth[k] = dep; d.iscore[k] = sc;
         }
     }
 }
@@ -197,9 +235,9 @@ __device__ __forceinline__ int band_lo(int total, int band, int nb) { return (in
 // on few tiles: a 1920x960 keyframe whose bottom eighth starts from random
 // planes and the rest from a warped result took 17.3 ms for 4 passes.)  Called
 // by the block's first wave; lane b < 8 looks at band home + b.
-template <int R, int NVS>
+template <int R, int F>
 __device__ __forceinline__ void take_tile(const BatchHdr PMP_CONST* hdr, int passes, unsigned int* heads, int bands,
-                                          PropShared<R, NVS>& sh) {
+                                          PropShared<R, F>& sh) {
     const int total = hdr->prop.total;
     unsigned int* ring = hdr->sync + 2 * (size_t)total;
     const int nb = bands ? 8 : 1;
@@ -286,16 +324,17 @@ __device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, con
 // One launch over `passes` red-black passes of every slot, the first being
 // pass `first` of the call.
 //
-// The zero-edge variant is held to 4 waves per SIMD (<= 128 VGPRs; left
-// alone it takes 132 and runs at 3 waves, 28 % slower); the wrap/clamp
-// variant fits by itself and is faster with the compiler's own allocation.
-template <bool kZero, int R>
-__global__ __launch_bounds__(64 * R) __attribute__((amdgpu_waves_per_eu(kZero ? 4 : 1))) void k_propagate_q(
+// A block has 64 threads to each wave of its form (prop_shape).
+template <int R, int F>
+constexpr int kPropThreads = 64 * PropShared<R, F>::kWaves;
+template <bool kZero, int R, int F>
+__global__ __launch_bounds__((kPropThreads<R, F>))
+    __attribute__((amdgpu_waves_per_eu(F != kLane || kZero ? 4 : 1))) void k_propagate_q(
     const SlotDesc PMP_CONST* slots, const BatchHdr PMP_CONST* hdr, int first, int passes,
     unsigned int* __restrict__ heads, unsigned long long* __restrict__ counters, int bands) {
-    __shared__ PropShared<R, kMaxViews> sh;
+    __shared__ PropShared<R, F> sh;
     const WorkList PMP_CONST* L = &hdr->prop;
-    unsigned int n_eval = 0, n_cand = 0;
+    unsigned int n_eval = 0, n_cand = 0;   // of the wave
     int cur = -1;
     for (;;) {
         if (threadIdx.x < 64) take_tile(hdr, passes, heads, bands, sh);
@@ -308,18 +347,19 @@ __global__ __launch_bounds__(64 * R) __attribute__((amdgpu_waves_per_eu(kZero ? 
         const SlotDesc& d = slot_ref(slots, s);
         if (s != cur) {
             load_wc(d.a.Wc, sh.sWc);
+            if constexpr (F != kLane) load_walk(d.a, sh.walk);
             cur = s;
         }
         const int pp = d.pass0 + first + pass;
         const int tx = local % d.nbx_prop, ty = local / d.nbx_prop;
         if (d.epochs) epoch_enter(d, tx, ty, pp);
-        propagate_tile<0, kZero, R>(d.a, sh, d.plane, d.depth, d.score, pp >> 1, pp & 1, tx, ty, 64 * (item & (R - 1)),
-                                    n_eval, n_cand);
+        propagate_tile<kZero, R, F>(d.a, sh, d.plane, d.depth, d.score, pp >> 1, pp & 1, tx, ty,
+                                     item & (PropShared<R, F>::kWaves - 1), n_eval, n_cand);
         if (d.epochs) epoch_leave(d, tx, ty, pp);
         if (pass + 1 < passes) release_tiles(hdr, d, heads, bands, item, tx, ty, pass);
     }
-    count_add(&counters[0], n_eval);
-    count_add(&counters[1], n_cand);
+    count_add_wave(&counters[0], n_eval);
+    count_add_wave(&counters[1], n_cand);
 }
 
 __global__ __launch_bounds__(256) void k_copyback_q(const SlotDesc PMP_CONST* slots, const BatchHdr PMP_CONST* hdr) {
@@ -444,7 +484,7 @@ void fill_list(WorkList& L, int n, const int* items) {
 }
 
 int slot_fill(pmp_ctx* ctx, const pmp_params* params, const pmp_keyframe& kf, const SlotBuf& b, const uint8_t* dmask,
-              int pass0, int rows, hipStream_t stream, SlotDesc& d, int items[3]) {
+              int pass0, hipStream_t stream, SlotDesc& d, int items[2]) {
     pmp_params pk = *params;
     if (kf.min_depth > 0.0f) pk.min_depth = kf.min_depth;
     if (kf.max_depth > 0.0f) pk.max_depth = kf.max_depth;
@@ -475,22 +515,80 @@ int slot_fill(pmp_ctx* ctx, const pmp_params* params, const pmp_keyframe& kf, co
     d.nbx_init = (W + 63) / 64;
     d.nbx_prop = ((W + 1) / 2 + kTileSame - 1) / kTileSame;
     items[0] = d.nbx_init * ((H + 3) / 4);
-    const int trows = 64 * rows / kTileSame;   // rows of a propagation tile
-    d.nby_prop = (H + trows - 1) / trows;
-    items[1] = d.nbx_prop * d.nby_prop;
-    items[2] = H;
+    items[1] = H;
     return PMP_OK;
 }
 
-static const void* prop_kernel(bool zero, int rows) {
-    if (zero) {
-        if (rows == 2) return (const void*)k_propagate_q<true, 2>;
-        if (rows == 4) return (const void*)k_propagate_q<true, 4>;
-        return (const void*)k_propagate_q<true, 8>;
+int slot_tiles(SlotDesc& d, int rows) {
+    const int trows = 64 * rows / kTileSame;   // rows of a propagation tile
+    d.nby_prop = (d.a.H + trows - 1) / trows;
+    return d.nbx_prop * d.nby_prop;
+}
+
+// The kernel of a form and tile size, and its block size.  Tiles of 8 rows
+// have no kWide kernel: one block of it would be 2048 threads.
+struct PropKernel {
+    const void* fn;
+    int threads;
+};
+template <bool kZero, int R, int F>
+static PropKernel prop_kernel_of() { return {(const void*)k_propagate_q<kZero, R, F>, kPropThreads<R, F>}; }
+template <bool kZero, int F>
+static PropKernel prop_kernel_f(int rows) {
+    if (rows == 2) return prop_kernel_of<kZero, 2, F>();
+    if (rows == 4) return prop_kernel_of<kZero, 4, F>();
+    return prop_kernel_of<kZero, 8, F == kWide ? kQuad : F>();
+}
+template <bool kZero>
+static PropKernel prop_kernel_z(int form, int rows) {
+    if (form == kLane) return prop_kernel_f<kZero, kLane>(rows);
+    if (form == kWide) return prop_kernel_f<kZero, kWide>(rows);
+    return prop_kernel_f<kZero, kQuad>(rows);
+}
+static PropKernel prop_kernel(bool zero, int form, int rows) {
+    return zero ? prop_kernel_z<true>(form, rows) : prop_kernel_z<false>(form, rows);
+}
+
+static bool is_default(const pmp_batch_config& c) {
+    return c.tile_rows == kDefaultConfig.tile_rows && c.blocks_per_cu == kDefaultConfig.blocks_per_cu;
+}
+
+void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
+                QueueRun& r) {
+    // work: the pixels of one colour in units of 64; chip: waves at four to a SIMD
+    double work = 0.0;
+    int views = 0;
+    for (int k = 0; k < n; ++k) {
+        const KfArgs& a = slots[slot ? slot[k] : k].a;
+        work += (double)a.W * a.H / 128.0;
+        views = std::max(views, (int)a.N);
     }
-    if (rows == 2) return (const void*)k_propagate_q<false, 2>;
-    if (rows == 4) return (const void*)k_propagate_q<false, 4>;
-    return (const void*)k_propagate_q<false, 8>;
+    const double chip = 16.0 * q.cus;
+    // Measured on densifications of 2 and (zero edges) 4 iterations, ms as
+    // kLane / kQuad / kWide, each with the tile rows below:
+    // - Below one and three quarters of the chip kWide: its tiles take four
+    //   times the waves that the other forms have for the same pixels, which
+    //   leave the chip idle there (480x240, 2 views: 2.7 / 3.2 / 1.8; 960x480,
+    //   8 views: 8.3 / 8.1 / 6.9; 1280x640, 8 views: 13.0 / 13.8 / 12.4;
+    //   1440x720, 4 views: 13.8 / 12.4 / -).
+    // - Above, kQuad: a quad's gathers fall into one patch (1920x960: 4 views
+    //   24.5 / 21.4 / 24.6, 6 views, 8 iterations 51.8 / 51.0 / -; 2880x1440,
+    //   10 views: 136 / 124 / -).
+    // - With one to three views some lanes of a quad have no view to
+    //   accumulate, so kLane, where it fills the chip well enough: one view
+    //   from 640x320 (1.06 / 1.3 / 1.13), two from 960x480 (2.39 / 2.53 /
+    //   2.62; 800x400: 1.88 / 2.09 / 1.89), three from there up to 1680x840
+    //   (960x480: 3.3 / 4.4 / 3.3; 1280x640: 5.1 / 5.7 / 5.7; 1680x840, zero
+    //   edges: 13.8 / 13.5 / 16.7).
+    const double lane_from = views == 1 ? 0.375 : 0.75, lane_to = views == 3 ? 2.5 : 1e30;
+    if (views <= 3 && work > lane_from * chip && work < lane_to * chip)
+        r.form = kLane;
+    else
+        r.form = work < 1.75 * chip ? kWide : kQuad;
+    // kQuad, 1920x960: 21.4 ms with 8 rows, 22.4 with 4, 23.2 with 2; kWide,
+    // 640x320, 4 views: 3.4 with 2, 3.5 with 4; kLane: pmp_queue.h
+    r.rows = !is_default(c) ? c.tile_rows : r.form == kLane ? 4 : r.form == kWide ? 2 : 8;
+    if (r.form == kWide && r.rows == 8) r.form = kQuad;
 }
 
 static int check_config(pmp_ctx* ctx, const pmp_batch_config& c) {
@@ -505,23 +603,23 @@ static int check_config(pmp_ctx* ctx, const pmp_batch_config& c) {
 int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
               QueueRun& r) {
     int occ = 0;
-    PMP_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, prop_kernel(zero, c.tile_rows),
-                                                              64 * c.tile_rows, 0));
+    const PropKernel kern = prop_kernel(zero, r.form, r.rows);
+    PMP_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern.fn, kern.threads, 0));
     if (occ < 1) occ = 1;
     int bpc = (c.blocks_per_cu <= 0 || c.blocks_per_cu > occ) ? occ : c.blocks_per_cu;
+    // one plane per lane: with 12 waves' gathers a CU's L1 is full (16 waves: 2-4 % slower)
+    if (c.blocks_per_cu <= 0 && r.form == kLane) bpc = std::min(bpc, std::max(1, 12 / r.rows));
     // blocks beyond one per tile would only look for work
     if (tiles > 0) bpc = std::min(bpc, (tiles + q.cus - 1) / q.cus);
     // One launch over all passes pays where the blocks in flight hold less
-    // than two thirds of the tiles (1920x960, 6 views: 51.5 against 57.9 ms;
-    // 1120x560, 8 views, 4 iterations: 17.7 against 19.9 ms), and where each
-    // tile has a compute unit to itself (480x240, 2 views: 2.9 against
-    // 3.3 ms).  In between most tiles are in flight at once and wait for each
-    // other tile by tile, while the launches' own barrier leaves the last ones
-    // whole compute units (800x400, 4 views, 4 iterations: 10.7 against 6.5 ms).
-    r.fused = tiles <= q.cus || 2 * tiles >= 3 * q.cus * bpc;
+    // than two thirds of the tiles (1920x960, 4 views, 4 iterations: 21.4
+    // against 24.9 ms; 640x320, 4 views: 3.4 against 4.2 ms).  Otherwise most
+    // tiles are in flight at once and wait for each other tile by tile, while
+    // the launches' own barrier leaves the last ones whole compute units
+    // (480x240, 4 views, 4 iterations: 4.4 against 2.4 ms).
+    r.fused = 2 * tiles >= 3 * q.cus * bpc;
     r.zero = zero;
     r.post = post;
-    r.rows = c.tile_rows;
     r.bands = c.xcd_bands ? 1 : 0;
     r.blocks = q.cus * bpc;
     if (r.bands) r.blocks = (r.blocks + 7) / 8 * 8;
@@ -596,21 +694,12 @@ int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
 // One launch over passes [first, first + passes), with the heads of launch `launch`.
 static int launch_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int launch, int first, int passes) {
     PMP_QPTRS
-    const dim3 grd((unsigned)r.blocks), blk((unsigned)(64 * r.rows));
     unsigned int* heads = d.d_heads + (size_t)launch * kHeadWords;
-#define PMP_PROP(Z, R)                                                                                              \
-    hipLaunchKernelGGL((k_propagate_q<Z, R>), grd, blk, 0, s, sl, hd, first, passes, heads, ctx->counters, r.bands)
-    if (r.zero) {
-        if (r.rows == 2) PMP_PROP(true, 2);
-        else if (r.rows == 4) PMP_PROP(true, 4);
-        else PMP_PROP(true, 8);
-    } else {
-        if (r.rows == 2) PMP_PROP(false, 2);
-        else if (r.rows == 4) PMP_PROP(false, 4);
-        else PMP_PROP(false, 8);
-    }
-#undef PMP_PROP
-    PMP_HIP(ctx, hipGetLastError());
+    unsigned long long* counters = ctx->counters;
+    int bands = r.bands;
+    void* args[] = {(void*)&sl, (void*)&hd, &first, &passes, &heads, &counters, &bands};
+    const PropKernel kern = prop_kernel(r.zero, r.form, r.rows);
+    PMP_HIP(ctx, hipLaunchKernel(kern.fn, dim3((unsigned)r.blocks), dim3((unsigned)kern.threads), args, 0, s));
     return PMP_OK;
 }
 
@@ -690,7 +779,7 @@ static int q_sequence(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r
 int q_densify(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes, bool use_graph) {
     // per-stage timing needs events between the launches: no graph then
     if (!use_graph || ctx->timing) return q_sequence(ctx, s, d, r, passes);
-    const GraphKey key{passes, r.zero ? 1 : 0, r.rows, r.blocks, r.bands, (r.post ? 1 : 0) + (r.fused ? 2 : 0)};
+    const GraphKey key{passes, (r.zero ? 1 : 0) + 2 * r.form, r.rows, r.blocks, r.bands, (r.post ? 1 : 0) + (r.fused ? 2 : 0)};
     auto it = d.graphs.find(key);
     if (it == d.graphs.end()) {
         hipGraph_t g = nullptr;
@@ -716,12 +805,12 @@ int q_densify(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int pa
 
 // ---------------------------------------------------------------- batched form
 
-// Descriptors and work lists for n keyframes (all from pass 0), uploaded to
-// the batch set.
+// Descriptors, propagation shape (r) and work lists for n keyframes (all from
+// pass 0), uploaded to the batch set.
 // arm: pass epochs for this batch (pmp_batch_densify; the autotuner reruns
 // passes from the same maps and does not arm them)
 static int batch_prepare(pmp_ctx* ctx, QueueState* q, const pmp_params* params, int n, const pmp_keyframe* kfs,
-                         int rows, bool arm) {
+                         const pmp_batch_config& c, QueueRun& r, bool arm) {
     int rc = check_params(ctx, params);
     if (rc) return rc;
     if (params->iterations > kMaxPasses / 2) return set_error(ctx, PMP_EINVAL, "iterations must be <= 64");
@@ -737,13 +826,14 @@ static int batch_prepare(pmp_ctx* ctx, QueueState* q, const pmp_params* params, 
         auto ir = ctx->images.find(kfs[k].ref_id);
         if (ir == ctx->images.end()) return set_error(ctx, PMP_ENOTFOUND, "unknown reference image id");
         if ((rc = ensure_slot(ctx, q->bufs[k], ir->second.W, ir->second.H))) return rc;
-        int items[3];
-        rc = slot_fill(ctx, params, kfs[k], q->bufs[k], nullptr, 0, rows, ctx->stream, q->batch.h_slots[k], items);
+        int items[2];
+        rc = slot_fill(ctx, params, kfs[k], q->bufs[k], nullptr, 0, ctx->stream, q->batch.h_slots[k], items);
         if (rc) return rc;
         it_init[k] = items[0];
-        it_prop[k] = items[1];
-        it_rows[k] = items[2];
+        it_rows[k] = items[1];
     }
+    prop_shape(*q, c, n, nullptr, q->batch.h_slots, r);
+    for (int k = 0; k < n; ++k) it_prop[k] = slot_tiles(q->batch.h_slots[k], r.rows);
     fill_list(q->batch.h_hdr->init, n, it_init);
     fill_list(q->batch.h_hdr->prop, n, it_prop);
     fill_list(q->batch.h_hdr->rows, n, it_rows);
@@ -767,8 +857,8 @@ int pmp_batch_densify(pmp_ctx* ctx, const pmp_params* params, int32_t n, const p
     int rc = queue_state(ctx, q);
     if (rc) return rc;
     q->n_last = 0;
-    if ((rc = batch_prepare(ctx, q, params, n, kfs, q->cfg.tile_rows, true))) return rc;
     QueueRun r;
+    if ((rc = batch_prepare(ctx, q, params, n, kfs, q->cfg, r, true))) return rc;
     if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0,
                         q->batch.h_hdr->prop.total, r)))
         return rc;
@@ -832,11 +922,11 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
     const int rows_set[3] = {2, 4, 8};
     const bool zero = params->edge_mode == PMP_EDGE_ZERO;
     for (int ri = 0; ri < 3 && rc == 0; ++ri) {
-        if ((rc = batch_prepare(ctx, q, params, n, kfs, rows_set[ri], false))) break;
         pmp_batch_config c = q->cfg;
         c.tile_rows = rows_set[ri];
         c.blocks_per_cu = 32;
         QueueRun r;
+        if ((rc = batch_prepare(ctx, q, params, n, kfs, c, r, false))) break;
         if ((rc = queue_run(ctx, *q, c, zero, false, q->batch.h_hdr->prop.total, r))) break;
         const int occ = r.blocks / (q->cus > 0 ? q->cus : 1);   // blocks per CU that fit (rounding aside)
         // at least 8 waves per CU (rows waves per block): fewer leave SIMDs

@@ -114,15 +114,20 @@ PMP_DF void gather(const KfArgs& a, const uint32_t* __restrict__ base, float u, 
     p.inside = inside;
 }
 
+// The sample times 2^-24.  The four bytes are taken as binary16
+// denormals (byte b is b 2^-24), exact in every step up to the two
+// interpolations, whose roundings a power of two does not change: two byte
+// permutes, one packed subtraction and two mixed-precision fmas instead of
+// four conversions, two subtractions and two fmas.
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+constexpr float kTexelScale = 16777216.0f;             // 2^24
 template <bool kZero>
 PMP_DF float blend(const Pend<kZero>& p) {
-    const uint32_t word = p.word;
-    const float b0 = (float)(word & 0xFFu);           // p(x, y)
-    const float b1 = (float)((word >> 8) & 0xFFu);    // p(x, y+1)
-    const float b2 = (float)((word >> 16) & 0xFFu);   // p(x+1, y)
-    const float b3 = (float)(word >> 24);             // p(x+1, y+1)
-    const float top = fma_(p.fx, b2 - b0, b0);
-    const float bot = fma_(p.fx, b3 - b1, b1);
+    const half2_t l = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(p.word, p.word, 0x0c010c00u));   // p(x, y), p(x, y+1)
+    const half2_t r = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(p.word, p.word, 0x0c030c02u));   // p(x+1, y), p(x+1, y+1)
+    const half2_t d = r - l;
+    const float top = fma_(p.fx, (float)d.x, (float)l.x);
+    const float bot = fma_(p.fx, (float)d.y, (float)l.y);
     const float val = fma_(p.fy, bot - top, top);
     if constexpr (kZero) return p.inside ? val : 0.0f;
     return val;
@@ -132,7 +137,7 @@ template <bool kZero>
 PMP_DF float sample(const KfArgs& a, const uint32_t* __restrict__ base, float u, float v) {
     Pend<kZero> p;
     gather<kZero>(a, base, u, v, p);
-    return blend<kZero>(p);
+    return blend<kZero>(p) * kTexelScale;
 }
 
 // Equirectangular projection (PatchMatchCuda.cu:132-144): the latitude
@@ -243,10 +248,9 @@ PMP_DF float aggregate_rt(const KfArgs& a, const float* sv, int ld) {
 PMP_DF void tap_dir(float bx, float by, float bz, float px, float py, float pz, float& sbx, float& sby, float& sbz,
                     float& as) {
     const float s = fma_(pz, bz, fma_(py, by, px * bx));
-    const uint32_t sg = f2u(s) & 0x80000000u;
-    sbx = u2f(f2u(bx) ^ sg);
-    sby = u2f(f2u(by) ^ sg);
-    sbz = u2f(f2u(bz) ^ sg);
+    sbx = flip_sign(bx, s);
+    sby = flip_sign(by, s);
+    sbz = flip_sign(bz, s);
     as = max_(abs_(s), 1e-6f);
 }
 
@@ -266,7 +270,7 @@ PMP_DF float view_sample(const KfArgs& a, float hu, float hv, const uint32_t* ba
                          float sbz, float as) {
     Pend<kZero> p;
     view_gather<kZero>(a, hu, hv, base, v, sbx, sby, sbz, as, p);
-    return blend<kZero>(p);
+    return blend<kZero>(p) * kTexelScale;
 }
 
 // Where the per-tap inputs of the score come from.  GlobalTaps reads the
@@ -424,7 +428,7 @@ PMP_DF void view_group(const KfArgs& a, const Taps& tp, const float* sWc, const 
         wxc = w * (xs - rs.mx);
     };
     auto accumulate = [&](int g, float val, float w, float wxc) {
-        const float yd = val - shift[g];
+        const float yd = fma_(val, kTexelScale, -shift[g]);
         const float tw = w * yd;
         acc0[g] = acc0[g] + tw;
         acc1[g] = fma_(tw, yd, acc1[g]);
@@ -489,6 +493,219 @@ PMP_DF void emit_views(const KfArgs& a, const RefStat& rs, int v0, const ViewMom
     }
 }
 
+// ---- evaluation by quads
+// Four lanes score one plane at one pixel, each sampling every fourth tap of
+// the walk in every view; one wave scores 16 planes at a time.  The four taps
+// of a quad lie in one patch, mostly a texel or two apart, so a wave's gather
+// touches 16 patches instead of 64.
+// A step of the walk is four taps.  After a step the samples are exchanged
+// through LDS, and lane v of the quad accumulates the moments of view v0 + v
+// over the four taps, in walk order: every sum is the one-lane sum, operation
+// for operation.  The walk's first tap is the centre tap, whose sample is the
+// view's shift (its own terms are exact zeros); the walk is padded to whole
+// steps with taps of weight 0, which add exact zeros.
+// VALU issue bounds it (a wave issues an operation per 8 cycles at most, so the
+// passes want four waves to a SIMD), then the gathers, whose hits cost a CU
+// about 28 cycles for 64 scattered texels and less the closer they lie.  All
+// red-black passes of a 1920x960 keyframe, 4 iterations: with 4 views 20.0 ms,
+// by a plane per lane 21.8; more sizes at prop_shape.
+struct QuadTap {
+    int row, col, ref;   // byte offsets of the tap's row, column and reference pixel from the pixel's own
+    float ws;            // exp(-|k|^2 / (2 sigma_space^2)); 0: padding
+};
+constexpr int kQuadTaps = (kMaxTaps + 3) / 4 * 4;
+
+// One wave's exchange area.
+struct QuadShared {
+    float val[4][64];
+    float w[64], wxc[64];
+    float sv[kMaxViews][16];
+};
+
+// Entry o of the walk table: the o-th tap from the centre tap on.
+PMP_DF QuadTap quad_tap(const KfArgs& a, int o) {
+    const int n = 2 * a.half / a.stride + 1;
+    const bool pad = o >= a.T;
+    int t = a.tc + (pad ? 0 : o);
+    if (t >= a.T) t -= a.T;
+    const int k1 = -a.half + (t / n) * a.stride, k2 = -a.half + (t - (t / n) * n) * a.stride;
+    return QuadTap{8 * k1, 8 * k2, k1 * kTileCols + k2, pad ? 0.0f : a.Ws[t]};
+}
+
+// LDS written by some lanes of a wave and read by others.
+PMP_DF void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Moments of view v0 + q (q = lane & 3 < G) of plane p at the quad's pixel.
+// srow, scol, sref: the pixel's own entries in the tile copies.
+template <int G, bool kZero>
+PMP_DF ViewMom quad_group(const KfArgs& a, const char* srow, const char* scol, const uint8_t* sref, const QuadTap* tab,
+                          const float* sWc, float Ic, float mx, float px, float py, float pz, int v0, QuadShared& qs) {
+    const int lane = threadIdx.x & 63, q = lane & 3;
+    const uint32_t* base[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) base[g] = a.vq[v0 + g];
+    const float hu = in_vgpr(a.hu), hv = in_vgpr(a.hv);
+    const int S = (a.T + 3) >> 2;
+    const QuadTap* tq = tab + q;
+    auto tap = [&](int s, float& sbx, float& sby, float& sbz, float& as, float& w, float& wxc) {
+        const QuadTap e = tq[4 * s];
+        const float2 rt = *(const float2*)(srow + e.row);
+        const float2 ct = *(const float2*)(scol + e.col);
+        tap_dir(rt.x * ct.x, -rt.y, rt.x * ct.y, px, py, pz, sbx, sby, sbz, as);
+        const float xs = (float)sref[e.ref] - Ic;
+        w = sWc[(int)abs_(xs)] * e.ws;
+        wxc = w * (xs - mx);
+    };
+    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, shift = 0.0f;
+    // the step's samples, exchanged: tap k of view q
+    auto accumulate = [&](bool first) {
+        const float4 y = *(const float4*)&qs.val[q][lane & ~3];
+        const float4 w4 = *(const float4*)&qs.w[lane & ~3];
+        const float4 x4 = *(const float4*)&qs.wxc[lane & ~3];
+        shift = first ? y.x * kTexelScale : shift;
+        auto add = [&](float v, float w, float wxc) {
+            const float yd = fma_(v, kTexelScale, -shift);
+            const float tw = w * yd;
+            a0 = a0 + tw;
+            a1 = fma_(tw, yd, a1);
+            a2 = fma_(wxc, yd, a2);
+        };
+        add(y.x, w4.x, x4.x);
+        add(y.y, w4.y, x4.y);
+        add(y.z, w4.z, x4.z);
+        add(y.w, w4.w, x4.w);
+    };
+    Pend<kZero> pd[G];
+    float w, wxc;
+    {
+        float sbx, sby, sbz, as;
+        tap(0, sbx, sby, sbz, as, w, wxc);
+#pragma unroll
+        for (int g = 0; g < G; ++g) view_gather<kZero>(a, hu, hv, base[g], v0 + g, sbx, sby, sbz, as, pd[g]);
+    }
+#pragma unroll 1
+    for (int s = 1; s < S; ++s) {
+        float sbx, sby, sbz, as, nw, nwxc;
+        tap(s, sbx, sby, sbz, as, nw, nwxc);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            qs.val[g][lane] = blend<kZero>(pd[g]);
+            view_gather<kZero>(a, hu, hv, base[g], v0 + g, sbx, sby, sbz, as, pd[g]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        qs.w[lane] = w;
+        qs.wxc[lane] = wxc;
+        wave_exchange();
+        accumulate(s == 1);
+        wave_exchange();
+        w = nw;
+        wxc = nwxc;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) qs.val[g][lane] = blend<kZero>(pd[g]);
+    qs.w[lane] = w;
+    qs.wxc[lane] = wxc;
+    wave_exchange();
+    accumulate(S == 1);
+    wave_exchange();
+    return ViewMom{a0, a1, a2, shift};
+}
+
+// Value of lane k of the quad (k uniform) in all four lanes.
+template <int K>
+PMP_DF float quad_bcast(float x) {
+    return u2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2u(x), K * 0x55, 0xf, 0xf, true));
+}
+
+// Hands a group's moments on, as emit_views: PMP_AGG_REF_FOLD pools them view
+// by view (the running state in rows 0..4 of qs.sv), the other aggregations
+// park each view's own NCC in row v.
+template <int G>
+PMP_DF void quad_emit(const KfArgs& a, const float4& r4, int v0, const ViewMom& m, QuadShared& qs) {
+    const RefStat rs{0.0f, r4.x, r4.y, r4.z, r4.w};
+    const int lane = threadIdx.x & 63, q = lane & 3, pix = lane >> 2;
+    if (a.agg_mode == PMP_AGG_REF_FOLD) {
+        Pool st{0.0f, 0.0f, 0.0f, 0.0f, -1.0f};
+        if (v0 > 0) st = Pool{qs.sv[0][pix], qs.sv[1][pix], qs.sv[2][pix], qs.sv[3][pix], qs.sv[4][pix]};
+        pool_view(a, rs, st, a.rn[v0], quad_bcast<0>(m.a0), quad_bcast<0>(m.a1), quad_bcast<0>(m.a2), quad_bcast<0>(m.sh));
+        if constexpr (G > 1)
+            pool_view(a, rs, st, a.rn[v0 + 1], quad_bcast<1>(m.a0), quad_bcast<1>(m.a1), quad_bcast<1>(m.a2),
+                      quad_bcast<1>(m.sh));
+        if constexpr (G > 2)
+            pool_view(a, rs, st, a.rn[v0 + 2], quad_bcast<2>(m.a0), quad_bcast<2>(m.a1), quad_bcast<2>(m.a2),
+                      quad_bcast<2>(m.sh));
+        if constexpr (G > 3)
+            pool_view(a, rs, st, a.rn[v0 + 3], quad_bcast<3>(m.a0), quad_bcast<3>(m.a1), quad_bcast<3>(m.a2),
+                      quad_bcast<3>(m.sh));
+        if (q == 0) {
+            qs.sv[0][pix] = st.C;
+            qs.sv[1][pix] = st.V;
+            qs.sv[2][pix] = st.mu;
+            qs.sv[3][pix] = st.q;
+            qs.sv[4][pix] = st.s;
+        }
+    } else {
+        const float s = ncc(rs, a.var_floor, m.a0, m.a1, m.a2);
+        if (q < G) qs.sv[v0 + q][pix] = s;
+    }
+}
+
+// Scores up to 64 planes of a wave: job(l, t, px, py, pz) gives plane l and its
+// pixel t of the tile (rs and ic hold the pixels' reference moments; at(t)
+// gives a pixel's row and column in the tile copies), put(l, score) takes its
+// score.  Jobs whose bit of `live` is 0 are not put (job must still give a
+// pixel of the tile for them); live, and the whole call, are the same in all
+// 64 lanes.  A round scores 16 planes; a round without any is skipped.
+template <bool kZero, class At, class Job, class Put>
+PMP_DF void score_wave(const KfArgs& a, const LdsTaps& tp, const QuadTap* tab, const float* sWc, const float4* rs,
+                       const float* ic, const At& at, const Job& job, const Put& put, unsigned long long live,
+                       QuadShared& qs) {
+    const int lane = threadIdx.x & 63;
+    const int N = a.N;
+#pragma unroll 1
+    for (int r = 0; r < 4; ++r) {
+        if (((unsigned int)(live >> (16 * r)) & 0xFFFFu) == 0u) continue;
+        const int l = 16 * r + (lane >> 2);
+        int t, row, col;
+        float px, py, pz;
+        job(l, t, px, py, pz);
+        at(t, row, col);
+        const char* srow = (const char*)(tp.srow + row);
+        const char* scol = (const char*)(tp.scol + col);
+        const uint8_t* sref = tp.sref + row * kTileCols + col;
+        const float Ic = ic[t], mx = rs[t].x;
+        // as few groups of at most 4 views as there can be, of even sizes
+        int left = (N + 3) >> 2;
+#pragma unroll 1
+        for (int v0 = 0; left > 0; --left) {
+            const int G = (N - v0 + left - 1) / left;
+            if (G == 4) {
+                const ViewMom m = quad_group<4, kZero>(a, srow, scol, sref, tab, sWc, Ic, mx, px, py, pz, v0, qs);
+                quad_emit<4>(a, rs[t], v0, m, qs);
+            } else if (G == 3) {
+                const ViewMom m = quad_group<3, kZero>(a, srow, scol, sref, tab, sWc, Ic, mx, px, py, pz, v0, qs);
+                quad_emit<3>(a, rs[t], v0, m, qs);
+            } else if (G == 2) {
+                const ViewMom m = quad_group<2, kZero>(a, srow, scol, sref, tab, sWc, Ic, mx, px, py, pz, v0, qs);
+                quad_emit<2>(a, rs[t], v0, m, qs);
+            } else {
+                const ViewMom m = quad_group<1, kZero>(a, srow, scol, sref, tab, sWc, Ic, mx, px, py, pz, v0, qs);
+                quad_emit<1>(a, rs[t], v0, m, qs);
+            }
+            wave_exchange();
+            v0 += G;
+        }
+        const float sc = a.agg_mode == PMP_AGG_REF_FOLD ? qs.sv[4][lane >> 2] : aggregate_rt(a, &qs.sv[0][lane >> 2], 16);
+        wave_exchange();
+        if ((lane & 3) == 0 && ((live >> l) & 1u)) put(l, sc);
+    }
+    wave_exchange();
+}
+
 // Score of plane (px, py, pz) at pixel (i, j); kZero selects PMP_EDGE_ZERO
 // sampling.  a.N views (uniform) in groups of 3, 2 or 1; between groups the
 // per-view scores (or the pooled state) are parked in LDS at sv[r * ld], r <
@@ -517,6 +734,24 @@ PMP_DF float score_plane_t(const KfArgs& a, const Taps& tp, const float* sWc, co
     }
     if (a.agg_mode == PMP_AGG_REF_FOLD) return sv[4 * ld];
     return aggregate_rt(a, sv, ld);
+}
+
+// One plane per lane: the same call with score_wave's arguments.  sv: kMaxViews
+// rows of 64 floats, the wave's own.
+template <bool kZero, class At, class Job, class Put>
+PMP_DF void score_lanes(const KfArgs& a, const LdsTaps& tp, const float* sWc, const float4* rs, const float* ic,
+                        const At& at, const Job& job, const Put& put, unsigned long long live, float* sv) {
+    const int lane = threadIdx.x & 63;
+    if ((live >> lane) & 1u) {
+        int t, row, col;
+        float px, py, pz;
+        job(lane, t, px, py, pz);
+        at(t, row, col);
+        const float4 r4 = rs[t];
+        const RefStat r{ic[t], r4.x, r4.y, r4.z, r4.w};
+        put(lane, score_plane_t<0, kZero>(a, tp, sWc, r, tp.r0 + row, tp.c0 + col, px, py, pz, sv + lane, 64));
+    }
+    wave_exchange();
 }
 
 template <int NV, bool kZero>
@@ -571,17 +806,22 @@ PMP_DF void random_plane(const KfArgs& a, int i, int j, float& p0, float& p1, fl
     plane_from_depth_normal(bx, by, bz, dep, nx, ny, nz, p0, p1, p2);
 }
 
-// Standard normals n of (pixel, iteration): counter (pixel, it, block, "RFNE").
+// Standard normals 4 b .. 4 b + 3 of (pixel, iteration): counter (pixel, it, b, "RFNE").
+PMP_DF void refine_block(const KfArgs& a, uint32_t pix, int it, int b, float& z0, float& z1, float& z2, float& z3) {
+    const u32x4 r = philox(pix, (uint32_t)it, (uint32_t)b, kStreamRefine, a.key0, a.key1);
+    box_muller(r.x, r.y, &z0, &z1);
+    box_muller(r.z, r.w, &z2, &z3);
+}
+
+// The first n of them.
 template <int NMAX>
 PMP_DF void refine_normals(const KfArgs& a, int i, int j, int it, int n, float (&z)[NMAX]) {
     const uint32_t pix = (uint32_t)(i * a.W + j);
 #pragma unroll
     for (int b = 0; b < (NMAX + 3) / 4; ++b) {
         if (4 * b < n) {
-            u32x4 r = philox(pix, (uint32_t)it, (uint32_t)b, kStreamRefine, a.key0, a.key1);
             float z0, z1, z2, z3;
-            box_muller(r.x, r.y, &z0, &z1);
-            box_muller(r.z, r.w, &z2, &z3);
+            refine_block(a, pix, it, b, z0, z1, z2, z3);
             if (4 * b + 0 < NMAX) z[4 * b + 0] = z0;
             if (4 * b + 1 < NMAX) z[4 * b + 1] = z1;
             if (4 * b + 2 < NMAX) z[4 * b + 2] = z2;

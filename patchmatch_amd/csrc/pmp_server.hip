@@ -175,6 +175,7 @@ class GpuExec final : public sched::Executor {
         TraceRange trace_range("pmp_server step");
         DescSet& d = desc[w];
         int items_init[kMaxSlots] = {0}, items_prop[kMaxSlots] = {0}, items_rows[kMaxSlots] = {0};
+        std::vector<int> props;
         bool post = false;
         std::vector<const sched::StepItem*> fin, seeds, warms;
         int rc = PMP_OK;
@@ -191,10 +192,9 @@ class GpuExec final : public sched::Executor {
                 SlotBuf& b = slots[it.slot];
                 b.W = j->W;
                 b.H = j->H;
-                int its[3];
+                int its[2];
                 const int pass0 = it.stage >= 1 && it.stage < j->last_stage ? it.stage - 1 : 0;
-                const int frc = slot_fill(ctx, &j->p, j->kf, b, nullptr, pass0, cfg.tile_rows, ctx->stream,
-                                          d.h_slots[it.slot], its);
+                const int frc = slot_fill(ctx, &j->p, j->kf, b, nullptr, pass0, ctx->stream, d.h_slots[it.slot], its);
                 if (frc) {
                     item_rc[k] = frc;
                     item_err[k] = ctx->last_error;
@@ -205,19 +205,21 @@ class GpuExec final : public sched::Executor {
                     if (j->n_lm > 0) seeds.push_back(&it);
                     if (j->prev_plane4) warms.push_back(&it);
                 } else if (it.stage < j->last_stage) {
-                    items_prop[it.slot] = its[1];
+                    props.push_back(it.slot);
                 } else {
-                    items_rows[it.slot] = its[2];
+                    items_rows[it.slot] = its[1];
                     post = post || j->p.postprocess;
                     fin.push_back(&it);
                 }
             }
         }
         const int n = (int)slots.size();
+        QueueRun run;
+        prop_shape(*ctx->queue, cfg, (int)props.size(), props.data(), d.h_slots, run);
+        for (int s : props) items_prop[s] = slot_tiles(d.h_slots[s], run.rows);
         fill_list(d.h_hdr->init, n, items_init);
         fill_list(d.h_hdr->prop, n, items_prop);
         fill_list(d.h_hdr->rows, n, items_rows);
-        QueueRun run;
         rc = queue_run(ctx, *ctx->queue, cfg, edge_mode == PMP_EDGE_ZERO, post, d.h_hdr->prop.total, run);
         if (!rc) rc = desc_upload(ctx, d, n, ctx->stream);
         if (!rc) rc = q_clear(ctx, ctx->stream, d, run, 1);

@@ -2,6 +2,8 @@
 // kernels (pmp_estimator.hip) and the work-queue kernels over many keyframes
 // (pmp_batch.hip).
 #pragma once
+#include <type_traits>
+
 #include "pmp_internal.h"
 #include "pmp_math.h"
 #include "pmp_score.h"
@@ -21,6 +23,11 @@ __device__ __forceinline__ void count_add(unsigned long long* ctr, unsigned int 
     if ((threadIdx.x & 63) == 0 && s) atomicAdd(ctr, (unsigned long long)s);
 }
 
+// The same for a count that is the wave's, not the lane's.
+__device__ __forceinline__ void count_add_wave(unsigned long long* ctr, unsigned int v) {
+    if ((threadIdx.x & 63) == 0 && v) atomicAdd(ctr, (unsigned long long)v);
+}
+
 // Workgroups are dispatched to the 8 XCDs round-robin by linear block id.  The
 // grid is padded to a multiple of 8 and block b is given tile
 // (b mod 8) * (nb8/8) + b/8, so each XCD walks one contiguous band of tiles
@@ -30,43 +37,27 @@ __device__ __forceinline__ int xcd_tile(int b, int nb8, int nb) {
     return t < nb ? t : -1;
 }
 
-// Random hypothesis, initial score and snapshot of pixel (i, j)
-// (RandomInitialization, PatchMatchCuda.cu:210-270, depthmap.cc:656-663).
-// sv/ld: per-view score scratch of the calling thread (NV == 0 only); tp:
-// where the reference taps come from (GlobalTaps or a staged LdsTaps).
-template <int NV, bool kZero, class Taps>
-__device__ __forceinline__ void init_pixel(const KfArgs& a, const Taps& tp, const float* sWc, int i, int j,
-                                           float4* __restrict__ plane, float* __restrict__ depth,
-                                           float* __restrict__ score, float4* __restrict__ iplane,
-                                           float* __restrict__ idepth, float* __restrict__ iscore,
-                                           float* sv = nullptr, int ld = 0) {
-    float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, dep = 0.0f;
-    if (in_init_grid(a, i, j)) random_plane(a, i, j, p0, p1, p2, dep);
-    float sc = __uint_as_float(0xFFFFFFFFu);   // cudaMemset(score, 0xFF) (depthmap.cc:657)
-    if (in_score_grid(a, i, j)) {
-        RefStat rs = ref_stats(a, tp, sWc, i, j);
-        sc = score_plane_t<NV, kZero>(a, tp, sWc, rs, i, j, p0, p1, p2, sv, ld);
-    }
-    const size_t k = (size_t)i * a.W + j;
-    const float4 pl = make_float4(p0, p1, p2, 0.0f);
-    plane[k] = pl; depth[k] = dep; score[k] = sc;
-    iplane[k] = pl; idepth[k] = dep; iscore[k] = sc;
+// The same for a keyframe's tap walk (quad_tap).
+__device__ __forceinline__ void load_walk(const KfArgs& a, QuadTap* tab) {
+    const int n = (a.T + 3) / 4 * 4;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) tab[k] = quad_tap(a, k);
+    __syncthreads();
 }
 
 // ---- red-black pass
-// A tile is 2R rows x 32 same-colour pixels (64 columns); thread t of the
-// 64R-thread block updates row i = 2R by + t / 32, column
-// j = 2 (32 bx + t % 32) + ((i + colour) & 1), i.e. every pixel of colour
-// (i+j)&1 == colour once (each wave covers two rows).  Candidates are at odd
+// A tile is 2R rows x 32 same-colour pixels (64 columns); its pixel t < 64R is
+// at row i = 2R by + t / 32, column j = 2 (32 bx + t % 32) + ((i + colour) & 1),
+// i.e. every pixel of colour (i+j)&1 == colour once.  A thread owns one pixel
+// (kWide: a quarter of a wave's threads do) and decides for it.  Candidates are at odd
 // distance (1 or 3), so they have the other colour and are not written by
 // this pass.
 //
-// Propagation candidates are scored by whichever threads of the block are
+// Propagation candidates are scored by whichever waves of the block are
 // free, in packed sweeps, and their raw scores handed back to the owning
 // threads, which apply the penalty and the acceptance test in candidate order:
 //   1. every pixel tests its 8 candidates against its state at entry (the
 //      exact pre-rejection below); the (candidate, pixel) pairs that pass are
-//      listed candidate-major and scored in one sweep over the block's threads;
+//      listed candidate-major and scored in one sweep over the block's waves;
 //   2. each pixel then walks its candidates in order against its running state
 //      (the test is repeated: an acceptance changes the plane and the score it
 //      is tested against).  A candidate that passes there but did not pass at
@@ -77,32 +68,55 @@ __device__ __forceinline__ void init_pixel(const KfArgs& a, const Taps& tp, cons
 //      stops again, so a tile takes at most two sweeps.
 // A candidate's raw score depends only on its plane and the pixel, so where
 // and when it is computed does not matter: each pixel's sequence of decisions
-// is that of the one-thread-per-pixel loop, and the results are identical.
+// is that of a loop over its own candidates, and the results are identical.
 // Scores computed for candidates that an acceptance makes unnecessary are
 // spent work (counted as evaluations).
-// NVS: per-view score scratch rows (kMaxViews for the run-time view count, 1
-// otherwise).
 // srow/scol/sref: the tile's rows and columns of the bearing tables and of
 // the reference image, with the patch halo (LdsTaps).
 // pl: the other colour's planes of the tile and 3 pixels around it, where its
-// candidates are (plane_at).
-// res[c * 64R + t]: raw score of candidate c of thread t's pixel; job: the
-// sweep's (candidate << 9 | thread) list.
+// candidates are (cand_plane).
+// walk: the keyframe's tap walk; eval: each wave's exchange area; rs, ic: the
+// pixels' reference moments.
+// res[c * 64R + t]: raw score of candidate c of pixel t; job: the sweep's
+// (candidate << 9 | pixel) list.
 constexpr int kPlaneCols = kTileSame + 3;   // one colour's pixels in a row of the tile and 3 columns each side
-template <int R, int NVS = 1>
+// How a propagation block evaluates planes: kLane one per lane, 64 to a wave;
+// kQuad one per four lanes; kWide as kQuad with four times the waves to a tile
+// (chosen by prop_shape).
+enum PropForm { kLane = 0, kQuad = 1, kWide = 2 };
+struct LaneShared {
+    float sv[kMaxViews][64];
+};
+template <int R, int F>
 struct PropShared {
-    float sWc[256];
-    float sv[NVS][64 * R];
-    float res[8 * 64 * R];
-    float4 rs[64 * R];
-    float ic[64 * R];
-    uint16_t job[8 * 64 * R];
-    float2 srow[64 * R / kTileSame + 2 * kMaxHalf];
+    static constexpr int kPix = 64 * R;              // pixels of a tile
+    static constexpr int kOwn = F == kWide ? 16 : 64;   // of them, a wave's own
+    static constexpr int kWaves = kPix / kOwn;
+    static constexpr int kRows = kPix / kTileSame;   // tile rows
+    QuadTap walk[F == kLane ? 1 : kQuadTaps];
+    std::conditional_t<F == kLane, LaneShared, QuadShared> eval[kWaves];
+    float4 rs[kPix];
+    union {
+        float4 pl[(kRows + 6) * kPlaneCols];
+        struct {                      // a refinement trial: its planes and their scores
+            float4 trial[kPix];
+            float trial_score[kPix];
+        };
+    };
+    float2 srow[kRows + 2 * kMaxHalf];
     float2 scol[kTileCols];
-    uint8_t sref[(64 * R / kTileSame + 2 * kMaxHalf) * kTileCols];
-    float4 pl[(64 * R / kTileSame + 6) * kPlaneCols];
-    int cnt[8 * R];
+    float sWc[256];
+    union {
+        struct {
+            float res[8 * kPix];
+            uint16_t job[8 * kPix];
+        };
+        float z[12 * kPix];           // normals of four refinement trials per pixel
+    };
+    float ic[kPix];
+    int cnt[8 * kWaves];
     int item, pass;
+    uint8_t sref[(kRows + 2 * kMaxHalf) * kTileCols];
 };
 
 // The maps that tiles of one launch hand each other (pass fusion: a tile of
@@ -182,11 +196,11 @@ __device__ __forceinline__ bool cand_test(const KfArgs& a, float4 pn, float bx, 
 // planes of the tile and 3 pixels around it (0 outside the image, where no
 // interior pixel's candidate lies).  Waits for the previous tile's readers
 // first.
-template <int R, int NVS>
-__device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, NVS>& sh, const float4* plane, int colour,
+template <int R, int F>
+__device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, F>& sh, const float4* plane, int colour,
                                               int tbx, int tby) {
-    constexpr int NT = 64 * R;
-    constexpr int TR = NT / kTileSame;   // tile rows
+    constexpr int NT = 64 * PropShared<R, F>::kWaves;
+    constexpr int TR = PropShared<R, F>::kRows;
     const int r0 = tby * TR - a.half, c0 = 2 * kTileSame * tbx - a.half;
     const int nr = TR + 2 * a.half, nc = 2 * kTileSame + 2 * a.half;
     __syncthreads();
@@ -214,54 +228,76 @@ __device__ __forceinline__ LdsTaps stage_tile(const KfArgs& a, PropShared<R, NVS
     return LdsTaps{sh.srow, sh.scol, sh.sref, r0, c0};
 }
 
-// The staged plane of the other colour's pixel (i, j) of tile (tbx, tby) or
-// within 3 pixels of it.
-template <int R, int NVS>
-__device__ __forceinline__ float4 plane_at(const PropShared<R, NVS>& sh, int tbx, int tby, int i, int j) {
-    constexpr int TR = 64 * R / kTileSame;
-    return sh.pl[(i - (tby * TR - 3)) * kPlaneCols + ((j - (2 * kTileSame * tbx - 3)) >> 1)];
+// The staged plane of candidate c of the tile's pixel t.
+template <int R, int F>
+__device__ __forceinline__ float4 cand_plane(const PropShared<R, F>& sh, int t, int colour, int tby, int c) {
+    int di, dj;
+    cand_offset(c, di, dj);
+    const int row = t / kTileSame;
+    const int col = 2 * (t % kTileSame) + ((tby * PropShared<R, F>::kRows + row + colour) & 1);
+    return sh.pl[(row + di + 3) * kPlaneCols + ((col + dj + 3) >> 1)];
 }
 
-// One tile of one red-black pass.  sh.sWc holds a.Wc; rot (a multiple of 64)
-// is the slot offset where the packed jobs start.
-template <int NV, bool kZero, int R, int NVS>
-__device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NVS>& sh, float4* __restrict__ plane,
+// One tile of one red-black pass by a block whose waves own PW pixels each
+// (pixel t = PW wave + lane, lanes beyond PW own none but take part in the
+// evaluations).  sh.sWc and sh.walk hold the keyframe's tables; rot is the wave
+// that takes the first packed jobs.
+template <bool kZero, int R, int F>
+__device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, F>& sh, float4* __restrict__ plane,
                                                float* __restrict__ depth, float* __restrict__ score, int it,
                                                int colour, int tbx, int tby, int rot, unsigned int& n_eval,
                                                unsigned int& n_cand) {
-    constexpr int NT = 64 * R;
+    using Sh = PropShared<R, F>;
+    constexpr int NP = Sh::kPix, NW = Sh::kWaves, TR = Sh::kRows, PW = Sh::kOwn;
+    constexpr int NJ = F == kLane ? 64 : 16;   // planes a wave scores at a time
     const float* sWc = sh.sWc;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int TR = NT / kTileSame;   // tile rows
-    const int i = tby * TR + tid / kTileSame;
-    const int j = 2 * (tbx * kTileSame + tid % kTileSame) + ((i + colour) & 1);
-    const bool active = i < a.H && j < a.W && in_prop_grid(a, i, j);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const bool owner = PW == 64 || lane < PW;
+    const int t = PW * wave + (owner ? lane : 0);
+    const int i = tby * TR + t / kTileSame;
+    const int j = 2 * (tbx * kTileSame + t % kTileSame) + ((i + colour) & 1);
+    const bool active = owner && i < a.H && j < a.W && in_prop_grid(a, i, j);
     const size_t k = active ? (size_t)i * a.W + j : 0;
+    // row and column of pixel p in the tile copies
+    auto at = [&](int p, int& row, int& col) {
+        const int y = p / kTileSame;
+        row = y + a.half;
+        col = 2 * (p % kTileSame) + ((tby * TR + y + colour) & 1) + a.half;
+    };
 
     const LdsTaps tp = stage_tile(a, sh, plane, colour, tbx, tby);
-    RefStat rs = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    auto evaluate = [&](const auto& job, const auto& put, unsigned long long live) {
+        if constexpr (F == kLane)
+            score_lanes<kZero>(a, tp, sWc, sh.rs, sh.ic, at, job, put, live, &sh.eval[wave].sv[0][0]);
+        else
+            score_wave<kZero>(a, tp, sh.walk, sWc, sh.rs, sh.ic, at, job, put, live, sh.eval[wave]);
+    };
     float sc = 0.0f, h0 = 0.0f, h1 = 0.0f, h2 = 0.0f, bx = 0.0f, by = 0.0f, bz = 0.0f, d0 = 1.0f, inv_d0 = 1.0f;
-    if (active) {
-        sc = load_map(&score[k]);
-        const float4 pk = load_map4(&plane[k]);
-        d0 = load_map(&depth[k]);
-        rs = ref_stats(a, tp, sWc, i, j);
-        h0 = pk.x; h1 = pk.y; h2 = pk.z;
-        tap_bearing(tp, i, j, bx, by, bz);
-        inv_d0 = rcp(d0);
+    {
+        RefStat rs = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (active) {
+            sc = load_map(&score[k]);
+            const float4 pk = load_map4(&plane[k]);
+            d0 = load_map(&depth[k]);
+            rs = ref_stats(a, tp, sWc, i, j);
+            h0 = pk.x; h1 = pk.y; h2 = pk.z;
+            tap_bearing(tp, i, j, bx, by, bz);
+            inv_d0 = rcp(d0);
+        }
+        if (owner) {
+            sh.rs[t] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
+            sh.ic[t] = rs.Ic;
+        }
     }
-    sh.rs[tid] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
-    sh.ic[tid] = rs.Ic;
 
     // 1. propagation (PatchMatchCuda.cu:311-338), in the order of cand_offset
     unsigned int want = 0;     // bit c: candidate c is to be scored in the next sweep
+    const unsigned long long alive = __ballot(active);
+    n_cand += (unsigned int)__popcll(alive) * (8u + (unsigned int)a.n_refine);
     if (active) {
-        n_cand += 8;
 #pragma unroll 1
         for (int c = 0; c < 8; ++c) {
-            int di, dj;
-            cand_offset(c, di, dj);
-            const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
+            const float4 pn = cand_plane(sh, t, colour, tby, c);
             float f;
             if (cand_test(a, pn, bx, by, bz, d0, inv_d0, h0, h1, h2, sc, f)) want |= 1u << c;
         }
@@ -274,7 +310,7 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
 #pragma unroll 1
         for (int c = 0; c < 8; ++c) {
             const unsigned long long bal = __ballot((want >> c) & 1u);
-            if (lane == 0) sh.cnt[c * R + wave] = __popcll(bal);
+            if (lane == 0) sh.cnt[c * NW + wave] = __popcll(bal);
         }
         __syncthreads();
         int J = 0;
@@ -282,33 +318,35 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
         for (int c = 0; c < 8; ++c) {
             int woff = 0, tot = 0;
 #pragma unroll
-            for (int w = 0; w < R; ++w) {
-                const int cw = sh.cnt[c * R + w];
+            for (int w = 0; w < NW; ++w) {
+                const int cw = sh.cnt[c * NW + w];
                 woff += (w < wave) ? cw : 0;
                 tot += cw;
             }
             const bool on = (want >> c) & 1u;
             const unsigned long long bal = __ballot(on);
-            if (on) sh.job[J + woff + __popcll(bal & ((1ull << lane) - 1ull))] = (uint16_t)((c << 9) | tid);
+            if (on) sh.job[J + woff + __popcll(bal & ((1ull << lane) - 1ull))] = (uint16_t)((c << 9) | t);
             J += tot;
         }
+        J = __builtin_amdgcn_readfirstlane(J);
         if (J == 0) break;   // the same in every thread
         __syncthreads();
-        // score the list: job g by thread (g + rot) mod NT
+        // score the list: NJ jobs per wave and turn, from wave rot on
 #pragma unroll 1
-        for (int g = (tid - rot) & (NT - 1); g < J; g += NT) {
-            const unsigned int e = sh.job[g];
-            const int c = (int)(e >> 9), jl = (int)(e & 511u);
-            const int il = tby * TR + jl / kTileSame;
-            const int jc = 2 * (tbx * kTileSame + jl % kTileSame) + ((il + colour) & 1);
-            int di, dj;
-            cand_offset(c, di, dj);
-            const float4 pn = plane_at(sh, tbx, tby, il + di, jc + dj);
-            const float4 q = sh.rs[jl];
-            RefStat r2;
-            r2.Ic = sh.ic[jl]; r2.mx = q.x; r2.inv = q.y; r2.mxc = q.z; r2.vx = q.w;
-            sh.res[c * NT + jl] = score_plane_t<NV, kZero>(a, tp, sWc, r2, il, jc, pn.x, pn.y, pn.z, &sh.sv[0][tid], NT);
-            ++n_eval;
+        for (int g0 = NJ * ((wave - rot) & (NW - 1)); g0 < J; g0 += NJ * NW) {
+            const int n = min(J - g0, NJ);
+            auto job = [&](int l, int& jt, float& px, float& py, float& pz) {
+                const unsigned int e = sh.job[g0 + (l < n ? l : 0)];
+                jt = (int)(e & 511u);
+                const float4 pn = cand_plane(sh, jt, colour, tby, (int)(e >> 9));
+                px = pn.x; py = pn.y; pz = pn.z;
+            };
+            auto put = [&](int l, float s) {
+                const unsigned int e = sh.job[g0 + l];
+                sh.res[(e >> 9) * NP + (e & 511u)] = s;
+            };
+            evaluate(job, put, ~0ull >> (64 - n));
+            n_eval += n;
         }
         __syncthreads();
         // walk the candidates in order against the running state, up to the
@@ -316,13 +354,11 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
         want = 0;
         if (active) {
             while (cpos < 8) {
-                int di, dj;
-                cand_offset(cpos, di, dj);
-                const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
+                const float4 pn = cand_plane(sh, t, colour, tby, cpos);
                 float f;
                 if (cand_test(a, pn, bx, by, bz, d0, inv_d0, h0, h1, h2, sc, f)) {
                     if (!((listed >> cpos) & 1u)) break;
-                    const float sh_ = sh.res[cpos * NT + tid] * f;
+                    const float sh_ = sh.res[cpos * NP + t] * f;
                     if (sh_ > sc) { h0 = pn.x; h1 = pn.y; h2 = pn.z; sc = sh_; }
                 }
                 ++cpos;
@@ -332,39 +368,62 @@ __device__ __forceinline__ void propagate_tile(const KfArgs& a, PropShared<R, NV
 #pragma unroll 1
                 for (int c = cpos; c < 8; ++c) {
                     if ((listed >> c) & 1u) continue;
-                    int di, dj;
-                    cand_offset(c, di, dj);
-                    const float4 pn = plane_at(sh, tbx, tby, i + di, j + dj);
+                    const float4 pn = cand_plane(sh, t, colour, tby, c);
                     if (c == cpos || cand_bound(a, pn, bx, by, bz, d0, inv_d0) > sc) want |= 1u << c;
                 }
                 listed |= want;
             }
         }
     }
+    // 2. refinement (PatchMatchCuda.cu:340-395); its normals and planes lie where
+    // the sweeps' scores, lists and planes were, which the other waves may
+    // still read
+    __syncthreads();
+    float dcur = 1.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
     if (active) {
-        // 2. refinement (PatchMatchCuda.cu:340-395)
-        float dcur = depth_of_plane(bx, by, bz, h0, h1, h2);
-        float c0 = h0, c1 = h1, c2 = h2;
-        float z[3 * kMaxRefine];
-        refine_normals<3 * kMaxRefine>(a, i, j, it, 3 * a.n_refine, z);
+        dcur = depth_of_plane(bx, by, bz, h0, h1, h2);
+        c0 = h0; c1 = h1; c2 = h2;
+    }
 #pragma unroll 1
-        for (int t = 0; t < a.n_refine; ++t) {
-            // z is indexed by the loop counter: select from the unrolled array
-            float ra = 0.0f, rb = 0.0f, rc = 0.0f;
-#pragma unroll
-            for (int u = 0; u < kMaxRefine; ++u)
-                if (u == t) { ra = z[3 * u]; rb = z[3 * u + 1]; rc = z[3 * u + 2]; }
-            const float dh = dcur * exp_(a.dr[t] * ra);
-            const float nx = fma_(a.nr[t], ra, c0);
-            const float ny = fma_(a.nr[t], rb, c1);
-            const float nz = fma_(a.nr[t], rc, c2);
-            float q0, q1, q2;
-            plane_from_depth_normal(bx, by, bz, dh, nx, ny, nz, q0, q1, q2);
-            const float sh_ = score_plane_t<NV, kZero>(a, tp, sWc, rs, i, j, q0, q1, q2, &sh.sv[0][tid], NT);
-            ++n_eval;
-            ++n_cand;
-            if (sh_ > sc) { c0 = q0; c1 = q1; c2 = q2; sc = sh_; dcur = dh; }
+    for (int n = 0; n < a.n_refine; ++n) {
+        // the normals of four trials at a time, in the pixel's own LDS column
+        if ((n & 3) == 0 && owner) {
+#pragma unroll 1
+            for (int b = 0; b < 3; ++b) {
+                float z0, z1, z2, z3;
+                refine_block(a, (uint32_t)(i * a.W + j), it, 3 * (n >> 2) + b, z0, z1, z2, z3);
+                float* zt = &sh.z[4 * b * NP + t];
+                zt[0] = z0; zt[NP] = z1; zt[2 * NP] = z2; zt[3 * NP] = z3;
+            }
         }
+        const float* zt = &sh.z[3 * (n & 3) * NP + t];
+        const float ra = zt[0], rb = zt[NP], rc = zt[2 * NP];
+        const float dh = dcur * exp_(a.dr[n] * ra);
+        const float nx = fma_(a.nr[n], ra, c0);
+        const float ny = fma_(a.nr[n], rb, c1);
+        const float nz = fma_(a.nr[n], rc, c2);
+        float q0, q1, q2;
+        tap_bearing(tp, i, j, bx, by, bz);
+        plane_from_depth_normal(bx, by, bz, dh, nx, ny, nz, q0, q1, q2);
+        if (owner) sh.trial[t] = make_float4(q0, q1, q2, dh);
+        wave_exchange();
+        auto job = [&](int l, int& jt, float& px, float& py, float& pz) {
+            jt = PW * wave + l;
+            const float4 pn = sh.trial[jt];
+            px = pn.x; py = pn.y; pz = pn.z;
+        };
+        auto put = [&](int l, float s) { sh.trial_score[PW * wave + l] = s; };
+        evaluate(job, put, alive);
+        n_eval += (unsigned int)__popcll(alive);
+        if (active && sh.trial_score[t] > sc) {
+            const float4 pn = sh.trial[t];
+            c0 = pn.x; c1 = pn.y; c2 = pn.z; dcur = pn.w;
+            sc = sh.trial_score[t];
+        }
+        wave_exchange();
+    }
+    tap_bearing(tp, i, j, bx, by, bz);
+    if (active) {
         store_map(&score[k], sc);
         store_map4(&plane[k], make_float4(c0, c1, c2, 0.0f));
         store_map(&depth[k], depth_of_plane(bx, by, bz, c0, c1, c2));
