@@ -337,7 +337,7 @@ class Context:
         H, W = img.shape[:2]
         C = 1 if img.ndim == 2 else img.shape[2]
         oH, oW = out_shape
-        out = np.zeros((oH, oW) if img.ndim == 2 else (oH, oW, C), np.uint8)
+        out = np.empty((oH, oW) if img.ndim == 2 else (oH, oW, C), np.uint8)
         self._chk(self.L.pmp_resize(self.h, _p(img, _u8p), W, H, W * C, C, _p(out, _u8p), oW, oH, 0), "pmp_resize")
         return out
 
@@ -352,7 +352,7 @@ class Context:
         hw = self.image_size(image_id)
         if shape is not None and tuple(shape) != hw:
             raise ValueError(f"image {image_id} is {hw[0]}x{hw[1]} (H x W), not {tuple(shape)}")
-        out = np.zeros(hw, np.uint8)
+        out = np.empty(hw, np.uint8)
         self._chk(self.L.pmp_image_get(self.h, image_id, _p(out, _u8p)), "pmp_image_get")
         return out
 
@@ -449,17 +449,17 @@ class Context:
 
     def get_maps(self, which=PMP_MAPS_WORK):
         H, W = self.H, self.W
-        plane = np.zeros((H, W, 4), np.float32)
-        depth = np.zeros((H, W), np.float32)
-        score = np.zeros((H, W), np.float32)
-        nghbr = np.zeros((H, W), np.int32) if which == PMP_MAPS_FINAL else None
+        plane = np.empty((H, W, 4), np.float32)
+        depth = np.empty((H, W), np.float32)
+        score = np.empty((H, W), np.float32)
+        nghbr = np.empty((H, W), np.int32) if which == PMP_MAPS_FINAL else None
         self._chk(self.L.pmp_get_maps(self.h, which, _p(plane, _f32p), _p(depth, _f32p), _p(score, _f32p),
                                       _p(nghbr, _i32p)), "pmp_get_maps")
         return (plane, depth, score, nghbr) if which == PMP_MAPS_FINAL else (plane, depth, score)
 
     def get_normals(self, which=PMP_MAPS_FINAL):
         """Unit camera-facing normals -p/|p| of a map set, (H, W, 3)."""
-        out = np.zeros((self.H, self.W, 3), np.float32)
+        out = np.empty((self.H, self.W, 3), np.float32)
         self._chk(self.L.pmp_get_normals(self.h, which, _p(out, _f32p)), "pmp_get_normals")
         return out
 
@@ -475,10 +475,10 @@ class Context:
 
     def batch_get_maps(self, k: int, shape):
         H, W = shape
-        plane = np.zeros((H, W, 4), np.float32)
-        depth = np.zeros((H, W), np.float32)
-        score = np.zeros((H, W), np.float32)
-        nghbr = np.zeros((H, W), np.int32)
+        plane = np.empty((H, W, 4), np.float32)
+        depth = np.empty((H, W), np.float32)
+        score = np.empty((H, W), np.float32)
+        nghbr = np.empty((H, W), np.int32)
         self._chk(self.L.pmp_batch_get_maps(self.h, k, _p(plane, _f32p), _p(depth, _f32p), _p(score, _f32p),
                                             _p(nghbr, _i32p)), "pmp_batch_get_maps")
         return plane, depth, score, nghbr
@@ -505,7 +505,7 @@ class Context:
         H, W = depths[0].shape
         arr = (_f32p * len(depths))(*[_p(d, _f32p) for d in depths])
         ps = (Pose * len(depths))(*[Pose.from12(p) for p in poses])
-        out = np.zeros((H, W), np.float32)
+        out = np.empty((H, W), np.float32)
         self._chk(self.L.pmp_clean(self.h, W, H, len(depths), arr, ps, thr, min_consistent, _p(out, _f32p)),
                   "pmp_clean")
         return out
@@ -516,7 +516,7 @@ class Context:
         H, W = depths[0].shape
         arr = (_f32p * len(depths))(*[_p(d, _f32p) for d in depths])
         ps = (Pose * len(depths))(*[Pose.from12(p) for p in poses])
-        out = np.zeros((H, W), np.float32)
+        out = np.empty((H, W), np.float32)
         self._chk(self.L.pmp_clean_noalloc(self.h, W, H, len(depths), arr, ps, thr, min_consistent, _p(out, _f32p)),
                   "pmp_clean_noalloc")
         return out
@@ -532,7 +532,7 @@ class Context:
             planes = [np.ascontiguousarray(q, dtype=np.float32).reshape(H, W, 4) for q in planes]
             parr = (_f32p * len(planes))(*[_p(q, _f32p) for q in planes])
         ps = (Pose * len(depths))(*[Pose.from12(p) for p in poses])
-        out = np.zeros((H, W), np.float32)
+        out = np.empty((H, W), np.float32)
         self._chk(self.L.pmp_clean_ex(self.h, W, H, len(depths), arr, parr, ps, thr, min_consistent,
                                       float(max_reproj_px), float(max_normal_deg), _p(out, _f32p)), "pmp_clean_ex")
         return out
@@ -567,7 +567,7 @@ class Context:
         return self.L.pmp_pruner_size(self.h)
 
     def pruner_get_map(self, index, shape):
-        out = np.zeros(shape, np.float32)
+        out = np.empty(shape, np.float32)
         self._chk(self.L.pmp_pruner_get_map(self.h, index, _p(out, _f32p)), "pmp_pruner_get_map")
         return out
 
@@ -696,10 +696,10 @@ class Server:
     def fetch(self, ticket: int):
         """(plane, depth, score, nghbr, info) of a finished request; forgets the ticket."""
         H, W = self.shapes.pop(ticket)
-        plane = np.zeros((H, W, 4), np.float32)
-        depth = np.zeros((H, W), np.float32)
-        score = np.zeros((H, W), np.float32)
-        nghbr = np.zeros((H, W), np.int32)
+        plane = np.empty((H, W, 4), np.float32)
+        depth = np.empty((H, W), np.float32)
+        score = np.empty((H, W), np.float32)
+        nghbr = np.empty((H, W), np.int32)
         info = RequestInfo()
         self._chk(self.L.pmp_server_fetch(self.h, ticket, _p(plane, _f32p), _p(depth, _f32p), _p(score, _f32p),
                                           _p(nghbr, _i32p), ctypes.byref(info)), "pmp_server_fetch")

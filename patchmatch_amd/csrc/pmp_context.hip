@@ -17,23 +17,18 @@ int set_error(pmp_ctx* ctx, int code, const std::string& msg) {
 
 int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch,
                      hipStream_t s) {
-    const size_t bytes = row * rows;
-    if (bytes == 0) return PMP_OK;
-    if (bytes > ctx->stage_cap) {
-        if (ctx->stage) (void)hipHostFree(ctx->stage);
-        ctx->stage = nullptr;
-        ctx->stage_cap = 0;
-        PMP_HIP(ctx, hipHostMalloc((void**)&ctx->stage, bytes, hipHostMallocDefault));
-        ctx->stage_cap = bytes;
-    }
-    if (pitch == row) {
-        memcpy(ctx->stage, src, bytes);
-    } else {
-        for (size_t r = 0; r < rows; ++r) memcpy(ctx->stage + r * row, src + r * pitch, row);
-    }
-    PMP_HIP(ctx, hipMemcpyAsync(dst, ctx->stage, bytes, hipMemcpyHostToDevice, s));
-    // the staging buffer is reused by the next upload
-    PMP_HIP(ctx, hipStreamSynchronize(s));
+    const HostCopy c{const_cast<uint8_t*>(src), dst, row, rows, pitch};
+    PMP_HIP(ctx, ctx->copier.to_device(s, &c, 1));
+    return PMP_OK;
+}
+
+int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n) {
+    PMP_HIP(ctx, ctx->copier.to_host(ctx->stream, c, n));
+    return PMP_OK;
+}
+
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n) {
+    PMP_HIP(ctx, ctx->copier.to_device(ctx->stream, c, n));
     return PMP_OK;
 }
 
@@ -285,7 +280,6 @@ void pmp_destroy(pmp_ctx* ctx) {
                     ctx->epochs};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (ctx->stage) (void)hipHostFree(ctx->stage);
     if (ctx->mask_pin) (void)hipHostFree(ctx->mask_pin);
     if (ctx->mask_copied) (void)hipEventDestroy(ctx->mask_copied);
     for (auto& kv : ctx->rowtabs) (void)hipFree(kv.second);
@@ -409,9 +403,8 @@ int pmp_image_get(pmp_ctx* ctx, uint64_t id, uint8_t* pixels) {
     PMP_ON_DEVICE(ctx);
     auto it = ctx->images.find(id);
     if (it == ctx->images.end()) return set_error(ctx, PMP_ENOTFOUND, "unknown image id");
-    PMP_HIP(ctx, hipMemcpyAsync(pixels, it->second.gray, it->second.bytes, hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    const HostCopy c = flat_copy(pixels, it->second.gray, it->second.bytes);
+    return copy_to_host(ctx, &c, 1);
 }
 
 int pmp_image_drop(pmp_ctx* ctx, uint64_t id) {

@@ -338,9 +338,13 @@ int pmp_set_maps(pmp_ctx* ctx, const float* plane4, const float* depth, const fl
     PMP_ON_DEVICE(ctx);
     if (!ctx->views_set) return set_error(ctx, PMP_ESTATE, "pmp_set_views has not been called");
     const size_t P = (size_t)ctx->W * ctx->H;
-    if (plane4) PMP_HIP(ctx, hipMemcpyAsync(ctx->ws.plane, plane4, P * 16, hipMemcpyHostToDevice, ctx->stream));
-    if (depth) PMP_HIP(ctx, hipMemcpyAsync(ctx->ws.depth, depth, P * 4, hipMemcpyHostToDevice, ctx->stream));
-    if (score) PMP_HIP(ctx, hipMemcpyAsync(ctx->ws.score, score, P * 4, hipMemcpyHostToDevice, ctx->stream));
+    HostCopy c[3];
+    int n = 0;
+    if (plane4) c[n++] = flat_copy(plane4, ctx->ws.plane, P * 16);
+    if (depth) c[n++] = flat_copy(depth, ctx->ws.depth, P * 4);
+    if (score) c[n++] = flat_copy(score, ctx->ws.score, P * 4);
+    int rc = copy_to_device(ctx, c, n);
+    if (rc) return rc;
     PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return PMP_OK;
 }
@@ -355,15 +359,14 @@ int pmp_get_maps(pmp_ctx* ctx, int32_t which, float* plane4, float* depth, float
     else if (which == PMP_MAPS_INIT) { sp = ctx->ws.iplane; sd = ctx->ws.idepth; ss = ctx->ws.iscore; }
     else if (which == PMP_MAPS_FINAL) { sp = ctx->ws.oplane; sd = ctx->ws.odepth; ss = ctx->ws.oscore; }
     else return set_error(ctx, PMP_EINVAL, "unknown map set");
-    if (plane4) PMP_HIP(ctx, hipMemcpyAsync(plane4, sp, P * 16, hipMemcpyDeviceToHost, ctx->stream));
-    if (depth) PMP_HIP(ctx, hipMemcpyAsync(depth, sd, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (score) PMP_HIP(ctx, hipMemcpyAsync(score, ss, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (nghbr) {
-        if (which != PMP_MAPS_FINAL) return set_error(ctx, PMP_EINVAL, "nghbr exists only for the final maps");
-        PMP_HIP(ctx, hipMemcpyAsync(nghbr, ctx->ws.onghbr, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    }
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    if (nghbr && which != PMP_MAPS_FINAL) return set_error(ctx, PMP_EINVAL, "nghbr exists only for the final maps");
+    HostCopy c[4];
+    int n = 0;
+    if (plane4) c[n++] = flat_copy(plane4, sp, P * 16);
+    if (depth) c[n++] = flat_copy(depth, sd, P * 4);
+    if (score) c[n++] = flat_copy(score, ss, P * 4);
+    if (nghbr) c[n++] = flat_copy(nghbr, ctx->ws.onghbr, P * 4);
+    return copy_to_host(ctx, c, n);
 }
 
 int pmp_get_normals(pmp_ctx* ctx, int32_t which, float* normal3) {
@@ -385,9 +388,8 @@ int pmp_get_normals(pmp_ctx* ctx, int32_t which, float* normal3) {
     }
     hipLaunchKernelGGL(k_normals, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, ctx->stream, sp, ctx->normals, (int)P);
     PMP_HIP(ctx, hipGetLastError());
-    PMP_HIP(ctx, hipMemcpyAsync(normal3, ctx->normals, 3 * P * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    const HostCopy c = flat_copy(normal3, ctx->normals, 3 * P * sizeof(float));
+    return copy_to_host(ctx, &c, 1);
 }
 
 int pmp_eval_counts(pmp_ctx* ctx, int64_t* evals, int64_t* candidates) {

@@ -358,10 +358,11 @@ static int clean_impl(pmp_ctx* ctx, int32_t width, int32_t height, int32_t n_map
         PMP_HIP(ctx, hipMalloc(&ctx->clean_maps, need * sizeof(float)));
         ctx->clean_cap = need;
     }
+    HostCopy up[2 * kMaxMaps];
+    int n_up = 0;
     for (int o = 0; o < n_maps; ++o) {
         if (!depth_maps[o]) return set_error(ctx, PMP_EINVAL, "null depth map");
-        PMP_HIP(ctx, hipMemcpyAsync(ctx->clean_maps + o * P, depth_maps[o], P * sizeof(float), hipMemcpyHostToDevice,
-                                    ctx->stream));
+        up[n_up++] = flat_copy(depth_maps[o], ctx->clean_maps + o * P, P * sizeof(float));
     }
     float* dout = ctx->clean_maps + n_maps * P;
     CleanChecks c;
@@ -374,19 +375,18 @@ static int clean_impl(pmp_ctx* ctx, int32_t width, int32_t height, int32_t n_map
         float* planes = ctx->clean_maps + poff;
         for (int o = 0; o < n_maps; ++o) {
             if (!plane4_maps[o]) return set_error(ctx, PMP_EINVAL, "null plane map");
-            PMP_HIP(ctx, hipMemcpyAsync(planes + 4 * o * P, plane4_maps[o], 4 * P * sizeof(float),
-                                        hipMemcpyHostToDevice, ctx->stream));
+            up[n_up++] = flat_copy(plane4_maps[o], planes + 4 * o * P, 4 * P * sizeof(float));
         }
         c.planes = planes;
         const double cs = cos((double)max_normal_deg * (M_PI / 180.0));
         c.cos2 = cs * cs;
     }
+    if ((rc = copy_to_device(ctx, up, n_up))) return rc;
     dim3 blk(256), grd((width + 255) / 256, height);
     hipLaunchKernelGGL(k_clean, grd, blk, 0, ctx->stream, a, c, ctx->clean_maps, min_consistent, dout);
     PMP_HIP(ctx, hipGetLastError());
-    PMP_HIP(ctx, hipMemcpyAsync(cleaned, dout, P * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    const HostCopy down = flat_copy(cleaned, dout, P * sizeof(float));
+    return copy_to_host(ctx, &down, 1);
 }
 
 int pmp_clean(pmp_ctx* ctx, int32_t width, int32_t height, int32_t n_maps, const float* const* depth_maps,
@@ -477,9 +477,13 @@ int pmp_pruner_add_view(pmp_ctx* ctx, const float* cleaned_depth, const pmp_pose
     }
     memcpy(v.pose, pose->R, 9 * sizeof(double));
     memcpy(v.pose + 9, pose->t, 3 * sizeof(double));
-    PMP_HIP(ctx, hipMemcpyAsync(v.depth, cleaned_depth, P * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    PMP_HIP(ctx, hipMemcpyAsync(v.bgr, bgr, 3 * P, hipMemcpyHostToDevice, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    const HostCopy up[2] = {flat_copy(cleaned_depth, v.depth, P * sizeof(float)), flat_copy(bgr, v.bgr, 3 * P)};
+    const int rc = copy_to_device(ctx, up, 2);
+    if (rc) {
+        (void)hipFree(v.depth);
+        (void)hipFree(v.bgr);
+        return rc;
+    }
     ctx->pruner.push_back(v);
     return PMP_OK;
 }
@@ -554,14 +558,15 @@ int pmp_pruner_prune(pmp_ctx* ctx, float same_depth_thr, float* pruned_depth, in
                        ctx->prune_alive, ctx->prune_blk, ctx->prune_pts, ctx->prune_cols, ctx->prune_kps);
     PMP_HIP(ctx, hipGetLastError());
     const int64_t nc = total < cap ? total : cap;
+    HostCopy down[4];
+    int n_down = 0;
     if (nc > 0) {
-        PMP_HIP(ctx, hipMemcpyAsync(pts, ctx->prune_pts, nc * 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        PMP_HIP(ctx, hipMemcpyAsync(cols, ctx->prune_cols, nc * 3, hipMemcpyDeviceToHost, ctx->stream));
-        PMP_HIP(ctx, hipMemcpyAsync(kps, ctx->prune_kps, nc * 2 * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+        down[n_down++] = flat_copy(pts, ctx->prune_pts, nc * 3 * sizeof(double));
+        down[n_down++] = flat_copy(cols, ctx->prune_cols, nc * 3);
+        down[n_down++] = flat_copy(kps, ctx->prune_kps, nc * 2 * sizeof(int32_t));
     }
-    if (pruned_depth)
-        PMP_HIP(ctx, hipMemcpyAsync(pruned_depth, ctx->prune_out, P * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (pruned_depth) down[n_down++] = flat_copy(pruned_depth, ctx->prune_out, P * sizeof(float));
+    if ((rc = copy_to_host(ctx, down, n_down))) return rc;
     if (count) *count = total;
     return PMP_OK;
 }
@@ -596,9 +601,8 @@ int pmp_pruner_get_map(pmp_ctx* ctx, int32_t index, float* depth) {
     PMP_ON_DEVICE(ctx);
     if (index < 0 || index >= (int)ctx->pruner.size()) return set_error(ctx, PMP_EINVAL, "pruner index out of range");
     const PrunerView& v = ctx->pruner[index];
-    PMP_HIP(ctx, hipMemcpyAsync(depth, v.depth, (size_t)v.W * v.H * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    const HostCopy c = flat_copy(depth, v.depth, (size_t)v.W * v.H * sizeof(float));
+    return copy_to_host(ctx, &c, 1);
 }
 
 }  // extern "C"

@@ -9,6 +9,8 @@
 
 #include "pmp/pmp.h"
 
+#include "pmp_copy.h"
+
 namespace pmp {
 
 constexpr int kMaxViews = PMP_MAX_VIEWS;
@@ -173,9 +175,7 @@ struct pmp_ctx {
     std::vector<int> epoch_tiles;
     size_t epoch_words = 0;
 
-    // pinned staging of host uploads (upload_host_rows)
-    uint8_t* stage = nullptr;
-    size_t stage_cap = 0;
+    pmp::Copier copier;                 // copies from and to the callers' memory
 };
 
 namespace pmp {
@@ -191,6 +191,11 @@ int check_hip(pmp_ctx* ctx, hipError_t e, const char* what);
 // memory at dst on stream s, and waits for the copy.  The rows are packed into
 // a pinned staging buffer of the context (grown on demand) and sent in one
 // copy: a 2D copy from pageable memory moves row by row, about 9 us a row.
+// The caller's memory from and to the device (Copier); from the device after
+// the work queued on s, complete on return; to the device in stream order, the
+// host memory read on return.
+int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n);
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n);
 int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch,
                      hipStream_t s);
 int ensure_workspace(pmp_ctx* ctx, int W, int H);

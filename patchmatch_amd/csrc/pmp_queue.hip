@@ -875,12 +875,13 @@ int pmp_batch_get_maps(pmp_ctx* ctx, int32_t k, float* plane4, float* depth, flo
     if (!q || k < 0 || k >= q->n_last) return set_error(ctx, PMP_EINVAL, "no such keyframe in the last batch");
     const SlotBuf& b = q->bufs[k];
     const size_t P = (size_t)b.W * b.H;
-    if (plane4) PMP_HIP(ctx, hipMemcpyAsync(plane4, b.oplane, P * 16, hipMemcpyDeviceToHost, ctx->stream));
-    if (depth) PMP_HIP(ctx, hipMemcpyAsync(depth, b.odepth, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (score) PMP_HIP(ctx, hipMemcpyAsync(score, b.oscore, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    if (nghbr) PMP_HIP(ctx, hipMemcpyAsync(nghbr, b.onghbr, P * 4, hipMemcpyDeviceToHost, ctx->stream));
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    HostCopy c[4];
+    int n = 0;
+    if (plane4) c[n++] = flat_copy(plane4, b.oplane, P * 16);
+    if (depth) c[n++] = flat_copy(depth, b.odepth, P * 4);
+    if (score) c[n++] = flat_copy(score, b.oscore, P * 4);
+    if (nghbr) c[n++] = flat_copy(nghbr, b.onghbr, P * 4);
+    return copy_to_host(ctx, c, n);
 }
 
 int pmp_batch_set_config(pmp_ctx* ctx, const pmp_batch_config* cfg) {

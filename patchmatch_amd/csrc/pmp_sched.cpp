@@ -425,8 +425,8 @@ int Server::submit(const pmp_request& req, const pmp_params& p, uint64_t* ticket
             err = "pinned host buffer of the previous result";
             rc = PMP_ENOMEM;
         } else {
-            memcpy(r->prev.p, req.prev_plane4, 16 * P);
-            memcpy(r->prev.p + 16 * P, req.prev_depth, 4 * P);
+            ex_->host_copy(r->prev.p, req.prev_plane4, 16 * P);
+            ex_->host_copy(r->prev.p + 16 * P, req.prev_depth, 4 * P);
             r->job.prev_plane4 = (const float*)r->prev.p;
             r->job.prev_depth = (const float*)(r->prev.p + 16 * P);
             memcpy(r->job.prev_pose, req.prev_pose->R, 9 * sizeof(double));
@@ -506,10 +506,10 @@ int Server::fetch(uint64_t ticket, float* plane4, float* depth, float* score, in
     } else {
         const size_t P = (size_t)r->job.W * r->job.H;
         const uint8_t* o = r->out.p;
-        if (plane4) memcpy(plane4, o, P * 16);
-        if (depth) memcpy(depth, o + P * 16, P * 4);
-        if (score) memcpy(score, o + P * 20, P * 4);
-        if (nghbr) memcpy(nghbr, o + P * 24, P * 4);
+        if (plane4) ex_->host_copy(plane4, o, P * 16);
+        if (depth) ex_->host_copy(depth, o + P * 16, P * 4);
+        if (score) ex_->host_copy(score, o + P * 20, P * 4);
+        if (nghbr) ex_->host_copy(nghbr, o + P * 24, P * 4);
     }
     give_host(r->out);
     give_host(r->lm);

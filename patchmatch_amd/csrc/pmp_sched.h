@@ -26,6 +26,7 @@
 // drives the scheduler in the CPU sanitizer tests).
 #pragma once
 #include <stdint.h>
+#include <string.h>
 
 #include <chrono>
 #include <condition_variable>
@@ -88,6 +89,8 @@ class Executor {
     // Pinned host buffers (nullptr on failure).
     virtual uint8_t* host_alloc(size_t bytes) = 0;
     virtual void host_free(uint8_t* p) = 0;
+    // Host to host, from and to the callers' memory.
+    virtual void host_copy(void* dst, const void* src, size_t bytes) { memcpy(dst, src, bytes); }
     // Issues one step into descriptor set w (0 or 1), asynchronously.
     // item_rc[k] != 0 leaves item k out (its request fails with that status
     // and item_err[k]); a non-zero return means the step could not be issued

@@ -39,12 +39,6 @@ class GpuExec final : public sched::Executor {
     // The scheduler thread keeps the context's device current; calls on the
     // caller's threads (submit, reset) hold a DeviceScope.
     std::mutex pool_mu;
-    // pinned staging of uploads (one copy from pinned memory instead of a
-    // pageable one), shared by the submitting threads
-    std::mutex stage_mu;
-    uint8_t* stage = nullptr;
-    size_t stage_cap = 0;
-
     int init(const pmp_server_opts& o) {
         cfg = o.config;
         edge_mode = o.edge_mode;
@@ -76,7 +70,6 @@ class GpuExec final : public sched::Executor {
         for (hipEvent_t e : step_done)
             if (e) (void)hipEventDestroy(e);
         if (copy) (void)hipStreamDestroy(copy);
-        if (stage) (void)hipHostFree(stage);
         pmp_destroy(ctx);   // frees the pooled images
     }
 
@@ -106,21 +99,10 @@ class GpuExec final : public sched::Executor {
         im.bytes = (size_t)W * H;
         hipError_t e = hipMalloc(&im.gray, im.bytes);
         if (e == hipSuccess) {
-            std::lock_guard<std::mutex> lk(stage_mu);
-            if (im.bytes > stage_cap) {
-                if (stage) (void)hipHostFree(stage);
-                stage = nullptr;
-                stage_cap = 0;
-                e = hipHostMalloc((void**)&stage, im.bytes, hipHostMallocDefault);
-                if (e == hipSuccess) stage_cap = im.bytes;
-            }
-            if (e == hipSuccess) {
-                memcpy(stage, pixels, im.bytes);
-                e = hipMemcpyAsync(im.gray, stage, im.bytes, hipMemcpyHostToDevice, copy);
-            }
-            // the staging buffer is reused by the next upload
-            if (e == hipSuccess) e = hipStreamSynchronize(copy);
+            const HostCopy c = flat_copy(pixels, im.gray, im.bytes);
+            e = ctx->copier.to_device(copy, &c, 1);
         }
+        if (e == hipSuccess) e = hipStreamSynchronize(copy);
         if (e != hipSuccess) {
             if (im.gray) (void)hipFree(im.gray);
             err = "upload of image " + std::to_string(id) + ": " + hipGetErrorString(e);
@@ -169,6 +151,7 @@ class GpuExec final : public sched::Executor {
         return p;
     }
     void host_free(uint8_t* p) override { (void)hipHostFree(p); }
+    void host_copy(void* dst, const void* src, size_t bytes) override { ctx->copier.copy(dst, src, bytes); }
 
     int step_issue(int w, const std::vector<sched::StepItem>& items, std::vector<int>& item_rc,
                    std::vector<std::string>& item_err, std::string& err) override {

@@ -153,8 +153,8 @@ int pmp_resize(pmp_ctx* ctx, const uint8_t* src, int32_t width, int32_t height, 
                             (int64_t)out_width * channels)))
         return rc;
     if (!on_device) {
-        PMP_HIP(ctx, hipMemcpyAsync(dst, ddst, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
-        PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        const HostCopy c = flat_copy(dst, ddst, out_bytes);
+        if ((rc = copy_to_host(ctx, &c, 1))) return rc;
     }
     return PMP_OK;
 }
