@@ -22,13 +22,13 @@ int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, si
     return PMP_OK;
 }
 
-int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n) {
-    PMP_HIP(ctx, ctx->copier.to_host(ctx->stream, c, n));
+int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n, bool fresh) {
+    PMP_HIP(ctx, ctx->copier.to_host(ctx->stream, c, n, fresh));
     return PMP_OK;
 }
 
-int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n) {
-    PMP_HIP(ctx, ctx->copier.to_device(ctx->stream, c, n));
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, bool waits) {
+    PMP_HIP(ctx, ctx->copier.to_device(ctx->stream, c, n, waits));
     return PMP_OK;
 }
 

@@ -40,10 +40,12 @@ inline HostCopy flat_copy(const void* host, const void* dev, size_t bytes) {
 class Copier {
 public:
     ~Copier();
-    // Device to host after the work queued on s; complete on return.
-    hipError_t to_host(hipStream_t s, const HostCopy* c, int n);
-    // Host to device in stream order; on return the host memory has been read.
-    hipError_t to_device(hipStream_t s, const HostCopy* c, int n);
+    // Device to host after the work queued on s; complete on return.  fresh:
+    // to memory that has hardly been touched since it was allocated.
+    hipError_t to_host(hipStream_t s, const HostCopy* c, int n, bool fresh = false);
+    // Host to device in stream order; on return the host memory has been read,
+    // unless the caller waits for the stream itself before it returns (waits).
+    hipError_t to_device(hipStream_t s, const HostCopy* c, int n, bool waits = false);
     // Host to host.
     void copy(void* dst, const void* src, size_t bytes);
 
@@ -56,9 +58,19 @@ private:
     static constexpr int kSlots = 2;
     static constexpr int kTasks = 256;       // a power of two above kSlots * kChunk / kPiece
     static constexpr int kThreads = 8;
-    // Transfers below this are copied by the caller alone, in one chunk: waking
-    // the threads costs more.
-    static constexpr size_t kAlone = size_t(768) << 10;
+    // Transfers below these are copied by the caller alone, in one chunk: waking
+    // the threads costs more (normals of 328x182, 716 KB down: 66 us alone, 52
+    // with them; a 614 KB image up: 75 and 76).
+    static constexpr size_t kAloneDown = size_t(512) << 10, kAloneUp = size_t(768) << 10;
+    // Uploads from kAloneUp to this are the runtime's own: it pins the pages and
+    // copies from them (five 640x320 maps to the cleaner and back: 222 us, with
+    // the threads 292; of 800x400: 363 and 353; of 1363x677: 863 and 638).
+    static constexpr size_t kPinned = size_t(6) << 20;
+    // So are downloads to fresh memory below this: pinning takes the page
+    // faults at once, which the threads would fight over (the pruner's points
+    // and map: of 320x160 views 189 us, with the threads 225; of 640x320 366
+    // and 375; of 1098x494 885 and 785).
+    static constexpr size_t kFresh = size_t(12) << 20;
     struct Span {               // bytes [off, off + len) of c, contiguous at lin
         HostCopy c;
         size_t off, len;

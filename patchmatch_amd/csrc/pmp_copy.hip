@@ -141,9 +141,12 @@ struct Copier::Walk {
     const HostCopy* c;
     int n, k = 0;
     size_t off = 0;
-    bool next(Span& p) {
+    bool end() {
         while (k < n && off >= c[k].row * c[k].rows) { ++k; off = 0; }
-        if (k == n) return false;
+        return k == n;
+    }
+    bool next(Span& p) {
+        if (end()) return false;
         p.c = c[k];
         p.off = off;
         p.len = std::min(kChunk, c[k].row * c[k].rows - off);
@@ -173,7 +176,7 @@ static size_t total(const HostCopy* c, int n) {
     return b;
 }
 
-static hipError_t plain(hipStream_t s, const HostCopy* c, int n, hipMemcpyKind kind) {
+static hipError_t plain(hipStream_t s, const HostCopy* c, int n, hipMemcpyKind kind, bool wait) {
     const bool in = kind == hipMemcpyHostToDevice;
     for (int k = 0; k < n; ++k) {
         if (c[k].row * c[k].rows == 0) continue;
@@ -184,7 +187,7 @@ static hipError_t plain(hipStream_t s, const HostCopy* c, int n, hipMemcpyKind k
                                    in ? c[k].pitch : c[k].row, c[k].row, c[k].rows, kind, s);
         if (e != hipSuccess) return e;
     }
-    return hipStreamSynchronize(s);
+    return wait ? hipStreamSynchronize(s) : hipSuccess;
 }
 
 hipError_t Copier::small(hipStream_t s, const HostCopy* c, int n, bool out) {
@@ -213,10 +216,12 @@ hipError_t Copier::small(hipStream_t s, const HostCopy* c, int n, bool out) {
 
 // Chunk k (of this transfer) uses slot k % kSlots; the slots' earlier pieces
 // are done (every transfer ends so), their DMAs perhaps not.
-hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n) {
+hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n, bool fresh) {
     std::lock_guard<std::mutex> lk(mu_);
-    if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyDeviceToHost);
-    if (total(c, n) < kAlone) return small(s, c, n, true);
+    const size_t bytes = total(c, n);
+    if (!pageable(c, n) || !start_ring() || (fresh && bytes < kFresh))
+        return plain(s, c, n, hipMemcpyDeviceToHost, true);
+    if (bytes < kAloneDown) return small(s, c, n, true);
     const bool alone = !start_threads();
     Walk w{c, n};
     bool more = true;
@@ -225,19 +230,21 @@ hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n) {
     for (;;) {
         while (more && issued < copied + kSlots) {
             Slot& sl = slot_[issued % kSlots];
-            if ((e = dma_done(sl)) != hipSuccess || !(more = w.next(sl.p))) break;
+            if ((e = dma_done(sl)) != hipSuccess || !w.next(sl.p)) break;
             sl.p.lin = pin_ + (issued % kSlots) * kChunk;
             sl.p.out = true;
             wait(sl.begin, sl.end);
             e = hipMemcpyAsync(sl.p.lin, (const uint8_t*)sl.p.c.dev + sl.p.off, sl.p.len, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipEventRecord(sl.ev, s);
             if (e != hipSuccess) break;
-            sl.dma = true;
             ++issued;
+            // the last chunk is waited for by the stream itself, without an
+            // event, after which the caller's next wait for it would cost 30 us
+            if ((more = !w.end()) && (e = hipEventRecord(sl.ev, s)) != hipSuccess) break;
+            sl.dma = more;
         }
         if (e != hipSuccess || copied == issued) break;
         Slot& sl = slot_[copied % kSlots];
-        if ((e = dma_done(sl)) != hipSuccess) break;
+        if ((e = sl.dma ? dma_done(sl) : hipStreamSynchronize(s)) != hipSuccess) break;
         sl.begin = next_;
         push(sl.p, alone);
         sl.end = next_;
@@ -248,10 +255,12 @@ hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n) {
     return e;
 }
 
-hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n) {
+hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, bool waits) {
     std::lock_guard<std::mutex> lk(mu_);
-    if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyHostToDevice);
-    if (total(c, n) < kAlone) return small(s, c, n, false);
+    if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
+    const size_t bytes = total(c, n);
+    if (bytes < kAloneUp) return small(s, c, n, false);
+    if (bytes < kPinned) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
     const bool alone = !start_threads();
     Walk w{c, n};
     bool more = true;
@@ -282,7 +291,7 @@ hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n) {
 
 void Copier::copy(void* dst, const void* src, size_t bytes) {
     std::unique_lock<std::mutex> lk(mu_, std::try_to_lock);
-    if (bytes < kAlone || !lk.owns_lock() || !start_threads()) {
+    if (bytes < kAloneUp || !lk.owns_lock() || !start_threads()) {
         memcpy(dst, src, bytes);
         return;
     }

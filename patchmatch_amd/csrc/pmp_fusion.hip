@@ -381,7 +381,7 @@ static int clean_impl(pmp_ctx* ctx, int32_t width, int32_t height, int32_t n_map
         const double cs = cos((double)max_normal_deg * (M_PI / 180.0));
         c.cos2 = cs * cs;
     }
-    if ((rc = copy_to_device(ctx, up, n_up))) return rc;
+    if ((rc = copy_to_device(ctx, up, n_up, true))) return rc;
     dim3 blk(256), grd((width + 255) / 256, height);
     hipLaunchKernelGGL(k_clean, grd, blk, 0, ctx->stream, a, c, ctx->clean_maps, min_consistent, dout);
     PMP_HIP(ctx, hipGetLastError());
@@ -566,7 +566,7 @@ int pmp_pruner_prune(pmp_ctx* ctx, float same_depth_thr, float* pruned_depth, in
         down[n_down++] = flat_copy(kps, ctx->prune_kps, nc * 2 * sizeof(int32_t));
     }
     if (pruned_depth) down[n_down++] = flat_copy(pruned_depth, ctx->prune_out, P * sizeof(float));
-    if ((rc = copy_to_host(ctx, down, n_down))) return rc;
+    if ((rc = copy_to_host(ctx, down, n_down, true))) return rc;
     if (count) *count = total;
     return PMP_OK;
 }

@@ -193,9 +193,9 @@ int check_hip(pmp_ctx* ctx, hipError_t e, const char* what);
 // copy: a 2D copy from pageable memory moves row by row, about 9 us a row.
 // The caller's memory from and to the device (Copier); from the device after
 // the work queued on s, complete on return; to the device in stream order, the
-// host memory read on return.
-int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n);
-int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n);
+// host memory read on return unless the caller waits for the stream (waits).
+int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n, bool fresh = false);
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, bool waits = false);
 int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch,
                      hipStream_t s);
 int ensure_workspace(pmp_ctx* ctx, int W, int H);
