@@ -141,7 +141,7 @@ int plain_prepare(pmp_ctx* ctx, const pmp_params* p, const uint8_t* dmask, bool 
             return set_error(ctx, PMP_ENOTFOUND, "mask image was dropped");
         return rc;
     }
-    prop_shape(*q, q->cfg, 1, nullptr, q->plain.h_slots, r);
+    prop_shape(*q, q->cfg, 1, nullptr, q->plain.h_slots, false, r);
     const int tiles = slot_tiles(q->plain.h_slots[0], r.rows);
     fill_list(q->plain.h_hdr->init, 1, &items[0]);
     fill_list(q->plain.h_hdr->prop, 1, &tiles);
@@ -343,7 +343,7 @@ int pmp_set_maps(pmp_ctx* ctx, const float* plane4, const float* depth, const fl
     if (plane4) c[n++] = flat_copy(plane4, ctx->ws.plane, P * 16);
     if (depth) c[n++] = flat_copy(depth, ctx->ws.depth, P * 4);
     if (score) c[n++] = flat_copy(score, ctx->ws.score, P * 4);
-    int rc = copy_to_device(ctx, c, n);
+    int rc = copy_to_device(ctx, c, n, true);
     if (rc) return rc;
     PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return PMP_OK;

@@ -136,9 +136,10 @@ int slot_fill(pmp_ctx* ctx, const pmp_params* p, const pmp_keyframe& kf, const S
 // Partitions the slot into propagation tiles of `rows` tile rows; their number.
 int slot_tiles(SlotDesc& d, int rows);
 // Evaluation form and tile rows (r.form, r.rows) of a propagation over n filled
-// slots (slots[slot[k]]; slot null: 0..n-1).
+// slots (slots[slot[k]]; slot null: 0..n-1).  single: a pass is a launch of its
+// own (the server's steps).
 void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
-                QueueRun& r);
+                bool single, QueueRun& r);
 void fill_list(WorkList& L, int n, const int* items);
 // The rest of a shaped run; tiles: propagation tiles of a pass.
 int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,

@@ -554,7 +554,7 @@ static bool is_default(const pmp_batch_config& c) {
 }
 
 void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
-                QueueRun& r) {
+                bool single, QueueRun& r) {
     // work: the pixels of one colour in units of 64; chip: waves at four to a SIMD
     double work = 0.0;
     int views = 0;
@@ -585,9 +585,11 @@ void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int
         r.form = kLane;
     else
         r.form = work < 1.75 * chip ? kWide : kQuad;
-    // kQuad, 1920x960: 21.4 ms with 8 rows, 22.4 with 4, 23.2 with 2; kWide,
-    // 640x320, 4 views: 3.4 with 2, 3.5 with 4; kLane: pmp_queue.h
-    r.rows = !is_default(c) ? c.tile_rows : r.form == kLane ? 4 : r.form == kWide ? 2 : 8;
+    // kQuad, 1440x720, 4 views: 12.4 ms with 8 rows, 14.0 with 4, 13.1 with 2;
+    // with a launch per pass, whose last tiles leave compute units idle, 15.2
+    // with 8, 14.1 with 4, 14.7 with 2.  kWide, 640x320, 4 views: 3.4 with 2,
+    // 3.5 with 4.  kLane: pmp_queue.h
+    r.rows = !is_default(c) ? c.tile_rows : r.form == kLane ? 4 : r.form == kWide ? 2 : single ? 4 : 8;
     if (r.form == kWide && r.rows == 8) r.form = kQuad;
 }
 
@@ -832,7 +834,7 @@ static int batch_prepare(pmp_ctx* ctx, QueueState* q, const pmp_params* params, 
         it_init[k] = items[0];
         it_rows[k] = items[1];
     }
-    prop_shape(*q, c, n, nullptr, q->batch.h_slots, r);
+    prop_shape(*q, c, n, nullptr, q->batch.h_slots, false, r);
     for (int k = 0; k < n; ++k) it_prop[k] = slot_tiles(q->batch.h_slots[k], r.rows);
     fill_list(q->batch.h_hdr->init, n, it_init);
     fill_list(q->batch.h_hdr->prop, n, it_prop);

@@ -198,7 +198,7 @@ class GpuExec final : public sched::Executor {
         }
         const int n = (int)slots.size();
         QueueRun run;
-        prop_shape(*ctx->queue, cfg, (int)props.size(), props.data(), d.h_slots, run);
+        prop_shape(*ctx->queue, cfg, (int)props.size(), props.data(), d.h_slots, true, run);
         for (int s : props) items_prop[s] = slot_tiles(d.h_slots[s], run.rows);
         fill_list(d.h_hdr->init, n, items_init);
         fill_list(d.h_hdr->prop, n, items_prop);
