@@ -68,7 +68,7 @@ struct BatchHdr {
 // host staging copy, the band heads of the propagation queue, its tiles'
 // arrivals and rings (reached through the header, grown on demand), and the
 // hipGraphs captured over this set's device pointers.
-using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero + 2 form, rows, blocks, bands, postprocess + 2 fused
+using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero + 2 form, rows, blocks, bands, postprocess + 2 fused + 4 init_own
 constexpr int kHeadStride = 32;           // words: every head lies in a cache line of its own
 constexpr int kHeadWords = 24 * kHeadStride;
 struct DescSet {
@@ -94,6 +94,7 @@ struct QueueRun {
     int blocks = 0;           // persistent grid
     int bands = 1;            // per-XCD bands
     bool fused = false;       // all passes of a call in one launch
+    int init_own = 64;        // an init wave's pixels
 };
 
 // Default launch shape: the tile rows follow the form that the size and the
@@ -141,8 +142,8 @@ int slot_tiles(SlotDesc& d, int rows);
 void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
                 bool single, QueueRun& r);
 void fill_list(WorkList& L, int n, const int* items);
-// The rest of a shaped run; tiles: propagation tiles of a pass.
-int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
+// The rest of a shaped run over the work lists of h.
+int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, const BatchHdr& h,
               QueueRun& r);
 int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes);
 int q_init(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);

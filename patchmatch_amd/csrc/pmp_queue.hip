@@ -62,9 +62,13 @@ __global__ void k_fill_u32(unsigned int* __restrict__ p, int n, unsigned int v) 
 // with 6 views takes 1.05 ms, with a plane per lane 1.32.
 constexpr int kInitRows = 4;
 constexpr int kInitStageRows = kInitRows + 2 * kMaxHalf;
+// A wave owns kOwn pixels of the tile: 64, or 32 or 16 where the launch would
+// leave the chip idle (queue_run), which takes fewer rounds of score_wave.
+template <int kOwn>
 struct InitShared {
+    static constexpr int kWaves = 64 * kInitRows / kOwn;
     QuadTap walk[kQuadTaps];
-    QuadShared quad[kInitRows];
+    QuadShared quad[kWaves];
     float4 rs[64 * kInitRows];
     float4 plane[64 * kInitRows];
     float score[64 * kInitRows];
@@ -77,13 +81,15 @@ struct InitShared {
 static_assert(64 + 2 * kMaxHalf <= kTileCols, "init tile columns");
 
 // Waits for the previous tile's readers first.
-__device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitShared& st, int tx, int ty) {
+template <int kOwn>
+__device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitShared<kOwn>& st, int tx, int ty) {
+    constexpr int NT = 64 * InitShared<kOwn>::kWaves;
     const int r0 = ty * kInitRows - a.half, c0 = 64 * tx - a.half;
     const int nr = kInitRows + 2 * a.half, nc = 64 + 2 * a.half;
     __syncthreads();
-    for (int e = threadIdx.x; e < nc; e += 256) st.col[e] = a.coltab[min(max(c0 + e, 0), a.W - 1)];
-    for (int e = threadIdx.x; e < nr; e += 256) st.row[e] = a.rowtab[min(max(r0 + e, 0), a.H - 1)];
-    for (int e = threadIdx.x; e < nr * nc; e += 256) {
+    for (int e = threadIdx.x; e < nc; e += NT) st.col[e] = a.coltab[min(max(c0 + e, 0), a.W - 1)];
+    for (int e = threadIdx.x; e < nr; e += NT) st.row[e] = a.rowtab[min(max(r0 + e, 0), a.H - 1)];
+    for (int e = threadIdx.x; e < nr * nc; e += NT) {
         const int r = e / nc, c = e - r * nc;
         const int y = min(max(r0 + r, 0), a.H - 1), x = min(max(c0 + c, 0), a.W - 1);
         st.ref[r * kTileCols + c] = a.ref[(size_t)y * a.W + x];
@@ -95,13 +101,15 @@ __device__ __forceinline__ LdsTaps stage_init_tile(const KfArgs& a, InitShared& 
 // kScore: only score the working planes (pmp_score_plane_depth); otherwise
 // random initialisation + score + snapshot (RandomInitialization,
 // PatchMatchCuda.cu:210-270, depthmap.cc:656-663).
-template <bool kZero, bool kScore>
-__global__ __launch_bounds__(256) void k_init_q(const SlotDesc PMP_CONST* slots, const BatchHdr PMP_CONST* hdr) {
-    __shared__ InitShared st;
+template <bool kZero, bool kScore, int kOwn>
+__global__ __launch_bounds__(64 * InitShared<kOwn>::kWaves) void k_init_q(const SlotDesc PMP_CONST* slots,
+                                                                        const BatchHdr PMP_CONST* hdr) {
+    __shared__ InitShared<kOwn> st;
     const WorkList PMP_CONST* L = &hdr->init;
     const int total = L->total;
-    const int t = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const bool owner = kOwn == 64 || lane < kOwn;   // lanes beyond own no pixel but take part in the evaluations
+    const int t = kOwn * wave + (owner ? lane : 0);
     int cur = -1;
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         int local;
@@ -118,7 +126,7 @@ __global__ __launch_bounds__(256) void k_init_q(const SlotDesc PMP_CONST* slots,
         const LdsTaps tp = stage_init_tile(a, st, tx, ty);
         const int j = tx * 64 + (t & 63);
         const int i = ty * kInitRows + (t >> 6);
-        const bool in = i < a.H && j < a.W;
+        const bool in = owner && i < a.H && j < a.W;
         const bool scored = in && in_score_grid(a, i, j);
         const size_t k = in ? (size_t)i * a.W + j : 0;
         float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, dep = 0.0f;
@@ -132,20 +140,22 @@ __global__ __launch_bounds__(256) void k_init_q(const SlotDesc PMP_CONST* slots,
         }
         RefStat rs = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         if (scored) rs = ref_stats(a, tp, st.sWc, i, j);
-        st.rs[t] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
-        st.ic[t] = rs.Ic;
-        st.plane[t] = make_float4(p0, p1, p2, 0.0f);
+        if (owner) {
+            st.rs[t] = make_float4(rs.mx, rs.inv, rs.mxc, rs.vx);
+            st.ic[t] = rs.Ic;
+            st.plane[t] = make_float4(p0, p1, p2, 0.0f);
+        }
         wave_exchange();   // a wave reads its own pixels' entries
         auto at = [&](int p, int& row, int& col) {
             row = (p >> 6) + a.half;
             col = (p & 63) + a.half;
         };
         auto job = [&](int l, int& jt, float& px, float& py, float& pz) {
-            jt = 64 * wave + l;
+            jt = kOwn * wave + l;
             const float4 p = st.plane[jt];
             px = p.x; py = p.y; pz = p.z;
         };
-        auto put = [&](int l, float v) { st.score[64 * wave + l] = v; };
+        auto put = [&](int l, float v) { st.score[kOwn * wave + l] = v; };
         score_wave<kZero>(a, tp, st.walk, st.sWc, st.rs, st.ic, at, job, put, __ballot(scored), st.quad[wave]);
         const float sc = scored ? st.score[t] : __uint_as_float(0xFFFFFFFFu);   // cudaMemset(score, 0xFF) (depthmap.cc:657)
         if constexpr (kScore) {
@@ -602,8 +612,9 @@ static int check_config(pmp_ctx* ctx, const pmp_batch_config& c) {
 
 // Persistent grid: the configured blocks per CU, capped by (and defaulting
 // to) what fits on a CU at once; a multiple of 8 with per-XCD bands.
-int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, int tiles,
+int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, const BatchHdr& h,
               QueueRun& r) {
+    const int tiles = h.prop.total;
     int occ = 0;
     const PropKernel kern = prop_kernel(zero, r.form, r.rows);
     PMP_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern.fn, kern.threads, 0));
@@ -620,6 +631,12 @@ int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool
     // the launches' own barrier leaves the last ones whole compute units
     // (480x240, 4 views, 4 iterations: 4.4 against 2.4 ms).
     r.fused = 2 * tiles >= 3 * q.cus * bpc;
+    // a block of 16 waves fits on a CU once, of 8 twice: while every tile has
+    // one, its planes are scored in one or two rounds instead of four (init of
+    // 320x160, 8 views: 72 us, 108 with four; of 480x240: 114 and 123); beyond,
+    // the small blocks fill the chip better (640x320, 2 views: 82 us, 107 with
+    // 16 waves)
+    r.init_own = h.init.total <= q.cus ? 16 : h.init.total <= 2 * q.cus ? 32 : 64;
     r.zero = zero;
     r.post = post;
     r.bands = c.xcd_bands ? 1 : 0;
@@ -675,22 +692,32 @@ int ensure_sync(pmp_ctx* ctx, DescSet& d, size_t tiles) {
     return PMP_OK;
 }
 
-int q_init(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
-    PMP_QPTRS
-    const dim3 grd((unsigned)grid_blocks(ctx)), blk(256);
-    if (r.zero) hipLaunchKernelGGL((k_init_q<true, false>), grd, blk, 0, s, sl, hd);
-    else hipLaunchKernelGGL((k_init_q<false, false>), grd, blk, 0, s, sl, hd);
+template <bool kScore, int kOwn>
+static void launch_init_own(hipStream_t s, dim3 grd, const SlotDesc PMP_CONST* sl, const BatchHdr PMP_CONST* hd,
+                            bool zero) {
+    const dim3 blk(64 * InitShared<kOwn>::kWaves);
+    if (zero) hipLaunchKernelGGL((k_init_q<true, kScore, kOwn>), grd, blk, 0, s, sl, hd);
+    else hipLaunchKernelGGL((k_init_q<false, kScore, kOwn>), grd, blk, 0, s, sl, hd);
+}
+template <bool kScore>
+static int launch_init(pmp_ctx* ctx, hipStream_t s, const SlotDesc PMP_CONST* sl, const BatchHdr PMP_CONST* hd,
+                       const QueueRun& r) {
+    const unsigned n = (unsigned)grid_blocks(ctx);
+    if (r.init_own == 16) launch_init_own<kScore, 16>(s, dim3(n / 8), sl, hd, r.zero);
+    else if (r.init_own == 32) launch_init_own<kScore, 32>(s, dim3(n / 4), sl, hd, r.zero);
+    else launch_init_own<kScore, 64>(s, dim3(n), sl, hd, r.zero);
     PMP_HIP(ctx, hipGetLastError());
     return PMP_OK;
 }
 
+int q_init(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
+    PMP_QPTRS
+    return launch_init<false>(ctx, s, sl, hd, r);
+}
+
 int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
     PMP_QPTRS
-    const dim3 grd((unsigned)grid_blocks(ctx)), blk(256);
-    if (r.zero) hipLaunchKernelGGL((k_init_q<true, true>), grd, blk, 0, s, sl, hd);
-    else hipLaunchKernelGGL((k_init_q<false, true>), grd, blk, 0, s, sl, hd);
-    PMP_HIP(ctx, hipGetLastError());
-    return PMP_OK;
+    return launch_init<true>(ctx, s, sl, hd, r);
 }
 
 // One launch over passes [first, first + passes), with the heads of launch `launch`.
@@ -781,7 +808,7 @@ static int q_sequence(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r
 int q_densify(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes, bool use_graph) {
     // per-stage timing needs events between the launches: no graph then
     if (!use_graph || ctx->timing) return q_sequence(ctx, s, d, r, passes);
-    const GraphKey key{passes, (r.zero ? 1 : 0) + 2 * r.form, r.rows, r.blocks, r.bands, (r.post ? 1 : 0) + (r.fused ? 2 : 0)};
+    const GraphKey key{passes, (r.zero ? 1 : 0) + 2 * r.form, r.rows, r.blocks, r.bands, (r.post ? 1 : 0) + (r.fused ? 2 : 0) + 4 * r.init_own};
     auto it = d.graphs.find(key);
     if (it == d.graphs.end()) {
         hipGraph_t g = nullptr;
@@ -862,7 +889,7 @@ int pmp_batch_densify(pmp_ctx* ctx, const pmp_params* params, int32_t n, const p
     QueueRun r;
     if ((rc = batch_prepare(ctx, q, params, n, kfs, q->cfg, r, true))) return rc;
     if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0,
-                        q->batch.h_hdr->prop.total, r)))
+                        *q->batch.h_hdr, r)))
         return rc;
     if ((rc = q_densify(ctx, ctx->stream, q->batch, r, 2 * params->iterations, q->cfg.use_graph != 0))) return rc;
     q->n_last = n;
@@ -930,7 +957,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
         c.blocks_per_cu = 32;
         QueueRun r;
         if ((rc = batch_prepare(ctx, q, params, n, kfs, c, r, false))) break;
-        if ((rc = queue_run(ctx, *q, c, zero, false, q->batch.h_hdr->prop.total, r))) break;
+        if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, r))) break;
         const int occ = r.blocks / (q->cus > 0 ? q->cus : 1);   // blocks per CU that fit (rounding aside)
         // at least 8 waves per CU (rows waves per block): fewer leave SIMDs
         // idle and measured 1.3-4x slower, and their trials are the longest
@@ -939,7 +966,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
             for (int bands = 0; bands <= 1 && rc == 0; ++bands) {
                 c.blocks_per_cu = bpc;
                 c.xcd_bands = bands;
-                if ((rc = queue_run(ctx, *q, c, zero, false, q->batch.h_hdr->prop.total, r))) break;
+                if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, r))) break;
                 // same starting maps for every candidate: init, then time every
                 // pass.  The first passes score random planes (most candidates
                 // survive pre-rejection, the gathers scatter); the converged
