@@ -245,9 +245,9 @@ int pmp_eval_counts(pmp_ctx* ctx, int64_t* evals, int64_t* candidates);
  * stream, reports the launches recorded since the previous call, and resets. */
 typedef struct pmp_timing {
     double init_ms;           /* random initialisation + initial score */
-    double propagate_ms;      /* sum over red-black pass launches */
+    double propagate_ms;      /* sum over red-black passes */
     double finalize_ms;       /* copy-back, gate, PostProcess */
-    int32_t propagate_launches;
+    int32_t propagate_launches;  /* red-black passes (several may share a launch) */
     int32_t densify_calls;
 } pmp_timing;
 int pmp_set_timing(pmp_ctx* ctx, int32_t enable);
