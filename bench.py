@@ -51,17 +51,17 @@ sys.path.insert(0, ROOT)
 FP32_PEAK_TFLOPS = 157.3            # MI355X published FP32 vector peak (counts packed FP32 FMA)
 FP32_NONPACKED_PEAK_TFLOPS = 78.6   # the same without packed FP32, which this build does not use
 HBM_PEAK_GBS = 8000.0
-# L2-to-memory bytes per k_propagate_q launch on the 1920x960 + 6-view
+# L2-to-memory bytes per red-black pass of k_propagate_q on the 1920x960 + 6-view
 # workload, from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a copy of known
 # size (profiles/k_propagate_q_c1_1920x960_6views.md); None for other workloads.
-TRAFFIC_BYTES_PER_LAUNCH_C1 = int((181_613 * 2.00 + 43_038 * 1.00) * 1024)
+TRAFFIC_BYTES_PER_LAUNCH_C1 = int((172_519 * 2.00 + 71_330 * 1.00) * 1024)
 TRAFFIC_SOURCE = ("profile-derived, not measured in this run: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of "
                   "k_propagate_q on this workload, scaled by a streaming copy of known size "
                   "(profiles/k_propagate_q_c1_1920x960_6views.md)")
-# VALU wave-instructions per k_propagate_q launch on the 1920x960 + 6-view
+# VALU wave-instructions per red-black pass of k_propagate_q on the 1920x960 + 6-view
 # workload (rocprofv3 --pmc SQ_INSTS_VALU, same profile): the issue side of
 # the roofline, against one wave64 VALU instruction per CU per clock.
-VALU_WAVE_INSTS_PER_LAUNCH_C1 = 2.539e9
+VALU_WAVE_INSTS_PER_LAUNCH_C1 = 2.614e9
 CUS, CLOCK_HZ = 256, 2.4e9
 
 
@@ -306,7 +306,7 @@ def main(argv=None):
                      "peak_nonpacked": FP32_NONPACKED_PEAK_TFLOPS,
                      "frac_nonpacked": round(achieved_tflops / FP32_NONPACKED_PEAK_TFLOPS, 4),
                      "traffic": TRAFFIC_BYTES_PER_LAUNCH_C1 if (args.width, args.height, N) == (1920, 960, 6) else None,
-                     "traffic_unit": "bytes per launch (L2 misses)", "traffic_source": TRAFFIC_SOURCE,
+                     "traffic_unit": "bytes per red-black pass (L2 misses)", "traffic_source": TRAFFIC_SOURCE,
                      "ops_model": "T (19 + 52 N) + 25 N + 10 FP32 ops per hypothesis evaluation "
                                   "(FMA 2, add/mul/compare 1, each elementary function 1); executed evaluations "
                                   "only (pre-rejected candidates are not scored)",
