@@ -28,16 +28,7 @@ __device__ __forceinline__ void count_add_wave(unsigned long long* ctr, unsigned
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(ctr, (unsigned long long)v);
 }
 
-// Workgroups are dispatched to the 8 XCDs round-robin by linear block id.  The
-// grid is padded to a multiple of 8 and block b is given tile
-// (b mod 8) * (nb8/8) + b/8, so each XCD walks one contiguous band of tiles
-// and its L2 holds that band's neighbour rows.  Returns -1 for padding blocks.
-__device__ __forceinline__ int xcd_tile(int b, int nb8, int nb) {
-    const int t = (b & 7) * (nb8 >> 3) + (b >> 3);
-    return t < nb ? t : -1;
-}
-
-// The same for a keyframe's tap walk (quad_tap).
+// A keyframe's tap walk (quad_tap) into LDS; every thread of the block takes part.
 __device__ __forceinline__ void load_walk(const KfArgs& a, QuadTap* tab) {
     const int n = (a.T + 3) / 4 * 4;
     for (int k = threadIdx.x; k < n; k += blockDim.x) tab[k] = quad_tap(a, k);
