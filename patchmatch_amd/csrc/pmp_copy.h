@@ -62,7 +62,7 @@ private:
     // the threads costs more (normals of 328x182, 716 KB down: 66 us alone, 52
     // with them; a 614 KB image up: 75 and 76).
     static constexpr size_t kAloneDown = size_t(512) << 10, kAloneUp = size_t(768) << 10;
-    // Uploads from kAloneUp to this are the runtime's own: it pins the pages and
+    // Uploads of contiguous rows from kAloneUp to this are the runtime's own: it pins the pages and
     // copies from them (five 640x320 maps to the cleaner and back: 222 us, with
     // the threads 292; of 800x400: 363 and 353; of 1363x677: 863 and 638).
     static constexpr size_t kPinned = size_t(6) << 20;

@@ -176,6 +176,15 @@ static size_t total(const HostCopy* c, int n) {
     return b;
 }
 
+// Whether the rows of every copy follow each other in host memory.  The runtime
+// moves other rows of pageable memory one by one, about 9 us each (a 1920x960
+// image with a pitch of 2048: 8.8 ms, through the ring 0.06).
+static bool contiguous(const HostCopy* c, int n) {
+    for (int k = 0; k < n; ++k)
+        if (c[k].row != c[k].pitch && c[k].rows > 1) return false;
+    return true;
+}
+
 static hipError_t plain(hipStream_t s, const HostCopy* c, int n, hipMemcpyKind kind, bool wait) {
     const bool in = kind == hipMemcpyHostToDevice;
     for (int k = 0; k < n; ++k) {
@@ -260,7 +269,7 @@ hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, bool waits
     if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
     const size_t bytes = total(c, n);
     if (bytes < kAloneUp) return small(s, c, n, false);
-    if (bytes < kPinned) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
+    if (bytes < kPinned && contiguous(c, n)) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
     const bool alone = !start_threads();
     Walk w{c, n};
     bool more = true;
