@@ -15,21 +15,19 @@ int set_error(pmp_ctx* ctx, int code, const std::string& msg) {
     return code;
 }
 
-int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch,
-                     hipStream_t s) {
-    const HostCopy c{const_cast<uint8_t*>(src), dst, row, rows, pitch};
-    PMP_HIP(ctx, ctx->copier.to_device(s, &c, 1));
-    return PMP_OK;
-}
-
 int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n, bool fresh) {
     PMP_HIP(ctx, ctx->copier.to_host(ctx->stream, c, n, fresh));
     return PMP_OK;
 }
 
-int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, bool waits) {
-    PMP_HIP(ctx, ctx->copier.to_device(ctx->stream, c, n, waits));
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, Until until) {
+    PMP_HIP(ctx, ctx->copier.to_device(ctx->stream, c, n, until));
     return PMP_OK;
+}
+
+int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch, Until until) {
+    const HostCopy c{const_cast<uint8_t*>(src), dst, row, rows, pitch};
+    return copy_to_device(ctx, &c, 1, until);
 }
 
 int check_hip(pmp_ctx* ctx, hipError_t e, const char* what) {
@@ -388,7 +386,7 @@ int pmp_image_put(pmp_ctx* ctx, uint64_t id, const uint8_t* pixels, int32_t widt
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         rc = e == hipSuccess ? PMP_OK : check_hip(ctx, e, "pmp_image_put copy");
     } else {
-        rc = upload_host_rows(ctx, im.gray, pixels, (size_t)width, (size_t)height, (size_t)pitch, ctx->stream);
+        rc = upload_host_rows(ctx, im.gray, pixels, (size_t)width, (size_t)height, (size_t)pitch);
     }
     if (rc) {
         free_image(im);

@@ -37,15 +37,21 @@ inline HostCopy flat_copy(const void* host, const void* dev, size_t bytes) {
     return HostCopy{const_cast<void*>(host), const_cast<void*>(dev), bytes, 1, bytes};
 }
 
+// What an upload has done when it returns.
+enum class Until {
+    kDone,     // it is complete
+    kRead,     // the host memory has been read
+    kQueued,   // it is queued: the caller waits for the stream before it returns (an upload that failed is not)
+};
+
 class Copier {
 public:
     ~Copier();
     // Device to host after the work queued on s; complete on return.  fresh:
     // to memory that has hardly been touched since it was allocated.
     hipError_t to_host(hipStream_t s, const HostCopy* c, int n, bool fresh = false);
-    // Host to device in stream order; on return the host memory has been read,
-    // unless the caller waits for the stream itself before it returns (waits).
-    hipError_t to_device(hipStream_t s, const HostCopy* c, int n, bool waits = false);
+    // Host to device in stream order.
+    hipError_t to_device(hipStream_t s, const HostCopy* c, int n, Until until = Until::kDone);
     // Host to host.
     void copy(void* dst, const void* src, size_t bytes);
 

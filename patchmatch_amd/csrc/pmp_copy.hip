@@ -194,7 +194,10 @@ static hipError_t plain(hipStream_t s, const HostCopy* c, int n, hipMemcpyKind k
                 ? hipMemcpyAsync(in ? c[k].dev : c[k].host, in ? c[k].host : c[k].dev, c[k].row * c[k].rows, kind, s)
                 : hipMemcpy2DAsync(in ? c[k].dev : c[k].host, in ? c[k].row : c[k].pitch, in ? c[k].host : c[k].dev,
                                    in ? c[k].pitch : c[k].row, c[k].row, c[k].rows, kind, s);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s);   // nothing reads or writes the host memory any more
+            return e;
+        }
     }
     return wait ? hipStreamSynchronize(s) : hipSuccess;
 }
@@ -264,12 +267,13 @@ hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n, bool fresh) 
     return e;
 }
 
-hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, bool waits) {
+hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, Until until) {
     std::lock_guard<std::mutex> lk(mu_);
-    if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
+    const bool wait_plain = until != Until::kQueued;   // the runtime may still read the host memory
+    if (!pageable(c, n) || !start_ring()) return plain(s, c, n, hipMemcpyHostToDevice, wait_plain);
     const size_t bytes = total(c, n);
     if (bytes < kAloneUp) return small(s, c, n, false);
-    if (bytes < kPinned && contiguous(c, n)) return plain(s, c, n, hipMemcpyHostToDevice, !waits);
+    if (bytes < kPinned && contiguous(c, n)) return plain(s, c, n, hipMemcpyHostToDevice, wait_plain);
     const bool alone = !start_threads();
     Walk w{c, n};
     bool more = true;
@@ -295,7 +299,10 @@ hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, bool waits
         ++sent;
     }
     for (const Slot& sl : slot_) wait(sl.begin, sl.end);   // no thread reads the caller's memory any more
-    return e;
+    if (e == hipSuccess && until != Until::kDone) return e;
+    const hipError_t d = hipStreamSynchronize(s);
+    for (Slot& sl : slot_) sl.dma = false;
+    return e == hipSuccess ? d : e;
 }
 
 void Copier::copy(void* dst, const void* src, size_t bytes) {

@@ -344,10 +344,7 @@ int pmp_set_maps(pmp_ctx* ctx, const float* plane4, const float* depth, const fl
     if (plane4) c[n++] = flat_copy(plane4, ctx->ws.plane, P * 16);
     if (depth) c[n++] = flat_copy(depth, ctx->ws.depth, P * 4);
     if (score) c[n++] = flat_copy(score, ctx->ws.score, P * 4);
-    int rc = copy_to_device(ctx, c, n, true);
-    if (rc) return rc;
-    PMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PMP_OK;
+    return copy_to_device(ctx, c, n);
 }
 
 int pmp_get_maps(pmp_ctx* ctx, int32_t which, float* plane4, float* depth, float* score, int32_t* nghbr) {

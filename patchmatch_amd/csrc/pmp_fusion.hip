@@ -381,10 +381,14 @@ static int clean_impl(pmp_ctx* ctx, int32_t width, int32_t height, int32_t n_map
         const double cs = cos((double)max_normal_deg * (M_PI / 180.0));
         c.cos2 = cs * cs;
     }
-    if ((rc = copy_to_device(ctx, up, n_up, true))) return rc;
+    if ((rc = copy_to_device(ctx, up, n_up, Until::kQueued))) return rc;
     dim3 blk(256), grd((width + 255) / 256, height);
     hipLaunchKernelGGL(k_clean, grd, blk, 0, ctx->stream, a, c, ctx->clean_maps, min_consistent, dout);
-    PMP_HIP(ctx, hipGetLastError());
+    const hipError_t launched = hipGetLastError();
+    if (launched != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);   // the uploads read the caller's maps
+        return check_hip(ctx, launched, "k_clean");
+    }
     const HostCopy down = flat_copy(cleaned, dout, P * sizeof(float));
     return copy_to_host(ctx, &down, 1);
 }

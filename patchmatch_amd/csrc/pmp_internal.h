@@ -187,17 +187,15 @@ enum { kStageInit = 0, kStagePropagate = 1, kStageFinalize = 2 };
 int timing_begin(pmp_ctx* ctx, int stage, int passes = 1);
 void timing_end(pmp_ctx* ctx, int pair);
 int check_hip(pmp_ctx* ctx, hipError_t e, const char* what);
-// `rows` host rows of `row` bytes, `pitch` bytes apart, to contiguous device
-// memory at dst on stream s, and waits for the copy.  The rows are packed into
-// a pinned staging buffer of the context (grown on demand) and sent in one
-// copy: a 2D copy from pageable memory moves row by row, about 9 us a row.
-// The caller's memory from and to the device (Copier); from the device after
-// the work queued on s, complete on return; to the device in stream order, the
-// host memory read on return unless the caller waits for the stream (waits).
+// The caller's memory from and to the device (Copier): from the device after
+// the work queued on the context's stream, complete on return; to the device in
+// stream order.
 int copy_to_host(pmp_ctx* ctx, const HostCopy* c, int n, bool fresh = false);
-int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, bool waits = false);
+int copy_to_device(pmp_ctx* ctx, const HostCopy* c, int n, Until until = Until::kDone);
+// `rows` host rows of `row` bytes, `pitch` bytes apart, to contiguous device
+// memory at dst, in stream order.
 int upload_host_rows(pmp_ctx* ctx, void* dst, const uint8_t* src, size_t row, size_t rows, size_t pitch,
-                     hipStream_t s);
+                     Until until = Until::kDone);
 int ensure_workspace(pmp_ctx* ctx, int W, int H);
 struct Tables {
     const float2* row = nullptr;

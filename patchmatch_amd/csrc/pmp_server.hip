@@ -102,7 +102,6 @@ class GpuExec final : public sched::Executor {
             const HostCopy c = flat_copy(pixels, im.gray, im.bytes);
             e = ctx->copier.to_device(copy, &c, 1);
         }
-        if (e == hipSuccess) e = hipStreamSynchronize(copy);
         if (e != hipSuccess) {
             if (im.gray) (void)hipFree(im.gray);
             err = "upload of image " + std::to_string(id) + ": " + hipGetErrorString(e);

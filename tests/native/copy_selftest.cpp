@@ -6,7 +6,6 @@
 #include <stdio.h>
 #include <stdlib.h>
 
-#include <random>
 #include <set>
 #include <string>
 #include <thread>
@@ -29,9 +28,13 @@ static hip_sim::Stats& st = hip_sim::stats();
 constexpr size_t KiB = 1024, MiB = 1024 * KiB;
 
 static Bytes noise(size_t n, unsigned seed) {
-    std::mt19937 g(seed);
-    Bytes b(n);
-    for (size_t k = 0; k < n; ++k) b[k] = (uint8_t)(g() >> 11);
+    Bytes b(n + 8);
+    uint64_t x = 0x9E3779B97F4A7C15ull * (seed + 1);
+    for (size_t k = 0; k < n; k += 8) {
+        x = x * 6364136223846793005ull + 1442695040888963407ull;
+        memcpy(&b[k], &x, 8);
+    }
+    b.resize(n);
     return b;
 }
 
@@ -43,7 +46,7 @@ static int round_trip(Copier& c, hipStream_t s, size_t row, size_t rows, size_t 
     const int before = st.copies_2d;
     const HostCopy up{const_cast<uint8_t*>(host.data()), dev.data(), row, rows, pitch};
     CHECK(c.to_device(s, &up, 1) == hipSuccess);
-    s->sync();
+    CHECK(s->idle());
     for (size_t r = 0; r < rows; ++r) CHECK(memcmp(&dev[r * row], &host[r * pitch], row) == 0);
     const HostCopy down = flat_copy(back.data(), dev.data(), row * rows);
     CHECK(c.to_host(s, &down, 1) == hipSuccess);
@@ -61,12 +64,53 @@ static void pitched() {
             for (size_t pad : {0, 5, 128}) CHECK(round_trip(c, &s, row, rows, row + pad) == 0);
 }
 
+// What an upload has done on return: everything by default, also in the sizes
+// that the runtime copies itself; read the host memory (kRead); and after a
+// failed copy nothing touches either side any more.
+static void until() {
+    hip_sim::Stream s;
+    Copier c;
+    for (size_t n : {1 * KiB, 700 * KiB, 2 * MiB, 7 * MiB, 13 * MiB, 30 * MiB}) {
+        st.delay_us = 1000;
+        const Bytes host = noise(n, (unsigned)n);
+        for (Until u : {Until::kDone, Until::kRead, Until::kQueued}) {
+            Bytes src = host, dev(n);
+            const HostCopy up = flat_copy(src.data(), dev.data(), n);
+            CHECK(c.to_device(&s, &up, 1, u) == hipSuccess);
+            if (u == Until::kDone) CHECK(s.idle());
+            if (u == Until::kQueued) s.sync();
+            std::fill(src.begin(), src.end(), uint8_t(0));   // the caller's own again
+            s.sync();
+            CHECK(dev == host);
+        }
+        for (int at = 0; at < 8; ++at)
+            for (bool out : {false, true}) {
+                st.delay_us = 200;
+                Bytes src = host, dev(n);
+                const HostCopy k = flat_copy(src.data(), dev.data(), n);
+                st.fail_copy_in = at;
+                const hipError_t e = out ? c.to_host(&s, &k, 1) : c.to_device(&s, &k, 1);
+                const bool hit = st.fail_copy_in < 0;
+                st.fail_copy_in = -1;
+                CHECK((e == hipSuccess) == !hit);
+                CHECK(s.idle());
+                // the next transfer is whole
+                st.delay_us = 0;
+                Bytes to(n);
+                src = host;
+                const HostCopy up = flat_copy(src.data(), to.data(), n);
+                CHECK(c.to_device(&s, &up, 1) == hipSuccess && to == host);
+            }
+    }
+    st.delay_us = 0;
+}
+
 int main(int argc, char** argv) {
     std::set<std::string> want(argv + 1, argv + argc);
     struct {
         const char* name;
         void (*f)();
-    } parts[] = {{"pitched", pitched}};
+    } parts[] = {{"pitched", pitched}, {"until", until}};
     for (auto& p : parts)
         if (want.empty() || want.count(p.name)) {
             p.f();
