@@ -3,6 +3,8 @@
 // the first failed check (or a sanitizer report).
 //
 //   copy_selftest [part ...]     the parts by name; all of them by default
+#include <dirent.h>
+#include <signal.h>
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -62,6 +64,11 @@ static void pitched() {
     for (size_t row : {700, 1920, 4099})
         for (size_t rows : {1, 3, 400, 960, 1100, 2300})
             for (size_t pad : {0, 5, 128}) CHECK(round_trip(c, &s, row, rows, row + pad) == 0);
+    // nor without pinned memory
+    st.fail_pinned = true;
+    Copier d;
+    for (size_t rows : {1, 400, 960, 2300}) CHECK(round_trip(d, &s, 1920, rows, 2048) == 0);
+    st.fail_pinned = false;
 }
 
 // What an upload has done on return: everything by default, also in the sizes
@@ -85,6 +92,7 @@ static void until() {
         }
         for (int at = 0; at < 8; ++at)
             for (bool out : {false, true}) {
+                if (n < 6 * MiB && at > 1) continue;   // one copy
                 st.delay_us = 200;
                 Bytes src = host, dev(n);
                 const HostCopy k = flat_copy(src.data(), dev.data(), n);
@@ -105,12 +113,95 @@ static void until() {
     st.delay_us = 0;
 }
 
+// The process's threads and, of those beside them, the ones that take no signal.
+static void threads(size_t* all, size_t* deaf) {
+    *all = *deaf = 0;
+    DIR* d = opendir("/proc/self/task");
+    CHECK(d);
+    while (dirent* e = readdir(d)) {
+        if (e->d_name[0] == '.') continue;
+        FILE* f = fopen(("/proc/self/task/" + std::string(e->d_name) + "/status").c_str(), "r");
+        if (!f) continue;   // gone meanwhile
+        ++*all;
+        char line[256];
+        unsigned long long blocked = 0;
+        while (fgets(line, sizeof(line), f)) sscanf(line, "SigBlk: %llx", &blocked);
+        fclose(f);
+        if ((blocked >> (SIGINT - 1)) & (blocked >> (SIGTERM - 1)) & (blocked >> (SIGUSR1 - 1)) & 1) ++*deaf;
+    }
+    closedir(d);
+}
+
+// Contexts share rings and threads: the second one's transfers allocate
+// nothing and start no thread, many at once stay within bounds, and the last
+// context gives everything back.
+static void shared() {
+    hip_sim::Stream s[12];
+    size_t all0, deaf0, all, deaf;
+    threads(&all0, &deaf0);
+    CHECK(st.pinned_held == 0);
+    {
+        Copier a;
+        CHECK(round_trip(a, &s[0], 20 * MiB, 1, 20 * MiB) == 0);
+        const int pins = st.pinned_allocs;
+        CHECK(pins > 0);
+        threads(&all, &deaf);
+        const size_t started = all - all0;
+        CHECK(started <= 8 && deaf - deaf0 == started);
+        CHECK(round_trip(a, &s[0], 20 * MiB, 1, 20 * MiB) == 0);
+        {
+            Copier b;
+            for (size_t n : {8 * KiB, 600 * KiB, 9 * MiB, 20 * MiB}) CHECK(round_trip(b, &s[1], n, 1, n) == 0);
+            CHECK(st.pinned_allocs == pins);
+            threads(&all, &deaf);
+            CHECK(all - all0 == started);
+        }
+        std::vector<std::thread> ts;
+        std::atomic<int> busy{0};
+        for (int k = 0; k < 12; ++k)
+            ts.emplace_back([&, k] {
+                Copier c;
+                busy++;
+                for (int r = 0; r < 4; ++r) {
+                    const size_t n = 8 * MiB + 4099 * k;
+                    round_trip(c, &s[k], n, 1, n);
+                }
+            });
+        for (auto& t : ts) t.join();
+        CHECK(st.pinned_held <= 4);
+        threads(&all, &deaf);
+        CHECK(all - all0 <= 8);
+    }
+    CHECK(st.pinned_held == 0 && st.events == 0);
+    threads(&all, &deaf);
+    CHECK(all == all0);
+}
+
+// A transfer does not wait for the DMAs that another stream's left behind.
+static void streams() {
+    hip_sim::Stream slow, s;
+    Copier a, b;
+    const size_t n = 8 * MiB;
+    const Bytes x = noise(n, 1);
+    Bytes dx(n), dy(n), y = x;
+    const HostCopy up = flat_copy(y.data(), dx.data(), n);
+    std::atomic<bool> go{false};
+    slow.push([&] { while (!go) std::this_thread::yield(); });   // work before the upload
+    CHECK(a.to_device(&slow, &up, 1, Until::kRead) == hipSuccess);
+    std::fill(y.begin(), y.end(), uint8_t(0));
+    const HostCopy up2 = flat_copy(x.data(), dy.data(), n);
+    CHECK(b.to_device(&s, &up2, 1) == hipSuccess && dy == x);    // would hang
+    go = true;
+    slow.sync();
+    CHECK(dx == x);
+}
+
 int main(int argc, char** argv) {
     std::set<std::string> want(argv + 1, argv + argc);
     struct {
         const char* name;
         void (*f)();
-    } parts[] = {{"pitched", pitched}, {"until", until}};
+    } parts[] = {{"pitched", pitched}, {"until", until}, {"shared", shared}, {"streams", streams}};
     for (auto& p : parts)
         if (want.empty() || want.count(p.name)) {
             p.f();

@@ -17,7 +17,7 @@
 #include <mutex>
 #include <thread>
 
-enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorUnknown = 999 };
+enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorNotReady = 600, hipErrorUnknown = 999 };
 enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
 enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2 };
 constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2;
@@ -28,7 +28,7 @@ struct hipPointerAttribute_t {
 namespace hip_sim {
 
 struct Stats {
-    std::atomic<int> pinned_allocs{0}, copies_1d{0}, copies_2d{0}, from_pageable{0}, events{0};
+    std::atomic<int> pinned_allocs{0}, pinned_held{0}, copies_1d{0}, copies_2d{0}, from_pageable{0}, events{0};
     std::atomic<int> fail_copy_in{-1};      // the n-th copy from now fails
     std::atomic<bool> fail_pinned{false};
     std::atomic<int> delay_us{0};           // of each copy
@@ -72,6 +72,10 @@ public:
             n = queued_;
         }
         wait(n);
+    }
+    bool reached(uint64_t n) {
+        std::lock_guard<std::mutex> lk(mu_);
+        return done_ >= n;
     }
     bool idle() {
         std::lock_guard<std::mutex> lk(mu_);
@@ -125,6 +129,7 @@ inline hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
     std::lock_guard<std::mutex> lk(hip_sim::ranges().mu);
     hip_sim::ranges().pinned[(uintptr_t)*p] = bytes;
     hip_sim::stats().pinned_allocs++;
+    hip_sim::stats().pinned_held++;
     return hipSuccess;
 }
 inline hipError_t hipHostFree(void* p) {
@@ -133,6 +138,7 @@ inline hipError_t hipHostFree(void* p) {
         hip_sim::ranges().pinned.erase((uintptr_t)p);
     }
     free(p);
+    hip_sim::stats().pinned_held--;
     return hipSuccess;
 }
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
@@ -167,6 +173,10 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) {
     }
     if (s) s->wait(at);
     return hipSuccess;
+}
+inline hipError_t hipEventQuery(hipEvent_t e) {
+    std::lock_guard<std::mutex> lk(e->mu);
+    return !e->s || e->s->reached(e->at) ? hipSuccess : hipErrorNotReady;
 }
 inline hipError_t hipStreamSynchronize(hipStream_t s) {
     s->sync();

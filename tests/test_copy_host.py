@@ -13,13 +13,13 @@ ENV = dict(os.environ, ASAN_OPTIONS="detect_leaks=1", UBSAN_OPTIONS="halt_on_err
 
 
 @pytest.mark.parametrize("san", ["asan", "tsan"])
-@pytest.mark.parametrize("part", ["pitched", "until"])
+@pytest.mark.parametrize("part", ["pitched", "until", "shared", "streams"])
 def test_copies(san, part):
     r = subprocess.run(["make", "-s", "-C", NATIVE, f"build/copy_selftest_{san}"], capture_output=True, text=True,
                        timeout=300)
     assert r.returncode == 0, r.stderr[-3000:]
     r = subprocess.run([os.path.join(NATIVE, "build", f"copy_selftest_{san}"), part], capture_output=True, text=True,
-                       timeout=120, env=ENV)
+                       timeout=100, env=ENV)
     if "unexpected memory mapping" in r.stderr:
         pytest.skip("ThreadSanitizer cannot map its shadow memory on this kernel")
     assert r.returncode == 0 and f"{part} ok" in r.stdout, f"rc {r.returncode}\n{r.stdout}\n{r.stderr[-6000:]}"
