@@ -224,6 +224,10 @@ __device__ __forceinline__ void epoch_leave(const SlotDesc& d, int tx, int ty, i
 // store (a ring slot announced but not written yet, one taken but not read
 // yet) are for blocks that are past every other wait.
 //
+// The hand-over is ordered: a completed tile's maps are released with its
+// arrivals, the last arrival acquires the others' and releases all with the
+// ring entry, and the wave that takes the entry acquires them for its block.
+//
 // heads: three words per band, each in a cache line of its own.
 __device__ __forceinline__ unsigned int* head_of(unsigned int* heads, int kind, int band) {
     return heads + (kind * 8 + band) * kHeadStride;
@@ -321,14 +325,20 @@ __device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, con
     if (x < 0 || y < 0 || x >= nbx || y >= nby) return;
     const int t = item - (ty * nbx + tx) + y * nbx + x;
     const int around = (min(x + 1, nbx - 1) - max(x - 1, 0) + 1) * (min(y + 1, nby - 1) - max(y - 1, 0) + 1);
-    const int arrived = (int)atomicAdd(&hdr->sync[(size_t)(pass & 1) * total + t], 1u) + 1;
+    const int arrived = (int)__hip_atomic_fetch_add(&hdr->sync[(size_t)(pass & 1) * total + t], 1u, __ATOMIC_ACQ_REL,
+                                                    __HIP_MEMORY_SCOPE_AGENT) + 1;
     if (arrived != around * (pass / 2 + 1)) return;
     int band = (int)(((long long)t * nb) / total);
     while (t >= band_lo(total, band + 1, nb)) ++band;
     const int lo = band_lo(total, band, nb), n = band_lo(total, band + 1, nb) - lo;
     const int q = (int)atomicAdd(head_of(heads, kHeadTail, band), 1u);
     unsigned int* slot = hdr->sync + 2 * (size_t)total + lo + q % n;
-    while (atomicCAS(slot, 0u, ((unsigned int)(pass + 1) << 24) | (unsigned int)t) != 0u) __builtin_amdgcn_s_sleep(1);
+    unsigned int empty = 0u;
+    while (!__hip_atomic_compare_exchange_strong(slot, &empty, ((unsigned int)(pass + 1) << 24) | (unsigned int)t,
+                                                 __ATOMIC_RELEASE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        empty = 0u;
+        __builtin_amdgcn_s_sleep(1);
+    }
 }
 
 // One launch over `passes` red-black passes of every slot, the first being
@@ -347,7 +357,11 @@ __global__ __launch_bounds__((kPropThreads<R, F>))
     unsigned int n_eval = 0, n_cand = 0;   // of the wave
     int cur = -1;
     for (;;) {
-        if (threadIdx.x < 64) take_tile(hdr, passes, heads, bands, sh);
+        if (threadIdx.x < 64) {
+            take_tile(hdr, passes, heads, bands, sh);
+            // the maps that the ring entry hands over (release_tiles), before the block reads any
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
         __syncthreads();
         const int item = sh.item, pass = sh.pass;
         __syncthreads();

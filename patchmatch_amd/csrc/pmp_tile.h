@@ -113,7 +113,7 @@ struct PropShared {
 // The maps that tiles of one launch hand each other (pass fusion: a tile of
 // pass p + 1 runs beside tiles of pass p) go through agent-scope accesses:
 // the XCDs' L2 caches are not coherent with each other for plain ones within
-// a launch.
+// a launch.  The taking of a tile orders them (take_tile, release_tiles).
 __device__ __forceinline__ float load_map(const float* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
