@@ -276,11 +276,15 @@ typedef struct pmp_keyframe {
 /* Result-invariant launch configuration of the batched kernels: every value
  * gives bit-identical maps, only the speed differs. */
 typedef struct pmp_batch_config {
-    int32_t tile_rows;        /* size of a propagation tile: 64*tile_rows same-colour pixels (2, 4 or 8).  With the
-                                 default, 2 and blocks_per_cu 0, large launches take 4 or 8 */
-    int32_t blocks_per_cu;    /* persistent propagation blocks per CU (0: as many as fit and pay) */
+    int32_t tile_rows;        /* size of a propagation tile: 64*tile_rows same-colour pixels (2, 4 or 8).  The
+                                 default, 2 with blocks_per_cu 0, chooses the size by the pixels and views of
+                                 the launch; any other setting is taken as it is (2 with blocks_per_cu 32: tiles
+                                 of 2 at every size, as many blocks as fit) */
+    int32_t blocks_per_cu;    /* persistent propagation blocks per CU (0: as many as fit and pay; at most as many
+                                 as fit, and as there are tiles for) */
     int32_t use_graph;        /* 1: replay the whole batch (init, 2*iterations passes, finalize) as one hipGraph */
-    int32_t xcd_bands;        /* 1: each XCD drains its own contiguous band of tiles first */
+    int32_t xcd_bands;        /* 1: the tiles are split into a contiguous band for each XCD, whose blocks take
+                                 from other bands where those are behind */
 } pmp_batch_config;
 
 /* Densify n <= PMP_MAX_BATCH keyframes of any sizes and view counts with one

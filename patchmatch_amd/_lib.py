@@ -483,7 +483,8 @@ class Context:
                                             _p(nghbr, _i32p)), "pmp_batch_get_maps")
         return plane, depth, score, nghbr
 
-    def batch_set_config(self, tile_rows=4, blocks_per_cu=0, use_graph=1, xcd_bands=1):
+    def batch_set_config(self, tile_rows=2, blocks_per_cu=0, use_graph=1, xcd_bands=1):
+        """tile_rows 2 with blocks_per_cu 0: the library's default, which chooses the launch shape."""
         c = BatchConfig(tile_rows, blocks_per_cu, use_graph, xcd_bands)
         self._chk(self.L.pmp_batch_set_config(self.h, ctypes.byref(c)), "pmp_batch_set_config")
 
