@@ -70,14 +70,15 @@ struct BatchHdr {
 // hipGraphs captured over this set's device pointers.
 using GraphKey = std::tuple<int, int, int, int, int, int>;   // passes, zero + 2 form, rows, blocks, bands, postprocess + 2 fused + 4 init_own
 constexpr int kHeadStride = 32;           // words: every head lies in a cache line of its own
-constexpr int kHeadWords = 24 * kHeadStride;
+constexpr int kFirstWords = 8 * kHeadStride;   // of a launch over one pass: its tickets
+constexpr int kHeadWords = 32 * kHeadStride;   // of a launch over several
 struct DescSet {
     int cap = 0;
     SlotDesc* h_slots = nullptr;
     BatchHdr* h_hdr = nullptr;
     SlotDesc* d_slots = nullptr;
     BatchHdr* d_hdr = nullptr;
-    unsigned int* d_heads = nullptr;     // kHeadWords per launch of a call
+    unsigned int* d_heads = nullptr;     // kFirstWords per launch of a call, or kHeadWords of its only one
     unsigned int* d_sync = nullptr;      // BatchHdr::sync
     size_t sync_cap = 0;                 // tiles
     hipEvent_t uploaded = nullptr;       // recorded after the last upload

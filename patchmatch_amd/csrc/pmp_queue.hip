@@ -228,14 +228,19 @@ __device__ __forceinline__ void epoch_leave(const SlotDesc& d, int tx, int ty, i
 // arrivals, the last arrival acquires the others' and releases all with the
 // ring entry, and the wave that takes the entry acquires them for its block.
 //
-// heads: three words per band, each in a cache line of its own.
+// heads: four words per band, each in a cache line of its own.  A block takes an
+// entry by a permit (ready, counted down) and then a ticket (ring): where most
+// blocks want the same band, each does two additions, while a compare-and-swap
+// of the ring's head let one of them through per 2.7 us (eight 960x480
+// keyframes, one view, in a single band: 157 ms, 15.4 now; 640x320, 2 views,
+// from a warped result: 2.89, 2.53 now).
 __device__ __forceinline__ unsigned int* head_of(unsigned int* heads, int kind, int band) {
     return heads + (kind * 8 + band) * kHeadStride;
 }
 // A block without work looks again after 64 x 64 cycles, then after up to
 // kMaxNaps times that: the looks share a few cache lines with the others' atomics.
 constexpr int kNap = 64, kMaxNaps = 4;
-enum { kHeadFirst = 0, kHeadRing = 1, kHeadTail = 2 };   // pass-0 tickets; ring entries taken, announced
+enum { kHeadFirst = 0, kHeadRing = 1, kHeadTail = 2, kHeadReady = 3 };   // pass-0 tickets; ring entries taken, announced, ready
 
 __device__ __forceinline__ int load_agent(const unsigned int* p) {
     return (int)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -261,18 +266,18 @@ __device__ __forceinline__ void take_tile(const BatchHdr PMP_CONST* hdr, int pas
     const int lo = band_lo(total, band, nb), n = band_lo(total, band + 1, nb) - lo;
     unsigned int* h0 = head_of(heads, kHeadFirst, band);
     unsigned int* hr = head_of(heads, kHeadRing, band);
-    unsigned int* ht = head_of(heads, kHeadTail, band);
+    unsigned int* ready = head_of(heads, kHeadReady, band);
     int item = -1, pass = 0, naps = 1;
     for (;;) {
-        int level = 0x7FFFFFFF, q = 0;   // the pass (about, in the ring) of the band's next tile
+        int level = 0x7FFFFFFF;          // the pass (about, in the ring) of the band's next tile
         bool left = false;
         if (lane < nb && n > 0) {
             if (load_agent(h0) < n) {
                 level = 0;
             } else if (passes > 1) {
-                q = load_agent(hr);
+                const int q = load_agent(hr);
                 left = q < n * (passes - 1);
-                if (q < load_agent(ht)) level = 1 + q / n;
+                if (load_agent(ready) > 0) level = 1 + q / n;
             }
         }
         int best = level;
@@ -292,12 +297,15 @@ __device__ __forceinline__ void take_tile(const BatchHdr PMP_CONST* hdr, int pas
                 got = h < n;
                 item = lo + h;
                 pass = 0;
-            } else if ((int)atomicCAS(hr, (unsigned int)q, (unsigned int)q + 1u) == q) {
+            } else if ((int)atomicSub(ready, 1u) > 0) {
+                const unsigned int q = atomicAdd(hr, 1u);
                 unsigned int v;
-                while ((v = atomicExch(&ring[lo + q % n], 0u)) == 0u) __builtin_amdgcn_s_sleep(1);
+                while ((v = atomicExch(&ring[lo + q % (unsigned int)n], 0u)) == 0u) __builtin_amdgcn_s_sleep(1);
                 got = true;
                 item = (int)(v & 0xFFFFFFu);
                 pass = (int)(v >> 24);
+            } else {
+                atomicAdd(ready, 1u);   // the last one went to another block
             }
             if (got) {
                 sh.item = item;
@@ -339,6 +347,7 @@ __device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, con
         empty = 0u;
         __builtin_amdgcn_s_sleep(1);
     }
+    atomicAdd(head_of(heads, kHeadReady, band), 1u);
 }
 
 // One launch over `passes` red-black passes of every slot, the first being
@@ -360,7 +369,7 @@ __global__ __launch_bounds__((kPropThreads<R, F>))
         if (threadIdx.x < 64) {
             take_tile(hdr, passes, heads, bands, sh);
             // the maps that the ring entry hands over (release_tiles), before the block reads any
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (passes > 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
         __syncthreads();
         const int item = sh.item, pass = sh.pass;
@@ -431,7 +440,7 @@ int desc_alloc(pmp_ctx* ctx, DescSet& d, int cap) {
     PMP_HIP(ctx, hipHostMalloc((void**)&d.h_hdr, sizeof(BatchHdr), hipHostMallocDefault));
     PMP_HIP(ctx, hipMalloc(&d.d_slots, cap * sizeof(SlotDesc)));
     PMP_HIP(ctx, hipMalloc(&d.d_hdr, sizeof(BatchHdr)));
-    PMP_HIP(ctx, hipMalloc(&d.d_heads, (size_t)kMaxPasses * kHeadWords * sizeof(unsigned int)));
+    PMP_HIP(ctx, hipMalloc(&d.d_heads, std::max(kMaxPasses * kFirstWords, kHeadWords) * sizeof(unsigned int)));
     PMP_HIP(ctx, hipEventCreateWithFlags(&d.uploaded, hipEventDisableTiming));
     return PMP_OK;
 }
@@ -685,7 +694,7 @@ int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int pass
     (void)sl;
     // a fill kernel, not memset nodes: the sequence may be captured
     const bool one = r.fused && passes > 1;
-    const int words = kHeadWords * (one ? 1 : std::max(passes, 1));
+    const int words = one ? kHeadWords : kFirstWords * std::max(passes, 1);
     hipLaunchKernelGGL(k_clear, dim3(one ? 64 : (words + 255) / 256), dim3(256), 0, s, hd, d.d_heads, words,
                        (unsigned int*)ctx->counters, one ? 1 : 0);
     PMP_HIP(ctx, hipGetLastError());
@@ -737,7 +746,7 @@ int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r) {
 // One launch over passes [first, first + passes), with the heads of launch `launch`.
 static int launch_prop(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int launch, int first, int passes) {
     PMP_QPTRS
-    unsigned int* heads = d.d_heads + (size_t)launch * kHeadWords;
+    unsigned int* heads = d.d_heads + (size_t)launch * kFirstWords;
     unsigned long long* counters = ctx->counters;
     int bands = r.bands;
     void* args[] = {(void*)&sl, (void*)&hd, &first, &passes, &heads, &counters, &bands};
