@@ -588,12 +588,16 @@ static bool is_default(const pmp_batch_config& c) {
 
 void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
                 bool single, QueueRun& r) {
-    // work: the pixels of one colour in units of 64; chip: waves at four to a SIMD
-    double work = 0.0;
+    // work: the pixels of one colour in units of 64; chip: waves at four to a
+    // SIMD; gain: what kLane wins over kQuad, per unit of work about 2 with one
+    // view, 1 with two, 0 with three and -3 with more
+    double work = 0.0, gain = 0.0;
     int views = 0;
     for (int k = 0; k < n; ++k) {
         const KfArgs& a = slots[slot ? slot[k] : k].a;
-        work += (double)a.W * a.H / 128.0;
+        const double w = (double)a.W * a.H / 128.0;
+        work += w;
+        gain += w * (a.N >= 4 ? -3.0 : 3.0 - a.N);
         views = std::max(views, (int)a.N);
     }
     const double chip = 16.0 * q.cus;
@@ -616,8 +620,14 @@ void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int
     const double lane_from = views == 1 ? 0.375 : 0.75, lane_to = views == 3 ? 2.5 : 1e30;
     if (views <= 3 && work > lane_from * chip && work < lane_to * chip)
         r.form = kLane;
+    else if (work < 1.75 * chip)
+        r.form = kWide;
     else
-        r.form = work < 1.75 * chip ? kWide : kQuad;
+        // - A launch over keyframes of several view counts takes what most of its
+        //   work is better with (eight of 960x480: seven with 1 view and one with
+        //   4 18.7 / 20.0, seven with 2 and one with 10 33.9 / 34.7, four with 2
+        //   and four with 4 33.5 / 32.2).
+        r.form = gain > 0.0 ? kLane : kQuad;
     // kQuad, 1440x720, 4 views: 12.4 ms with 8 rows, 14.0 with 4, 13.1 with 2;
     // with a launch per pass, whose last tiles leave compute units idle, 15.2
     // with 8, 14.1 with 4, 14.7 with 2.  kWide, 640x320, 4 views: 3.4 with 2,

@@ -2,6 +2,7 @@
 what a call that leaves the shape alone keeps."""
 import time
 
+import numpy as np
 import pytest
 
 from patchmatch_amd import synth
@@ -42,3 +43,29 @@ def test_one_band_keeps_pace():
             ms[bands] = min(ms.get(bands, 1e9), 1e3 * min(t))
             print(f"[config] xcd_bands {bands}: {min(t) * 1e3:.2f} ms", flush=True)
     assert ms[0] < 1.5 * ms[1], ms
+
+
+@pytest.mark.parametrize("views,rows", [((1,) * 7 + (4,), 4), ((4,) + (2,) * 7, 4), ((2,) * 4 + (4,) * 4, 8),
+                                        ((3,) * 7 + (4,), 8), ((1, 1, 3, 3, 3, 3, 3, 3), 4)])
+def test_mixed_view_counts(views, rows):
+    """A batch takes the form that most of its work is better with: tiles of 4
+    rows where one or two views dominate, of 8 otherwise."""
+    W, H = 420, 290
+    kf = synth.make_keyframe(6, W, H, 4, baseline=(0.05, 0.4), spheres=4)
+    p = config1_params(iterations=1)
+    with Context(0) as ctx:
+        ctx.image_put(1, kf.ref)
+        for v, img in enumerate(kf.views):
+            ctx.image_put(2 + v, img)
+        kfs = [Keyframe.make(1, kf.ref_pose, [2 + v for v in range(n)], kf.view_poses[:n]) for n in views]
+        ctx.debug_epochs(1)
+        ctx.batch_densify(p, kfs)
+        rep = ctx.debug_epoch_report()
+        got = [ctx.batch_get_maps(k, (H, W)) for k in range(len(kfs))]
+        ctx.debug_epochs(0)
+        assert rep["tiles"] == 8 * -(-((W + 1) // 2) // 32) * -(-H // (2 * rows)) and rep["violations"] == 0, rep
+        for k, n in enumerate(views):   # the same bits as alone
+            ctx.set_views(1, kf.ref_pose, [2 + v for v in range(n)], kf.view_poses[:n])
+            ctx.densify(p)
+            for a, b in zip(ctx.get_maps(2), got[k]):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (k, n)
