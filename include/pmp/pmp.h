@@ -544,6 +544,13 @@ int pmp_debug_epochs(pmp_ctx* ctx, int32_t mode);
 int pmp_debug_epoch_report(pmp_ctx* ctx, int32_t* tiles, int32_t* violations, int32_t* min_epoch,
                            int32_t* max_epoch);
 
+/* How the last call of the one-keyframe or batched form runs (or would run) its
+ * red-black passes: planes evaluated one per lane (form 0), by four lanes (1)
+ * or by four lanes with four times the waves to a tile (2), the tile rows, the
+ * persistent blocks, and whether several passes share one launch.  PMP_ESTATE
+ * before any such call. */
+int pmp_debug_launch(pmp_ctx* ctx, int32_t* form, int32_t* tile_rows, int32_t* blocks, int32_t* one_launch);
+
 /* roctx ranges around the main calls (pmp_densify and the other stages,
  * pmp_batch_*, pmp_clean, pmp_pruner_prune, pmp_preinit_*, pmp_image_put, and
  * the served form's uploads and steps), for rocprofv3 --marker-trace: host

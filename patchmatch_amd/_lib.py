@@ -45,7 +45,7 @@ EXPORTS = [
     "pmp_pruner_add_view", "pmp_pruner_prune", "pmp_pruner_pop_head", "pmp_pruner_reset",
     "pmp_pruner_size", "pmp_pruner_get_map", "pmp_debug_eval_math", "pmp_debug_refine_normals",
     "pmp_set_timing", "pmp_get_timing", "pmp_set_mask", "pmp_debug_copy", "pmp_debug_epochs",
-    "pmp_debug_epoch_report", "pmp_set_roctx",
+    "pmp_debug_epoch_report", "pmp_debug_launch", "pmp_set_roctx",
     "pmp_batch_densify", "pmp_batch_get_maps", "pmp_batch_set_config", "pmp_batch_get_config",
     "pmp_batch_autotune", "pmp_server_create", "pmp_server_destroy", "pmp_server_last_error",
     "pmp_server_submit", "pmp_server_wait", "pmp_server_fetch", "pmp_server_stats", "pmp_server_pause",
@@ -184,6 +184,7 @@ def load():
         "pmp_debug_epochs": ([_vp, i32], c_int),
         "pmp_set_roctx": ([i32], c_int),
         "pmp_debug_epoch_report": ([_vp, _i32p, _i32p, _i32p, _i32p], c_int),
+        "pmp_debug_launch": ([_vp, _i32p, _i32p, _i32p, _i32p], c_int),
         "pmp_batch_densify": ([_vp, P(Params), i32, P(Keyframe)], c_int),
         "pmp_batch_get_maps": ([_vp, i32, _f32p, _f32p, _f32p, _i32p], c_int),
         "pmp_batch_set_config": ([_vp, P(BatchConfig)], c_int),
@@ -593,6 +594,11 @@ class Context:
         v = [ctypes.c_int32(0) for _ in range(4)]
         self._chk(self.L.pmp_debug_epoch_report(self.h, *[ctypes.byref(x) for x in v]), "pmp_debug_epoch_report")
         return dict(zip(("tiles", "violations", "min_epoch", "max_epoch"), (x.value for x in v)))
+
+    def debug_launch(self) -> dict:
+        v = [ctypes.c_int32(0) for _ in range(4)]
+        self._chk(self.L.pmp_debug_launch(self.h, *[ctypes.byref(x) for x in v]), "pmp_debug_launch")
+        return dict(zip(("form", "tile_rows", "blocks", "one_launch"), (x.value for x in v)))
 
     def debug_copy(self, nbytes: int, repeats: int = 1):
         self._chk(self.L.pmp_debug_copy(self.h, nbytes, repeats), "pmp_debug_copy")

@@ -6,6 +6,7 @@
 
 #include "pmp_internal.h"
 #include "pmp_math.h"
+#include "pmp_queue.h"
 #include "pmp_score.h"
 
 namespace pmp {
@@ -130,6 +131,17 @@ int pmp_debug_epoch_report(pmp_ctx* ctx, int32_t* tiles, int32_t* violations, in
     *violations = (int32_t)bad;
     *min_epoch = (int32_t)lo;
     *max_epoch = (int32_t)hi;
+    return PMP_OK;
+}
+
+int pmp_debug_launch(pmp_ctx* ctx, int32_t* form, int32_t* tile_rows, int32_t* blocks, int32_t* one_launch) {
+    if (!ctx || !form || !tile_rows || !blocks || !one_launch) return PMP_EINVAL;
+    if (!ctx->queue || ctx->queue->last.blocks == 0) return set_error(ctx, PMP_ESTATE, "no kernel has been launched");
+    const QueueRun& r = ctx->queue->last;
+    *form = r.form;
+    *tile_rows = r.rows;
+    *blocks = r.blocks;
+    *one_launch = r.fused ? 1 : 0;
     return PMP_OK;
 }
 

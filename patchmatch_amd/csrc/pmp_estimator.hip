@@ -151,6 +151,7 @@ int plain_prepare(pmp_ctx* ctx, const pmp_params* p, const uint8_t* dmask, bool 
     if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0,
                         *q->plain.h_hdr, r)))
         return rc;
+    q->last = r;
     if (p->iterations > kMaxPasses / 2) return set_error(ctx, PMP_EINVAL, "iterations must be <= 64");
     return desc_upload(ctx, q->plain, 1, ctx->stream);
 }

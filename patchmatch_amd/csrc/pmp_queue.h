@@ -111,6 +111,7 @@ struct QueueState {
     DescSet batch;            // pmp_batch_*
     std::vector<SlotBuf> bufs;
     int n_last = 0;
+    QueueRun last;            // of the last call
 };
 
 int queue_state(pmp_ctx* ctx, QueueState*& out);

@@ -663,7 +663,16 @@ int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool
     // tiles are in flight at once and wait for each other tile by tile, while
     // the launches' own barrier leaves the last ones whole compute units
     // (480x240, 4 views, 4 iterations: 4.4 against 2.4 ms).
-    r.fused = 2 * tiles >= 3 * q.cus * bpc;
+    // With many tiles to each block the idle end of a pass is a small part of
+    // it, while the tiles of a pass come in the order in which the pass before
+    // completed them, farther apart in the images the longer the passes are.
+    // kLane, 4 iterations: 2400x1200, 1 view (7 tiles to a block) 12.1 / 12.2,
+    // eight of 960x480 (9) 15.1 / 15.2, 2880x1440 (11) 17.3 / 17.0, 4600x2300
+    // (27) 48.4 / 43.0.  kQuad: three of 2880x1440, 10 views (24), 3 iterations
+    // 325 / 329, eight of 1920x960, 4 views (28), 4 iterations 167 / 169,
+    // 5760x2880 (32), 3 iterations 200 / 193, eight of 2880x1440 (63) 335 / 328.
+    const int in_flight = q.cus * bpc;
+    r.fused = 2 * tiles >= 3 * in_flight && tiles <= (r.form == kLane ? 10 : 30) * in_flight;
     // a block of 16 waves fits on a CU once, of 8 twice: while every tile has
     // one, its planes are scored in one or two rounds instead of four (init of
     // 320x160, 8 views: 72 us, 108 with four; of 480x240: 114 and 123); beyond,
@@ -924,6 +933,7 @@ int pmp_batch_densify(pmp_ctx* ctx, const pmp_params* params, int32_t n, const p
     if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0,
                         *q->batch.h_hdr, r)))
         return rc;
+    q->last = r;
     if ((rc = q_densify(ctx, ctx->stream, q->batch, r, 2 * params->iterations, q->cfg.use_graph != 0))) return rc;
     q->n_last = n;
     ctx->densify_calls += n;

@@ -69,3 +69,29 @@ def test_mixed_view_counts(views, rows):
             ctx.densify(p)
             for a, b in zip(ctx.get_maps(2), got[k]):
                 assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (k, n)
+
+
+# (W, H, views, keyframes, tile_rows, blocks_per_cu): whether the passes of a call share a launch on 256 CUs
+@pytest.mark.parametrize("W,H,n,count,rows,bpc,one", [
+    (203, 97, 1, 1, 4, 3, 0), (640, 320, 2, 1, 2, 1, 1), (640, 320, 2, 1, 2, 2, 1), (701, 187, 3, 1, 2, 1, 1),
+    (960, 480, 1, 8, 2, 0, 1), (960, 480, 1, 9, 2, 0, 0),      # 9.4 and 10.5 tiles to a block
+    (960, 480, 4, 34, 2, 0, 1), (960, 480, 4, 35, 2, 0, 0),    # 29.9 and 30.8
+])
+def test_passes_share_a_launch(W, H, n, count, rows, bpc, one):
+    kf = synth.make_keyframe(7, W, H, 4, baseline=(0.05, 0.4), spheres=4)
+    p = config1_params(iterations=2)
+    with Context(0) as ctx:
+        ctx.image_put(1, kf.ref)
+        for v, img in enumerate(kf.views):
+            ctx.image_put(2 + v, img)
+        k = Keyframe.make(1, kf.ref_pose, [2 + v for v in range(n)], kf.view_poses[:n])
+        ctx.batch_set_config(tile_rows=rows, blocks_per_cu=bpc)
+        ctx.batch_densify(p, [k] * count)
+        shape = ctx.debug_launch()
+        got = [ctx.batch_get_maps(k, (H, W)) for k in {0, count // 2, count - 1}]
+        assert shape["one_launch"] == one, shape
+        ctx.set_views(1, kf.ref_pose, [2 + v for v in range(n)], kf.view_poses[:n])
+        ctx.densify(p)
+        want = ctx.get_maps(2)
+        for g in got:
+            assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(g, want))
