@@ -292,6 +292,7 @@ class Context:
             raise PmpError(f"pmp_create(device={device}) failed: {STATUS.get(rc, rc)} (is a GPU visible?)")
         self.h = h
         self.W = self.H = 0
+        self._batch_shapes = []
 
     def close(self):
         if getattr(self, "h", None):
@@ -473,13 +474,16 @@ class Context:
     def batch_densify(self, p: Params, kfs):
         arr = (Keyframe * len(kfs))(*kfs)
         self._chk(self.L.pmp_batch_densify(self.h, ctypes.byref(p), len(kfs), arr), "pmp_batch_densify")
+        self._batch_shapes = [self.image_size(kf.ref_id) for kf in kfs]
 
     def batch_get_maps(self, k: int, shape):
         H, W = shape
-        plane = np.empty((H, W, 4), np.float32)
-        depth = np.empty((H, W), np.float32)
-        score = np.empty((H, W), np.float32)
-        nghbr = np.empty((H, W), np.int32)
+        # in another shape than the keyframe's, what it does not fill is 0
+        new = np.empty if (H, W) in self._batch_shapes[k:k + 1] else np.zeros
+        plane = new((H, W, 4), np.float32)
+        depth = new((H, W), np.float32)
+        score = new((H, W), np.float32)
+        nghbr = new((H, W), np.int32)
         self._chk(self.L.pmp_batch_get_maps(self.h, k, _p(plane, _f32p), _p(depth, _f32p), _p(score, _f32p),
                                             _p(nghbr, _i32p)), "pmp_batch_get_maps")
         return plane, depth, score, nghbr
@@ -569,7 +573,7 @@ class Context:
         return self.L.pmp_pruner_size(self.h)
 
     def pruner_get_map(self, index, shape):
-        out = np.empty(shape, np.float32)
+        out = np.zeros(shape, np.float32)   # the caller's shape: what the map does not fill is 0
         self._chk(self.L.pmp_pruner_get_map(self.h, index, _p(out, _f32p)), "pmp_pruner_get_map")
         return out
 
