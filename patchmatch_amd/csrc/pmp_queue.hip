@@ -1002,9 +1002,10 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
         if ((rc = batch_prepare(ctx, q, params, n, kfs, c, r, false))) break;
         if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, r))) break;
         const int occ = r.blocks / (q->cus > 0 ? q->cus : 1);   // blocks per CU that fit (rounding aside)
-        // at least 8 waves per CU (rows waves per block): fewer leave SIMDs
-        // idle and measured 1.3-4x slower, and their trials are the longest
-        const int bpc_min = std::min(occ, (8 + rows_set[ri] - 1) / rows_set[ri]);
+        // at least 8 waves per CU: fewer leave SIMDs idle and measured 1.3-4x
+        // slower, and their trials are the longest
+        const int waves = prop_kernel(zero, r.form, r.rows).threads / 64;   // of a block
+        const int bpc_min = std::min(occ, (8 + waves - 1) / waves);
         for (int bpc = bpc_min; bpc <= occ && rc == 0; ++bpc) {
             for (int bands = 0; bands <= 1 && rc == 0; ++bands) {
                 c.blocks_per_cu = bpc;
