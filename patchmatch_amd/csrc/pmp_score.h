@@ -133,13 +133,6 @@ PMP_DF float blend(const Pend<kZero>& p) {
     return val;
 }
 
-template <bool kZero>
-PMP_DF float sample(const KfArgs& a, const uint32_t* __restrict__ base, float u, float v) {
-    Pend<kZero> p;
-    gather<kZero>(a, base, u, v, p);
-    return blend<kZero>(p) * kTexelScale;
-}
-
 // Equirectangular projection (PatchMatchCuda.cu:132-144): the latitude
 // asin(y / |X|) there is the same angle as atan2(y, sqrt(x^2 + z^2)) here.
 // hu, hv are a.hu, a.hv (callers may pass copies held in vector registers).
