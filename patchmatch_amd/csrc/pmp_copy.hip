@@ -29,8 +29,10 @@ static constexpr int kTasks = 256;       // a power of two above kSlots * kChunk
 static constexpr int kThreads = 8, kRings = 4, kAllRings = 64;
 // Transfers below these are copied by the caller alone, in one chunk: waking
 // the threads costs more (normals of 328x182, 716 KB down: 66 us alone, 52
-// with them; a 614 KB image up: 75 and 76).
-static constexpr size_t kAloneDown = size_t(512) << 10, kAloneUp = size_t(768) << 10;
+// with them; a 614 KB image up: 75 and 76).  Three copies and more, each of
+// which is a chunk, are worth it later (the three maps of 240x120, 691 KB: 60
+// us alone, 74 with them, of 300x150 77 and 73).
+static constexpr size_t kAloneDown = size_t(512) << 10, kAloneDownMaps = size_t(1) << 20, kAloneUp = size_t(768) << 10;
 // Uploads of contiguous rows from kAloneUp to these are the runtime's own, on
 // the caller's thread: several copies in a call (five 640x320 maps to the
 // cleaner and back: 222 us, with the threads 290; of 800x400: 342 and 345; of
@@ -428,7 +430,7 @@ hipError_t Copier::to_host(hipStream_t s, const HostCopy* c, int n, bool fresh) 
     const Lent lent(pool, s);
     if (!lent.r) return plain(s, c, n, hipMemcpyDeviceToHost, true);
     Ring& r = *lent.r;
-    if (bytes < kAloneDown) return small(r, s, c, n, true);
+    if (bytes < (n > 2 ? kAloneDownMaps : kAloneDown)) return small(r, s, c, n, true);
     const bool alone = !pool->start_threads(bytes);
     Walk w{c, n};
     uint64_t issued = 0, copied = 0;

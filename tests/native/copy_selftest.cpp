@@ -196,12 +196,31 @@ static void streams() {
     CHECK(dx == x);
 }
 
+// Small downloads of several maps are the caller's alone, larger ones the
+// threads' too; whole either way.
+static void maps() {
+    hip_sim::Stream s;
+    Copier c;
+    size_t all0, all, deaf;
+    threads(&all0, &deaf);
+    for (size_t px : {size_t(240 * 120), size_t(640 * 320)}) {
+        const Bytes plane = noise(16 * px, 1), depth = noise(4 * px, 2), score = noise(4 * px, 3);
+        Bytes p(16 * px), d(4 * px), sc(4 * px);
+        const HostCopy down[3] = {flat_copy(p.data(), plane.data(), 16 * px), flat_copy(d.data(), depth.data(), 4 * px),
+                                  flat_copy(sc.data(), score.data(), 4 * px)};
+        CHECK(c.to_host(&s, down, 3) == hipSuccess);
+        CHECK(p == plane && d == depth && sc == score);
+        threads(&all, &deaf);
+        CHECK((all > all0) == (24 * px > 1 * MiB));
+    }
+}
+
 int main(int argc, char** argv) {
     std::set<std::string> want(argv + 1, argv + argc);
     struct {
         const char* name;
         void (*f)();
-    } parts[] = {{"pitched", pitched}, {"until", until}, {"shared", shared}, {"streams", streams}};
+    } parts[] = {{"pitched", pitched}, {"until", until}, {"shared", shared}, {"streams", streams}, {"maps", maps}};
     for (auto& p : parts)
         if (want.empty() || want.count(p.name)) {
             p.f();
