@@ -149,7 +149,7 @@ int plain_prepare(pmp_ctx* ctx, const pmp_params* p, const uint8_t* dmask, bool 
     if ((rc = ensure_sync(ctx, q->plain, (size_t)tiles))) return rc;
     if (propagates && (rc = epochs_arm(ctx, ctx->stream, 1, &q->plain.h_slots[0], &tiles, pass0))) return rc;
     if ((rc = queue_run(ctx, *q, q->cfg, p->edge_mode == PMP_EDGE_ZERO, p->postprocess != 0,
-                        *q->plain.h_hdr, r)))
+                        *q->plain.h_hdr, q->plain.h_slots, r)))
         return rc;
     q->last = r;
     if (p->iterations > kMaxPasses / 2) return set_error(ctx, PMP_EINVAL, "iterations must be <= 64");

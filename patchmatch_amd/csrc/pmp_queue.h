@@ -95,7 +95,7 @@ struct QueueRun {
     int blocks = 0;           // persistent grid
     int bands = 1;            // per-XCD bands
     bool fused = false;       // all passes of a call in one launch
-    int init_own = 64;        // an init wave's pixels
+    int init_own = 64;        // an init wave's pixels (0: 64, a plane per lane)
 };
 
 // Default launch shape: the tile rows follow the form that the size and the
@@ -144,9 +144,9 @@ int slot_tiles(SlotDesc& d, int rows);
 void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int* slot, const SlotDesc* slots,
                 bool single, QueueRun& r);
 void fill_list(WorkList& L, int n, const int* items);
-// The rest of a shaped run over the work lists of h.
+// The rest of a shaped run over the work lists of h, whose slots are in slots.
 int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, const BatchHdr& h,
-              QueueRun& r);
+              const SlotDesc* slots, QueueRun& r);
 int q_clear(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r, int passes);
 int q_init(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);
 int q_score(pmp_ctx* ctx, hipStream_t s, DescSet& d, const QueueRun& r);

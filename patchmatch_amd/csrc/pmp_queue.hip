@@ -59,16 +59,21 @@ __global__ void k_fill_u32(unsigned int* __restrict__ p, int n, unsigned int v) 
 // reads never wait behind the neighbour gathers issued before them.  The planes
 // are random, so each pixel's patches lie elsewhere and the gathers' cache
 // lines bound the kernel; by quads of lanes (score_wave) a 1920x960 keyframe
-// with 6 views takes 1.05 ms, with a plane per lane 1.32.
+// with 6 views takes 1.05 ms, with a plane per lane 1.25.  With one view only
+// a quarter of a quad's lanes have one to accumulate, and a plane per lane is
+// the faster form (queue_run).
 constexpr int kInitRows = 4;
 constexpr int kInitStageRows = kInitRows + 2 * kMaxHalf;
 // A wave owns kOwn pixels of the tile: 64, or 32 or 16 where the launch would
 // leave the chip idle (queue_run), which takes fewer rounds of score_wave.
+// kOwn 0: 64 pixels, a plane per lane.
 template <int kOwn>
 struct InitShared {
-    static constexpr int kWaves = 64 * kInitRows / kOwn;
-    QuadTap walk[kQuadTaps];
-    QuadShared quad[kWaves];
+    static constexpr bool kLanes = kOwn == 0;
+    static constexpr int kPix = kLanes ? 64 : kOwn;     // a wave's pixels
+    static constexpr int kWaves = 64 * kInitRows / kPix;
+    QuadTap walk[kLanes ? 1 : kQuadTaps];
+    std::conditional_t<kLanes, LaneShared, QuadShared> eval[kWaves];
     float4 rs[64 * kInitRows];
     float4 plane[64 * kInitRows];
     float score[64 * kInitRows];
@@ -108,8 +113,9 @@ __global__ __launch_bounds__(64 * InitShared<kOwn>::kWaves) void k_init_q(const 
     const WorkList PMP_CONST* L = &hdr->init;
     const int total = L->total;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    const bool owner = kOwn == 64 || lane < kOwn;   // lanes beyond own no pixel but take part in the evaluations
-    const int t = kOwn * wave + (owner ? lane : 0);
+    constexpr int PW = InitShared<kOwn>::kPix;
+    const bool owner = PW == 64 || lane < PW;   // lanes beyond own no pixel but take part in the evaluations
+    const int t = PW * wave + (owner ? lane : 0);
     int cur = -1;
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         int local;
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(64 * InitShared<kOwn>::kWaves) void k_init_q(const 
         if (s != cur) {
             __syncthreads();
             load_wc(a.Wc, st.sWc);
-            load_walk(a, st.walk);
+            if constexpr (kOwn != 0) load_walk(a, st.walk);
             cur = s;
         }
         const int tx = local % d.nbx_init, ty = local / d.nbx_init;
@@ -151,12 +157,15 @@ __global__ __launch_bounds__(64 * InitShared<kOwn>::kWaves) void k_init_q(const 
             col = (p & 63) + a.half;
         };
         auto job = [&](int l, int& jt, float& px, float& py, float& pz) {
-            jt = kOwn * wave + l;
+            jt = PW * wave + l;
             const float4 p = st.plane[jt];
             px = p.x; py = p.y; pz = p.z;
         };
-        auto put = [&](int l, float v) { st.score[kOwn * wave + l] = v; };
-        score_wave<kZero>(a, tp, st.walk, st.sWc, st.rs, st.ic, at, job, put, __ballot(scored), st.quad[wave]);
+        auto put = [&](int l, float v) { st.score[PW * wave + l] = v; };
+        if constexpr (kOwn == 0)
+            score_lanes<kZero>(a, tp, st.sWc, st.rs, st.ic, at, job, put, __ballot(scored), &st.eval[wave].sv[0][0]);
+        else
+            score_wave<kZero>(a, tp, st.walk, st.sWc, st.rs, st.ic, at, job, put, __ballot(scored), st.eval[wave]);
         const float sc = scored ? st.score[t] : __uint_as_float(0xFFFFFFFFu);   // cudaMemset(score, 0xFF) (depthmap.cc:657)
         if constexpr (kScore) {
             if (scored) d.score[k] = sc;
@@ -646,7 +655,7 @@ static int check_config(pmp_ctx* ctx, const pmp_batch_config& c) {
 // Persistent grid: the configured blocks per CU, capped by (and defaulting
 // to) what fits on a CU at once; a multiple of 8 with per-XCD bands.
 int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool zero, bool post, const BatchHdr& h,
-              QueueRun& r) {
+              const SlotDesc* slots, QueueRun& r) {
     const int tiles = h.prop.total;
     int occ = 0;
     const PropKernel kern = prop_kernel(zero, r.form, r.rows);
@@ -677,8 +686,20 @@ int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool
     // one, its planes are scored in one or two rounds instead of four (init of
     // 320x160, 8 views: 72 us, 108 with four; of 480x240: 114 and 123); beyond,
     // the small blocks fill the chip better (640x320, 2 views: 82 us, 107 with
-    // 16 waves)
-    r.init_own = h.init.total <= q.cus ? 16 : h.init.total <= 2 * q.cus ? 32 : 64;
+    // 16 waves).
+    // There, a plane per lane with one view (us against quads: 640x320 58 / 66,
+    // 1920x960 271 / 285, 3840x1920 1069 / 1061), with two or three up to six
+    // tiles to a CU (800x400: 95 / 98 and 110 / 112; 960x480: 124 / 127 and 152
+    // / 144), and with any but four up to four (640x320: 5 views 127 / 136, 4
+    // views 117 / 115, 10 views 229 / 231; 720x360: 10 views 287 / 276).
+    int views = 0;
+    for (int k = 0; k < h.init.n; ++k) views = std::max(views, (int)slots[h.init.slot[k]].a.N);
+    r.init_own = h.init.total <= q.cus       ? 16
+                 : h.init.total <= 2 * q.cus ? 32
+                 : views == 1 || (views <= 3 && h.init.total <= 6 * q.cus) ||
+                         (views != 4 && h.init.total <= 4 * q.cus)
+                     ? 0
+                     : 64;
     r.zero = zero;
     r.post = post;
     r.bands = c.xcd_bands ? 1 : 0;
@@ -747,6 +768,7 @@ static int launch_init(pmp_ctx* ctx, hipStream_t s, const SlotDesc PMP_CONST* sl
     const unsigned n = (unsigned)grid_blocks(ctx);
     if (r.init_own == 16) launch_init_own<kScore, 16>(s, dim3(n / 8), sl, hd, r.zero);
     else if (r.init_own == 32) launch_init_own<kScore, 32>(s, dim3(n / 4), sl, hd, r.zero);
+    else if (r.init_own == 0) launch_init_own<kScore, 0>(s, dim3(n), sl, hd, r.zero);
     else launch_init_own<kScore, 64>(s, dim3(n), sl, hd, r.zero);
     PMP_HIP(ctx, hipGetLastError());
     return PMP_OK;
@@ -931,7 +953,7 @@ int pmp_batch_densify(pmp_ctx* ctx, const pmp_params* params, int32_t n, const p
     QueueRun r;
     if ((rc = batch_prepare(ctx, q, params, n, kfs, q->cfg, r, true))) return rc;
     if ((rc = queue_run(ctx, *q, q->cfg, params->edge_mode == PMP_EDGE_ZERO, params->postprocess != 0,
-                        *q->batch.h_hdr, r)))
+                        *q->batch.h_hdr, q->batch.h_slots, r)))
         return rc;
     q->last = r;
     if ((rc = q_densify(ctx, ctx->stream, q->batch, r, 2 * params->iterations, q->cfg.use_graph != 0))) return rc;
@@ -1000,7 +1022,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
         c.blocks_per_cu = 32;
         QueueRun r;
         if ((rc = batch_prepare(ctx, q, params, n, kfs, c, r, false))) break;
-        if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, r))) break;
+        if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, q->batch.h_slots, r))) break;
         const int occ = r.blocks / (q->cus > 0 ? q->cus : 1);   // blocks per CU that fit (rounding aside)
         // at least 8 waves per CU: fewer leave SIMDs idle and measured 1.3-4x
         // slower, and their trials are the longest
@@ -1010,7 +1032,7 @@ int pmp_batch_autotune(pmp_ctx* ctx, const pmp_params* params, int32_t n, const 
             for (int bands = 0; bands <= 1 && rc == 0; ++bands) {
                 c.blocks_per_cu = bpc;
                 c.xcd_bands = bands;
-                if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, r))) break;
+                if ((rc = queue_run(ctx, *q, c, zero, false, *q->batch.h_hdr, q->batch.h_slots, r))) break;
                 // same starting maps for every candidate: init, then time every
                 // pass.  The first passes score random planes (most candidates
                 // survive pre-rejection, the gathers scatter); the converged

@@ -202,7 +202,7 @@ class GpuExec final : public sched::Executor {
         fill_list(d.h_hdr->init, n, items_init);
         fill_list(d.h_hdr->prop, n, items_prop);
         fill_list(d.h_hdr->rows, n, items_rows);
-        rc = queue_run(ctx, *ctx->queue, cfg, edge_mode == PMP_EDGE_ZERO, post, *d.h_hdr, run);
+        rc = queue_run(ctx, *ctx->queue, cfg, edge_mode == PMP_EDGE_ZERO, post, *d.h_hdr, d.h_slots, run);
         if (!rc) rc = desc_upload(ctx, d, n, ctx->stream);
         if (!rc) rc = q_clear(ctx, ctx->stream, d, run, 1);
         if (!rc && d.h_hdr->init.n) rc = q_init(ctx, ctx->stream, d, run);

@@ -5,8 +5,9 @@ import time
 import numpy as np
 import pytest
 
+from oracle import or_py
 from patchmatch_amd import synth
-from patchmatch_amd._lib import Context, Keyframe
+from patchmatch_amd._lib import PMP_MAPS_INIT, PMP_MAPS_WORK, Context, Keyframe
 from patchmatch_amd.params import config1_params
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,29 @@ def test_passes_share_a_launch(W, H, n, count, rows, bpc, one):
         want = ctx.get_maps(2)
         for g in got:
             assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(g, want))
+
+
+# lanes and quads on both sides of the lines between them (on 256 CUs), sizes that do not fill their tiles
+@pytest.mark.parametrize("W,H,n,edge", [(601, 303, 1, 0), (601, 303, 2, 2), (601, 303, 5, 1), (601, 303, 4, 0),
+                                        (801, 410, 3, 2), (801, 410, 5, 0), (961, 470, 2, 0), (961, 470, 1, 2)])
+def test_initial_scores(W, H, n, edge):
+    """Initial planes and scores by the form that the launch takes, against the oracle bit for bit."""
+    kf = synth.make_keyframe(8, W, H, n, baseline=(0.05, 0.4), spheres=4)
+    p = config1_params(iterations=0, seed=4, topk=min(n, 2), edge_mode=edge)
+    want = or_py.densify(or_py.Keyframe.from_synth(kf), p, None)
+    with Context(0) as ctx:
+        ctx.load_keyframe(kf.ref, kf.views, kf.ref_pose, kf.view_poses)
+        ctx.densify(p)
+        got = ctx.get_maps(2)
+        for name, g, o in (("plane", got[0][..., :3], want["plane"]), ("depth", got[1], want["depth"]),
+                           ("score", got[2], want["score"])):
+            eq = np.ascontiguousarray(g).view(np.uint32) == np.ascontiguousarray(o).view(np.uint32)
+            assert eq.all(), f"{name}: {np.count_nonzero(~eq)} of {eq.size} differ"
+        # the score call takes the same form
+        ctx.random_initialization(p)
+        plane, depth, score = ctx.get_maps(PMP_MAPS_INIT)
+        ctx.set_maps(plane, depth, np.full_like(score, 7.0))
+        ctx.score_plane_depth(p)
+        again = ctx.get_maps(PMP_MAPS_WORK)[2]
+        scored = again != 7.0
+        assert scored.any() and np.array_equal(again[scored].view(np.uint32), score[scored].view(np.uint32))
