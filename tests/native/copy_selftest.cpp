@@ -215,12 +215,62 @@ static void maps() {
     }
 }
 
+// Several threads on one context: host copies with more pieces than the ring
+// has tasks, uploads and downloads of every path beside them, lists that mix
+// pinned and pageable memory, downloads to fresh memory on both sides of their
+// line.
+static void together() {
+    Copier c;
+    std::vector<std::thread> ts;
+    for (int k = 0; k < 2; ++k)
+        ts.emplace_back([&, k] {
+            const Bytes src = noise(70 * MiB + 12345, (unsigned)k);   // 281 pieces of 256 tasks
+            for (int r = 0; r < 2; ++r) {
+                Bytes dst(src.size());
+                c.copy(dst.data(), src.data(), src.size());
+                CHECK(dst == src);
+                for (size_t n : {1 * KiB, 700 * KiB, 900 * KiB}) {
+                    Bytes d(n);
+                    c.copy(d.data(), src.data(), n);
+                    CHECK(memcmp(d.data(), src.data(), n) == 0);
+                }
+            }
+        });
+    for (int k = 0; k < 2; ++k)
+        ts.emplace_back([&] {
+            hip_sim::Stream s;
+            for (size_t n : {40 * KiB, 1 * MiB, 5 * MiB, 11 * MiB, 13 * MiB, 21 * MiB}) {
+                const Bytes src = noise(n, (unsigned)n);
+                Bytes dev(n), back(n);
+                const HostCopy up = flat_copy(src.data(), dev.data(), n), down = flat_copy(back.data(), dev.data(), n);
+                CHECK(c.to_device(&s, &up, 1) == hipSuccess && dev == src);
+                CHECK(c.to_host(&s, &down, 1, true) == hipSuccess && back == src);
+            }
+        });
+    ts.emplace_back([&] {
+        hip_sim::Stream s;
+        for (size_t n : {300 * KiB, 7 * MiB}) {
+            void* pin = nullptr;
+            CHECK(hipHostMalloc(&pin, n, hipHostMallocDefault) == hipSuccess);
+            const Bytes a = noise(n, 3), b = noise(n, 4);
+            memcpy(pin, b.data(), n);
+            Bytes da(n), db(n), ra(n);
+            const HostCopy up[2] = {flat_copy(a.data(), da.data(), n), flat_copy(pin, db.data(), n)};
+            CHECK(c.to_device(&s, up, 2) == hipSuccess && da == a && db == b);
+            const HostCopy down[2] = {flat_copy(ra.data(), db.data(), n), flat_copy(pin, da.data(), n)};
+            CHECK(c.to_host(&s, down, 2) == hipSuccess && ra == b && memcmp(pin, a.data(), n) == 0);
+            hipHostFree(pin);
+        }
+    });
+    for (auto& t : ts) t.join();
+}
+
 int main(int argc, char** argv) {
     std::set<std::string> want(argv + 1, argv + argc);
     struct {
         const char* name;
         void (*f)();
-    } parts[] = {{"pitched", pitched}, {"until", until}, {"shared", shared}, {"streams", streams}, {"maps", maps}};
+    } parts[] = {{"pitched", pitched}, {"until", until}, {"shared", shared}, {"streams", streams}, {"maps", maps}, {"together", together}};
     for (auto& p : parts)
         if (want.empty() || want.count(p.name)) {
             p.f();

@@ -13,7 +13,7 @@ ENV = dict(os.environ, ASAN_OPTIONS="detect_leaks=1", UBSAN_OPTIONS="halt_on_err
 
 
 @pytest.mark.parametrize("san", ["asan", "tsan"])
-@pytest.mark.parametrize("part", ["pitched", "until", "shared", "streams", "maps"])
+@pytest.mark.parametrize("part", ["pitched", "until", "shared", "streams", "maps", "together"])
 def test_copies(san, part):
     r = subprocess.run(["make", "-s", "-C", NATIVE, f"build/copy_selftest_{san}"], capture_output=True, text=True,
                        timeout=300)

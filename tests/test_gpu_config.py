@@ -122,3 +122,29 @@ def test_initial_scores(W, H, n, edge):
         again = ctx.get_maps(PMP_MAPS_WORK)[2]
         scored = again != 7.0
         assert scored.any() and np.array_equal(again[scored].view(np.uint32), score[scored].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [5, 6, 10])   # groups of 3 + 2, 3 + 3 and 4 + 3 + 3 views
+def test_several_groups_in_one_launch(n):
+    """Quads with more than one group of views, all passes in one launch: the
+    oracle's maps for every keyframe of the batch, bit for bit."""
+    W, H = 403, 291
+    kf = synth.make_keyframe(9, W, H, n, baseline=(0.05, 0.4), spheres=4)
+    p = config1_params(iterations=2, seed=n)
+    want = or_py.densify(or_py.Keyframe.from_synth(kf), p, kf.mask)
+    with Context(0) as ctx:
+        ctx.image_put(1, kf.ref)
+        ctx.image_put(90, kf.mask)
+        for v, img in enumerate(kf.views):
+            ctx.image_put(2 + v, img)
+        k = Keyframe.make(1, kf.ref_pose, [2 + v for v in range(n)], kf.view_poses, mask_id=90)
+        for _ in range(2):   # the graph's first launch and a replay
+            ctx.batch_densify(p, [k] * 9)
+            shape = ctx.debug_launch()
+            assert (shape["form"], shape["tile_rows"], shape["one_launch"]) == (1, 8, 1), shape
+            for i in range(9):
+                got = ctx.batch_get_maps(i, (H, W))
+                for name, g, o in (("plane", got[0][..., :3], want["plane"]), ("depth", got[1], want["depth"]),
+                                   ("score", got[2], want["score"])):
+                    eq = np.ascontiguousarray(g).view(np.uint32) == np.ascontiguousarray(o).view(np.uint32)
+                    assert eq.all(), f"keyframe {i} {name}: {np.count_nonzero(~eq)} of {eq.size} differ"
