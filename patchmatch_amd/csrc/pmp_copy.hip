@@ -496,9 +496,12 @@ hipError_t Copier::to_device(hipStream_t s, const HostCopy* c, int n, Until unti
         Ring::Slot& sl = r.slot[sent % kSlots];
         r.wait(sl.begin, sl.end);
         e = hipMemcpyAsync((uint8_t*)sl.p.c.dev + sl.p.off, sl.p.lin, sl.p.len, hipMemcpyHostToDevice, s);
+        ++sent;
+        // where the transfer ends with a wait for the stream, without an event
+        // for the chunks that no other follows in their slots (see to_host)
+        if (until == Until::kDone && w.end()) continue;
         if (e == hipSuccess) e = hipEventRecord(sl.ev, s);
         if (e == hipSuccess) sl.dma = true;
-        ++sent;
     }
     for (const Ring::Slot& sl : r.slot) r.wait(sl.begin, sl.end);   // no thread reads the caller's memory any more
     if (e == hipSuccess && until != Until::kDone) return e;
