@@ -104,7 +104,14 @@ typedef struct pmp_pose {
  * (depthmap.cc:522,557-558,652-656,771-800): buffers live in the context and
  * grow on demand.  device: HIP device ordinal.  Every call on a context (and
  * on a server) runs on that device from any thread and leaves the calling
- * thread's current HIP device as it found it. */
+ * thread's current HIP device as it found it.
+ * Copies of 512 KiB and more between host memory that is not pinned and the
+ * GPU are shared with at most eight threads of the library, started as
+ * transfers need them, on the CPUs that the calling thread may use, with all
+ * signals blocked.  They and the copies' pinned memory (8 MiB, at most four
+ * times per GPU) serve every context and server of the process, spin for some
+ * 100 us after a piece of work before they sleep, and end with the last of
+ * them. */
 int pmp_create(pmp_ctx** out, int32_t device);
 void pmp_destroy(pmp_ctx* ctx);
 /* Replaces printing cudaGetErrorString and continuing (PatchMatchCuda.cu:447-451). */
@@ -120,9 +127,8 @@ int pmp_synchronize(pmp_ctx* ctx);
  * Replaces InitTextureImages (PatchMatchCuda.cu:697-797, float textures built
  * from depthmap.cc:569-571); images stay resident as uint8 plus a packed
  * 2x2-neighbourhood copy for bilinear sampling.  on_device != 0: pixels is a
- * device pointer on the context's device.  Host rows (pitch bytes apart) go
- * through a pinned staging buffer of the context in one copy; the call
- * returns once the image is on the device. */
+ * device pointer on the context's device.  Host rows may lie pitch bytes
+ * apart.  The call returns once the image is on the device. */
 int pmp_image_put(pmp_ctx* ctx, uint64_t id, const uint8_t* pixels, int32_t width, int32_t height,
                   int64_t pitch, int32_t on_device);
 int pmp_image_drop(pmp_ctx* ctx, uint64_t id);

@@ -610,22 +610,22 @@ void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int
         views = std::max(views, (int)a.N);
     }
     const double chip = 16.0 * q.cus;
-    // Measured on densifications of 2 and (zero edges) 4 iterations, ms as
-    // kLane / kQuad / kWide, each with the tile rows below:
+    // Measured on densifications of 4 iterations, ms as kLane / kQuad / kWide,
+    // each with the tile rows below:
     // - Below one and three quarters of the chip kWide: its tiles take four
     //   times the waves that the other forms have for the same pixels, which
-    //   leave the chip idle there (480x240, 2 views: 2.7 / 3.2 / 1.8; 960x480,
-    //   8 views: 8.3 / 8.1 / 6.9; 1280x640, 8 views: 13.0 / 13.8 / 12.4;
-    //   1440x720, 4 views: 13.8 / 12.4 / -).
+    //   leave the chip idle there (480x240, 2 views: 2.2 / 2.9 / 1.7; 960x480,
+    //   8 views: 13.9 / 13.7 / 11.2; 1280x640, 8 views: 20.7 / 21.3 / 20.1;
+    //   1440x720, 4 views: 13.5 / 12.8 / 14.3).
     // - Above, kQuad: a quad's gathers fall into one patch (1920x960: 4 views
-    //   24.5 / 21.4 / 24.6, 6 views, 8 iterations 51.8 / 51.0 / -; 2880x1440,
-    //   10 views: 136 / 124 / -).
+    //   23.5 / 21.6 / 25.9, 6 views 34.9 / 33.6 / 37.1; 2880x1440, 10 views: 152
+    //   / 131 / 135).
     // - With one to three views some lanes of a quad have no view to
     //   accumulate, so kLane, where it fills the chip well enough: one view
-    //   from 640x320 (1.06 / 1.3 / 1.13), two from 960x480 (2.39 / 2.53 /
-    //   2.62; 800x400: 1.88 / 2.09 / 1.89), three from there up to 1680x840
-    //   (960x480: 3.3 / 4.4 / 3.3; 1280x640: 5.1 / 5.7 / 5.7; 1680x840, zero
-    //   edges: 13.8 / 13.5 / 16.7).
+    //   from 640x320 (1.73 / 2.26 / 1.74), two from 960x480 (3.79 / 4.23 / 4.32;
+    //   800x400: 3.19 / 4.11 / 3.10), three from there up to 1680x840 (960x480:
+    //   5.2 / 5.6 / 5.3; 1280x640: 7.8 / 8.5 / 9.2; 1680x840: 13.3 / 13.2 /
+    //   16.2).
     const double lane_from = views == 1 ? 0.375 : 0.75, lane_to = views == 3 ? 2.5 : 1e30;
     if (views <= 3 && work > lane_from * chip && work < lane_to * chip)
         r.form = kLane;
@@ -637,9 +637,9 @@ void prop_shape(const QueueState& q, const pmp_batch_config& c, int n, const int
         //   4 18.7 / 20.0, seven with 2 and one with 10 33.9 / 34.7, four with 2
         //   and four with 4 33.5 / 32.2).
         r.form = gain > 0.0 ? kLane : kQuad;
-    // kQuad, 1440x720, 4 views: 12.4 ms with 8 rows, 14.0 with 4, 13.1 with 2;
-    // with a launch per pass, whose last tiles leave compute units idle, 15.2
-    // with 8, 14.1 with 4, 14.7 with 2.  kWide, 640x320, 4 views: 3.4 with 2,
+    // kQuad, 1440x720, 4 views: 13.0 ms with 8 rows, 14.4 with 4, 12.9 with 2
+    // (1920x960, 6 views: 33.1, 33.4, 35.0); with a launch per pass, whose last
+    // tiles leave compute units idle, 15.5 with 8, 14.0 with 4, 14.3 with 2.  kWide, 640x320, 4 views: 3.4 with 2,
     // 3.5 with 4.  kLane: pmp_queue.h
     r.rows = !is_default(c) ? c.tile_rows : r.form == kLane ? 4 : r.form == kWide ? 2 : single ? 4 : 8;
     if (r.form == kWide && r.rows == 8) r.form = kQuad;
@@ -667,11 +667,11 @@ int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool
     // blocks beyond one per tile would only look for work
     if (tiles > 0) bpc = std::min(bpc, (tiles + q.cus - 1) / q.cus);
     // One launch over all passes pays where the blocks in flight hold less
-    // than two thirds of the tiles (1920x960, 4 views, 4 iterations: 21.4
-    // against 24.9 ms; 640x320, 4 views: 3.4 against 4.2 ms).  Otherwise most
+    // than two thirds of the tiles (1920x960, 4 views, 4 iterations: 21.5
+    // against 24.6 ms; 640x320, 4 views: 3.4 against 4.2 ms).  Otherwise most
     // tiles are in flight at once and wait for each other tile by tile, while
     // the launches' own barrier leaves the last ones whole compute units
-    // (480x240, 4 views, 4 iterations: 4.4 against 2.4 ms).
+    // (480x240, 4 views, 4 iterations: 3.3 against 2.3 ms).
     // With many tiles to each block the idle end of a pass is a small part of
     // it, while the tiles of a pass come in the order in which the pass before
     // completed them, farther apart in the images the longer the passes are.

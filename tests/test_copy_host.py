@@ -23,3 +23,15 @@ def test_copies(san, part):
     if "unexpected memory mapping" in r.stderr:
         pytest.skip("ThreadSanitizer cannot map its shadow memory on this kernel")
     assert r.returncode == 0 and f"{part} ok" in r.stdout, f"rc {r.returncode}\n{r.stdout}\n{r.stderr[-6000:]}"
+
+
+def test_scheduler_under_tsan():
+    """The serving scheduler's own self-test under ThreadSanitizer (tests/native/host_selftest.cpp)."""
+    r = subprocess.run(["make", "-s", "-C", NATIVE, "build/host_selftest_tsan"], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+    r = subprocess.run([os.path.join(NATIVE, "build", "host_selftest_tsan")], capture_output=True, text=True,
+                       timeout=120, env=ENV)
+    if "unexpected memory mapping" in r.stderr:
+        pytest.skip("ThreadSanitizer cannot map its shadow memory on this kernel")
+    assert r.returncode == 0 and "host_selftest: ok" in r.stdout, f"rc {r.returncode}\n{r.stdout}\n{r.stderr[-6000:]}"
