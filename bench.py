@@ -54,7 +54,7 @@ HBM_PEAK_GBS = 8000.0
 # L2-to-memory bytes per red-black pass of k_propagate_q on the 1920x960 + 6-view
 # workload, from rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a copy of known
 # size (profiles/k_propagate_q_c1_1920x960_6views.md); None for other workloads.
-TRAFFIC_BYTES_PER_LAUNCH_C1 = int((174_844 * 2.00 + 71_375 * 1.00) * 1024)
+TRAFFIC_BYTES_PER_LAUNCH_C1 = int((171_331 * 2.00 + 71_375 * 1.00) * 1024)
 TRAFFIC_SOURCE = ("profile-derived, not measured in this run: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of "
                   "k_propagate_q on this workload, scaled by a streaming copy of known size "
                   "(profiles/k_propagate_q_c1_1920x960_6views.md)")
